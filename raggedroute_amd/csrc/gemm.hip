@@ -29,6 +29,8 @@
 
 #include "launchers.h"
 #include "raggedroute_capi.h"
+#include "split_gemm.h"
+#include "tiles.h"
 #include "wave.h"
 
 namespace rr::kern {
@@ -36,33 +38,11 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int kGroupM = 8;  // row tiles per swizzle group
-constexpr int kXcds = 8;    // MI355X: 8 XCDs, workgroups dispatched round-robin
-
 enum Mode : int {
   kDense = 0,         // one segment [0, dense_rows), weights W
   kGrouped = 1,       // segments from offsets, weights W[e]
   kChainGrouped = 2,  // grouped with A rows gathered through sorted_route, x_permuted
                       // written, and the top-2 unpermute folded into the epilogue
-};
-
-struct GemmParams {
-  const float* X;
-  const float* W;
-  const int32_t* offsets;
-  float* Y;
-  int experts;
-  int dense_rows;
-  int K;
-  int N;
-  // kChainGrouped: segment row r holds token sorted_route[r] / top_k of X; the
-  // gathered rows go to x_permuted (when given) and, when y_out is given
-  // (top-2), y_out[token] += route_weights[route] * Y[r].
-  const int32_t* sorted_route;
-  const float* route_weights;
-  float* x_permuted;
-  float* y_out;
-  int top_k;
 };
 
 template <int BM_, int BN_, int WM_, int WN_, int BK_>
@@ -267,18 +247,6 @@ __device__ __forceinline__ void mfma_steps(v4f (&acc)[TM][TN], const v4f (&af)[T
   }
 }
 
-// Tile space decode: row tiles are grouped kGroupM at a time so that workgroups
-// running together share both A row blocks and B column strips.
-__device__ __forceinline__ void decode_tile(int t, int row_tiles, int col_tiles, int* rt, int* ct) {
-  const int group_size = kGroupM * col_tiles;
-  const int group = t / group_size;
-  const int first = group * kGroupM;
-  const int rows_in_group = row_tiles - first < kGroupM ? row_tiles - first : kGroupM;
-  const int within = t - group * group_size;
-  *rt = first + within % rows_in_group;
-  *ct = within / rows_in_group;
-}
-
 // Wave layouts of a tile's MFMA work. WaveLayout: the tile shape's WM x WN
 // grid of (BM / WM) x (BN / WN) wave tiles. SlabLayout: every wave takes all
 // TM 16-row blocks of the tile's top rows and a COLS-wide column slab.
@@ -327,54 +295,11 @@ __global__ __launch_bounds__(S::kThreads, 2) void rr_gemm_mfma_kernel(GemmParams
   const int N = prm.N;
 
   // ---- device-side scheduler: per-expert row-tile prefixes in LDS ----
-  // With slab layouts (below) an expert's last row tile is "short" when it
-  // holds at most BM / 2 rows: its MFMA work is a fraction of a full tile's.
-  // The tile space lists every full tile first and the short ones after, so
-  // the grid-stride rounds finish on cheap tiles instead of putting a short
-  // tile's worker behind a full round.
   for (int e = tid; e <= experts; e += S::kThreads) {
     s_off[e] = kGroupedRows ? prm.offsets[e] : (e == 0 ? 0 : prm.dense_rows);
   }
   __syncthreads();
-  auto full_tiles = [](int32_t cnt) -> int32_t {
-    if (cnt <= 0) return 0;
-    if constexpr (kSlabs) return cnt / S::BM + (cnt % S::BM > S::BM / 2 ? 1 : 0);
-    return (cnt + S::BM - 1) / S::BM;
-  };
-  auto short_tiles = [](int32_t cnt) -> int32_t {
-    if constexpr (kSlabs) return cnt > 0 && cnt % S::BM != 0 && cnt % S::BM <= S::BM / 2 ? 1 : 0;
-    return 0;
-  };
-  if (wave == 0) {
-    // Lane l owns experts [l*per, (l+1)*per); experts <= 1024 -> per <= 16.
-    const int per = (experts + 63) / 64;
-    int32_t local = 0, local2 = 0;
-    for (int j = 0; j < per; ++j) {
-      const int e = lane * per + j;
-      if (e < experts) {
-        const int32_t cnt = s_off[e + 1] - s_off[e];
-        local += full_tiles(cnt);
-        local2 += short_tiles(cnt);
-      }
-    }
-    const int32_t incl = rr::dev::wave_inclusive_scan(local);
-    const int32_t incl2 = rr::dev::wave_inclusive_scan(local2);
-    int32_t run = incl - local, run2 = incl2 - local2;
-    for (int j = 0; j < per; ++j) {
-      const int e = lane * per + j;
-      if (e < experts) {
-        s_pre[e] = run;
-        s_pre2[e] = run2;
-        const int32_t cnt = s_off[e + 1] - s_off[e];
-        run += full_tiles(cnt);
-        run2 += short_tiles(cnt);
-      }
-    }
-    if (lane == 63) {
-      s_pre[experts] = incl;
-      s_pre2[experts] = incl2;
-    }
-  }
+  if (wave == 0) build_tile_prefix<S::BM, kSlabs>(s_off, s_pre, s_pre2, experts, lane);
   __syncthreads();
   const int full_rows = s_pre[experts];
   const int short_rows = s_pre2[experts];
@@ -382,11 +307,8 @@ __global__ __launch_bounds__(S::kThreads, 2) void rr_gemm_mfma_kernel(GemmParams
   const long total_full = static_cast<long>(full_rows) * col_tiles;
   const long total = total_full + static_cast<long>(short_rows) * col_tiles;
 
-  // Workgroups are dispatched round-robin over the XCDs; give the workgroups
-  // of one XCD consecutive tile ids so their operands meet in the same L2.
   const int grid = static_cast<int>(gridDim.x);
-  const int b = static_cast<int>(blockIdx.x);
-  const int worker = (grid % kXcds == 0) ? (b % kXcds) * (grid / kXcds) + b / kXcds : b;
+  const int worker = tile_worker(static_cast<int>(blockIdx.x), grid);
 
   const int g = lane >> 4;
   const int li = lane & 15;
@@ -398,13 +320,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void rr_gemm_mfma_kernel(GemmParams
     int rt, ct;
     decode_tile(static_cast<int>(is_short ? t - total_full : t), is_short ? short_rows : full_rows,
                 col_tiles, &rt, &ct);
-    // expert = last e with pre[e] <= rt (binary search over the prefix)
-    int lo = 0, hi = experts - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (pre[mid] <= rt) lo = mid; else hi = mid - 1;
-    }
-    const int e = lo;
+    const int e = tile_expert(pre, experts, rt);
     // a short tile is its expert's last: the rows past its full tiles
     const int row0 = s_off[e] + (is_short ? (s_off[e + 1] - s_off[e]) / S::BM : rt - s_pre[e]) * S::BM;
     const int row_end = s_off[e + 1];
@@ -882,6 +798,17 @@ bool direct_any_disabled() {
   return v != nullptr && std::strcmp(v, "aligned") == 0;
 }
 
+// Whether a grouped GEMM runs on the FP16 matrix cores (split_gemm.hip).
+// RR_GEMM_STAGING=fp32 keeps it on the FP32 instructions and RR_GEMM_STAGING=
+// split takes the split kernel wherever it is correct (N >= 2), for tests and
+// A/B runs.
+bool split_chosen(const GemmParams& prm, long rows, long cus) {
+  const char* v = std::getenv("RR_GEMM_STAGING");
+  if (v != nullptr && std::strcmp(v, "fp32") == 0) return false;
+  if (v != nullptr && std::strcmp(v, "split") == 0) return prm.K > 0 && prm.N >= 2;
+  return split_gemm_ok(prm.K, prm.N, prm.experts, rows, static_cast<int>(cus));
+}
+
 template <class S, int MODE>
 hipError_t launch_gemm(const GemmParams& prm, long tile_bound, hipStream_t stream) {
   const bool vec = (prm.K % 4 == 0) && (prm.N % 4 == 0) && aligned16(prm.X) && aligned16(prm.W) &&
@@ -980,6 +907,11 @@ hipError_t gemm_dispatch(const GemmParams& prm, long rows_per_expert, long total
     case 6: return launch_tile<TileMediumK256, MODE>(prm, rows_per_expert, stream);
     case 7: return launch_tile<TileNarrowK256, MODE>(prm, rows_per_expert, stream);
     default: break;
+  }
+  if constexpr (MODE != kDense) {
+    if (split_chosen(prm, total_rows_estimate, cus)) {
+      return split_grouped(prm, rows_per_expert, static_cast<int>(cus), stream);
+    }
   }
   // Largest tile that still gives every CU work (two tiles per CU for the
   // large tile, whose LDS and registers allow two resident workgroups).

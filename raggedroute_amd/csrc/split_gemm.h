@@ -1,0 +1,15 @@
+// Grouped FP32 GEMM on the FP16 matrix cores (split_gemm.hip).
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+
+#include "tiles.h"
+
+namespace rr::kern {
+
+// Whether a grouped GEMM of this size takes the split kernel (rows: of all experts).
+bool split_gemm_ok(int k, int n, int experts, long rows, int cus);
+// Grouped (prm.sorted_route null) or chain form; rows_per_expert sizes the grid only.
+hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, int cus, hipStream_t stream);
+
+}  // namespace rr::kern

@@ -1,0 +1,645 @@
+// Grouped FP32 GEMM on the FP16 matrix cores (v_mfma_f32_32x32x16_f16).
+//
+// The FP32 matrix instructions run at 157 TFLOP/s, the FP16 ones at 2.5 PFLOP/s
+// with FP32 accumulation. Every operand x is scaled by a power of two of its
+// own row (A) or column (B), xs = x * s, and split into two FP16 numbers
+//     h = fp16(xs),   l = fp16(xs - h),
+// both rounded to nearest; xs - h is exact in FP32, so h + l carries x to
+// within half a unit in its 23rd bit (most values exactly). A product is
+//     xs * ys = hx hy + (lx hy + hx ly) + lx ly;
+// the first three terms are computed (three MFMAs), the last is below 2^-24 of
+// the product and left out. hx hy is summed in one FP32 accumulator and the two
+// small terms in another, which are added once at the end: the large sum is
+// rounded once per 16 k instead of once per 4 k as on the FP32 instructions.
+// Against 64-bit sums the result is closer than the FP32 instructions' at
+// every K (2-norm error over N(0,1) operands, this / FP32 MFMA: K = 64 0.98 /
+// 1.43e-7, K = 256 1.31 / 2.87e-7, K = 1024 2.2 / 5.8e-7, K = 4096 4.1 /
+// 11.4e-7; likewise for non-negative and half-zero operands).
+//
+// Range. The scale puts the largest of a row's (column's) first nonzero slice
+// of 32 k near 2^4, so later values may be 2^12 times larger before fp16(xs)
+// overflows, and values 2^-5 of it and up split without loss; below that the
+// split's error stops shrinking at 2^-25, which is 2^-29 of the sampled
+// maximum. Values this cannot carry are never computed this way: an operand
+// that is infinite, NaN or past the FP16 range makes every output it meets
+// non-finite, and sampled maxima below 2^-100 are seen when the scale is taken.
+// A tile that shows either is computed again on the FP32 instructions before
+// anything is stored (with the FP32 rules for infinities, NaN and overflow).
+//
+// Work split: 128 x 128 output tiles, four waves, two workgroups per CU, tiles
+// dealt as in gemm.hip. A slice of 32 k of both operands is loaded into
+// registers one slice ahead (16-byte A quads, 8-byte B pairs; rows may start at
+// any 4-byte boundary), split there, and written to LDS as FP16 planes in MFMA
+// operand order (k contiguous per row of A and per column of B), two stages of
+// 32 KiB; the split costs 2.5 instructions per element, under the MFMAs of the
+// other waves. Columns are paired: thread `pair` owns columns 2 pair and
+// 2 pair + 1, held in plane rows pair and 64 + pair, so its loads and the output
+// stores of a lane are pairs of adjacent columns.
+// Tiles with few rows use layouts of 32-row blocks, so padding costs no MFMA
+// work beyond that granule.
+// Measured, FP32 instructions / this: T = 8192, E = 8, K = 4096, N = 14336 (top-2,
+// 1.92 TFLOP) 14.2 / 7.3 ms (264 TFLOP/s of FP32 products, 790 of FP16: the
+// matrix pipes are 44 % busy at the 1.5 GHz that the power limit leaves, with
+// operands of ones it runs 16 % faster); T = 16384, E = 128, K = 2048, N = 768
+// chain 1031 / 657 us.
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+
+#include "split_gemm.h"
+#include "tiles.h"
+#include "wave.h"
+
+namespace rr::kern {
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+constexpr int kBM = 128, kBN = 128, kBK = 32;
+constexpr int kThreads = 256;
+constexpr int kPlane = 128 * kBK;           // halfs of one operand plane (8 KiB)
+constexpr int kStage = 4 * kPlane;          // A high, A low, B high, B low
+constexpr int kRefLd = kBK + 1;             // FP32 recomputation: padded LDS row (floats)
+static_assert(2 * kBM * kRefLd * sizeof(float) <= 2 * kStage * sizeof(_Float16), "the FP32 slices fit the stages");
+
+// Wave tiles of TM x TN blocks of 32 x 32. kGrid: 2 x 2 waves, the wave's TN
+// = 2 column blocks being the even and the odd columns of 64; kSlab: every wave
+// takes all rows and 32 columns (lanes 0-15 the even, 16-31 the odd ones).
+template <int TM_, bool GRID, int PASSES>
+struct Layout {
+  static constexpr int TM = TM_;
+  static constexpr int kPasses = PASSES;  // 32-row passes that hold the tile's rows
+  static constexpr int TN = GRID ? 2 : 1;
+  __device__ static int row(int wave) { return GRID ? (wave >> 1) * 32 * TM_ : 0; }
+  // plane row of the lane's column in block 0 (block 1: 64 rows further)
+  __device__ static int plane_row(int wave, int li) {
+    return GRID ? 32 * (wave & 1) + li : 16 * wave + (li & 15) + 64 * (li >> 4);
+  }
+  // tile column of the lane in block 0 (block 1: the next column)
+  __device__ static int col(int wave, int li) {
+    return GRID ? 64 * (wave & 1) + 2 * li : 32 * wave + 2 * (li & 15) + (li >> 4);
+  }
+};
+
+// 16-byte chunk c (8 halfs) of plane row r sits at chunk c ^ ((r >> 2) & 3): the
+// 16 rows read together land in 16 distinct 16-byte bank groups.
+__device__ __forceinline__ int plane_swizzle(int r) { return (r >> 2) & 3; }
+
+// x * s = h + l (see the file comment)
+__device__ __forceinline__ void split2(float x0, float x1, float s, h2& h, h2& l) {
+  h[0] = static_cast<_Float16>(__builtin_fmaf(x0, s, 0.0F));
+  h[1] = static_cast<_Float16>(__builtin_fmaf(x1, s, 0.0F));
+  asm("" : "+v"(h));  // both halves in their register: the next two read them there
+  l[0] = static_cast<_Float16>(__builtin_fmaf(x0, s, -static_cast<float>(h[0])));
+  l[1] = static_cast<_Float16>(__builtin_fmaf(x1, s, -static_cast<float>(h[1])));
+}
+
+__device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFU; }
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+
+// The scale of a row or column whose sampled maximum has these bits: s = 2^t
+// with t = 4 - floor(log2(max)); 1 for an all-zero sample.
+struct Scale {
+  float s;
+  int t;
+  bool bad;  // not computed in FP16: not finite, or below 2^-100
+};
+__device__ __forceinline__ Scale scale_of(uint32_t bits) {
+  Scale sc;
+  int e = static_cast<int>(bits >> 23);
+  sc.bad = bits != 0 && (e == 255 || e < 27);
+  e = bits == 0 ? 131 : (e < 27 ? 27 : e);
+  sc.t = 131 - e;
+  sc.s = __uint_as_float(static_cast<uint32_t>(258 - e) << 23);
+  return sc;
+}
+
+// What a tile needs from the kernel (all workgroup-uniform).
+struct Tile {
+  const float* B;  // the expert's weights
+  int row0, rows;  // first segment row, rows in the tile (1..128)
+  int n0, ct;      // first column, column tile
+};
+struct Lds {
+  _Float16* stages;  // [2][kStage]
+  int32_t* ta;       // [128] scale exponents of the rows
+  int32_t* tb;       // [128] ... of the plane rows of B
+  uint2* cmax;       // [4][64] column samples
+  int32_t* src;      // [128] chain: token row of X per tile row (-1: none)
+  float* w;          // [128] chain: route weight per tile row
+};
+
+// One output tile for one wave layout (L::kPasses 32-row passes hold its rows).
+template <class L, bool CHAIN>
+__device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, const Lds& sh, int col_tiles, int wave) {
+  constexpr int P = L::kPasses;
+  constexpr int TM = L::TM, TN = L::TN;
+  // (the thread id passes an empty asm so that nothing of this is built before
+  // the tile loop, for all four layouts, and kept live across it)
+  int tid = static_cast<int>(threadIdx.x);
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63;
+  const int K = prm.K;
+  const int N = prm.N;
+  const int rows = tl.rows;
+  const int nk = (K + kBK - 1) / kBK;
+  // the last slice is loaded float by float where a quad or pair could cross
+  // the end of a row
+  const int guarded = (K % kBK != 0 || (N & 1) != 0) ? nk - 1 : nk;
+  const int li = lane & 31;
+  const int hi = lane >> 5;
+  // staging: A quad ac of row 32 p + ar; B columns 2 pair, 2 pair + 1 at k
+  // 8 wave .. + 7
+  const int ar = tid >> 3;
+  const int ac = tid & 7;
+  const int pair = lane;
+  const int a_put = ar * kBK + (((ac >> 1) ^ plane_swizzle(ar)) << 3) + ((ac & 1) << 2);
+  const int b_put = pair * kBK + ((wave ^ plane_swizzle(pair)) << 3);
+
+  // Rows past the tile's last read a row that exists (their products land in
+  // output rows that are never stored); columns past N the last pair.
+  const float* asrc[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int r = 32 * p + ar;
+    int src = r < rows ? tl.row0 + r : tl.row0;
+    if constexpr (CHAIN) {
+      src = sh.src[r];
+      if (src < 0) src = 0;
+    }
+    asrc[p] = prm.X + static_cast<std::size_t>(src) * K + 4 * ac;
+  }
+  const int n = tl.n0 + 2 * pair;
+  const int nl = n < N ? n : N - 2;
+  const uint32_t b_lane = static_cast<uint32_t>(8 * wave) * static_cast<uint32_t>(N) + static_cast<uint32_t>(nl);
+
+  f4u ra[P];
+  f2u rb[8];
+  auto load = [&](int kt) {  // whole slices
+    const float* Bk = tl.B + static_cast<std::size_t>(kt) * kBK * N;
+#pragma unroll
+    for (int p = 0; p < P; ++p) ra[p] = *reinterpret_cast<const f4u*>(asrc[p] + kt * kBK);
+    // (a pair that crosses N reads the next k row's first float)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      rb[j] = *reinterpret_cast<const f2u*>(Bk + static_cast<std::size_t>(j) * N + b_lane);
+    }
+  };
+  auto load_any = [&](int kt) {
+    if (kt != guarded) {
+      load(kt);
+      return;
+    }
+    const float* Bk = tl.B + static_cast<std::size_t>(kt) * kBK * N;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v = 0.0F;
+        if (kt * kBK + 4 * ac + q < K) v = asrc[p][kt * kBK + q];
+        ra[p][q] = v;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float* b = Bk + static_cast<std::size_t>(j) * N + b_lane;
+      float v0 = 0.0F, v1 = 0.0F;
+      if (kt * kBK + 8 * wave + j < K) {
+        v0 = b[0];
+        if (nl + 1 < N) v1 = b[1];
+      }
+      rb[j] = f2u{v0, v1};
+    }
+  };
+
+  // ---- scales: the first slice with a nonzero value, per row and column ----
+  // (almost always slice 0; a tile with an all-zero row or column reads on)
+  load_any(0);
+  uint32_t ma[P] = {};
+  uint32_t mb0 = 0, mb1 = 0;
+#pragma unroll 1
+  for (int kt = 0;;) {
+    bool need = false;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      uint32_t m = umax(umax(abs_bits(ra[p][0]), abs_bits(ra[p][1])), umax(abs_bits(ra[p][2]), abs_bits(ra[p][3])));
+      // over the row's eight lanes: quad neighbours, then the half row's mirror
+      m = umax(m, rr::dev::dpp_move<0xB1>(m));
+      m = umax(m, rr::dev::dpp_move<0x4E>(m));
+      m = umax(m, rr::dev::dpp_move<0x141>(m));
+      if (ma[p] == 0) ma[p] = m;
+      need = need || (ma[p] == 0 && 32 * p + ar < rows);
+    }
+    uint32_t c0 = 0, c1 = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      c0 = umax(c0, abs_bits(rb[j][0]));
+      c1 = umax(c1, abs_bits(rb[j][1]));
+    }
+    sh.cmax[64 * wave + pair] = make_uint2(c0, c1);
+    __syncthreads();
+    c0 = c1 = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint2 m = sh.cmax[64 * w + pair];
+      c0 = umax(c0, m.x);
+      c1 = umax(c1, m.y);
+    }
+    if (mb0 == 0) mb0 = c0;
+    if (mb1 == 0) mb1 = c1;
+    need = need || (mb0 == 0 && n < N) || (mb1 == 0 && n + 1 < N);
+    if (__syncthreads_or(need ? 1 : 0) == 0 || kt + 1 >= nk) {
+      if (kt > 0) load_any(0);
+      break;
+    }
+    load_any(++kt);
+  }
+  bool bad = false;
+  float sa[P], sb0, sb1;
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const Scale sc = scale_of(ma[p]);
+    sa[p] = sc.s;
+    bad = bad || (sc.bad && 32 * p + ar < rows);
+    if (ac == 0) sh.ta[32 * p + ar] = sc.t;
+  }
+  {
+    const Scale x = scale_of(mb0), y = scale_of(mb1);
+    sb0 = x.s;
+    sb1 = y.s;
+    bad = bad || (x.bad && n < N) || (y.bad && n + 1 < N);
+    if (wave == 0) {
+      sh.tb[pair] = x.t;
+      sh.tb[64 + pair] = y.t;
+    }
+  }
+
+  // Gathered rows go to x_permuted spread over the column tiles: tile ct
+  // writes the k slices kt with kt % col_tiles == ct.
+  int next_xp = CHAIN && prm.x_permuted != nullptr ? tl.ct : -1;
+  auto store_xp = [&](int kt) {
+    if constexpr (CHAIN) {
+      if (kt != next_xp) return;
+      next_xp += col_tiles;
+      const int k = kt * kBK + 4 * ac;
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int r = 32 * p + ar;
+        if (r < rows) {
+          float* out = prm.x_permuted + static_cast<std::size_t>(tl.row0 + r) * K + k;
+          if (k + 4 <= K) {
+            __builtin_nontemporal_store(ra[p], reinterpret_cast<f4u*>(out));
+          } else {
+            for (int q = 0; k + q < K; ++q) out[q] = ra[p][q];
+          }
+        }
+      }
+    } else {
+      (void)kt;
+    }
+  };
+  // the slice in registers, split, into an LDS stage
+  auto put = [&](_Float16* __restrict__ st) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      h2 h0, l0, h1, l1;
+      split2(ra[p][0], ra[p][1], sa[p], h0, l0);
+      split2(ra[p][2], ra[p][3], sa[p], h1, l1);
+      *reinterpret_cast<h4*>(st + p * 32 * kBK + a_put) = h4{h0[0], h0[1], h1[0], h1[1]};
+      *reinterpret_cast<h4*>(st + kPlane + p * 32 * kBK + a_put) = h4{l0[0], l0[1], l1[0], l1[1]};
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      h8 h, l;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        h2 hh, ll;
+        split2(rb[2 * q][j], rb[2 * q + 1][j], j == 0 ? sb0 : sb1, hh, ll);
+        h[2 * q] = hh[0];
+        h[2 * q + 1] = hh[1];
+        l[2 * q] = ll[0];
+        l[2 * q + 1] = ll[1];
+      }
+      *reinterpret_cast<h8*>(st + 2 * kPlane + b_put + j * 64 * kBK) = h;
+      *reinterpret_cast<h8*>(st + 3 * kPlane + b_put + j * 64 * kBK) = l;
+    }
+  };
+
+  const int wrow = L::row(wave);
+  v16f acc[TM][TN], low[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.0F;
+    }
+  }
+  {
+    const int prow = L::plane_row(wave, li);
+    // operand chunk of k step ks: k = 16 ks + 8 hi .. + 7
+    const int aget = (wrow + li) * kBK, bget = prow * kBK;
+    const int achunk[2] = {(hi ^ plane_swizzle(li)) << 3, ((2 + hi) ^ plane_swizzle(li)) << 3};
+    const int bchunk[2] = {(hi ^ plane_swizzle(prow)) << 3, ((2 + hi) ^ plane_swizzle(prow)) << 3};
+    auto multiply = [&](const _Float16* __restrict__ st, int ks) {
+      h8 ah[TM], al[TM], bh[TN], bl[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        ah[i] = *reinterpret_cast<const h8*>(st + aget + achunk[ks] + i * 32 * kBK);
+        al[i] = *reinterpret_cast<const h8*>(st + kPlane + aget + achunk[ks] + i * 32 * kBK);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        bh[j] = *reinterpret_cast<const h8*>(st + 2 * kPlane + bget + bchunk[ks] + j * 64 * kBK);
+        bl[j] = *reinterpret_cast<const h8*>(st + 3 * kPlane + bget + bchunk[ks] + j * 64 * kBK);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], low[i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], low[i][j], 0, 0, 0);
+      }
+    };
+    put(sh.stages);
+    store_xp(0);
+    if (nk > 1) load_any(1);
+    __syncthreads();
+    int kt = 0;
+    // slice kt is multiplied while slice kt + 2 is on its way; slice kt + 1 has
+    // landed and goes to the other stage first, so its registers take the loads
+#pragma unroll 1
+    for (; kt + 3 < nk; ++kt) {
+      put(sh.stages + (~kt & 1) * kStage);
+      store_xp(kt + 1);
+      load(kt + 2);
+      __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to the slice's end)
+      const _Float16* cur = sh.stages + (kt & 1) * kStage;
+      multiply(cur, 0);
+      multiply(cur, 1);
+      __syncthreads();
+    }
+#pragma unroll 1
+    for (; kt < nk; ++kt) {
+      if (kt + 1 < nk) {
+        put(sh.stages + (~kt & 1) * kStage);
+        store_xp(kt + 1);
+      }
+      if (kt + 2 < nk) load_any(kt + 2);
+      const _Float16* cur = sh.stages + (kt & 1) * kStage;
+      multiply(cur, 0);
+      multiply(cur, 1);
+      __syncthreads();
+    }
+  }
+
+  // (the lane id passes an empty asm so that none of the epilogue's addresses
+  // is built before the loop and kept live across it)
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int eli = ln & 31;
+  const int ehi = ln >> 5;
+  // output rows of accumulator register r: 32 i + 8 (r / 4) + 4 hi + r % 4 of the wave's
+  const int col = tl.n0 + L::col(wave, eli);
+  const int prow = L::plane_row(wave, eli);
+  auto store_tile = [&](bool scaled) {
+    int tb[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) tb[j] = sh.tb[prow + 64 * j];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
+        if (rl >= rows) continue;
+        const int ta = sh.ta[rl];
+        float v[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) v[j] = scaled ? ldexpf(acc[i][j][r], -(ta + tb[j])) : acc[i][j][r];
+        float* yrow = prm.Y + static_cast<std::size_t>(tl.row0 + rl) * N + col;
+        float* comb = nullptr;
+        float w = 0.0F;
+        if constexpr (CHAIN) {
+          if (prm.y_out != nullptr) {
+            comb = prm.y_out + static_cast<std::size_t>(sh.src[rl]) * N + col;
+            w = sh.w[rl];
+          }
+        }
+        auto put1 = [&](int j) {
+          if (comb != nullptr) {
+            __builtin_nontemporal_store(v[j], yrow + j);  // y_permuted is not read again by the chain
+          } else {
+            yrow[j] = v[j];
+          }
+        };
+        if constexpr (TN == 2) {
+          if (col + 1 < N) {
+            if (comb != nullptr) {
+              __builtin_nontemporal_store(f2u{v[0], v[1]}, reinterpret_cast<f2u*>(yrow));
+            } else {
+              *reinterpret_cast<f2u*>(yrow) = f2u{v[0], v[1]};
+            }
+          } else if (col < N) {
+            put1(0);
+          }
+        } else if (col < N) {
+          put1(0);
+        }
+        if (comb != nullptr) {
+          // Both routes of a token add into the zeroed output: fl(0 + a) + b
+          // is the same in either order, so the combine is deterministic
+          // and equals the rank-order unpermute.
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            if (col + j < N) unsafeAtomicAdd(comb + j, __fmul_rn(w, v[j]));
+          }
+        }
+      }
+    }
+  };
+  bool overflow = bad;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
+        acc[i][j][r] += low[i][j][r];
+        overflow = overflow || (rl < rows && col + j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
+      }
+    }
+  }
+  const bool redo = __syncthreads_or(overflow ? 1 : 0) != 0;
+  if (redo) {
+    // the same tile on the FP32 instructions, slices staged unscaled
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0F;
+      }
+    }
+    float* As = reinterpret_cast<float*>(sh.stages);
+    float* Bs = As + kBM * kRefLd;
+#pragma unroll 1
+    for (int kt = 0; kt < nk; ++kt) {
+      load_any(kt);
+      __syncthreads();  // the previous slice is used up
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) As[(32 * p + ar) * kRefLd + 4 * ac + q] = ra[p][q];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        Bs[pair * kRefLd + 8 * wave + j] = rb[j][0];
+        Bs[(64 + pair) * kRefLd + 8 * wave + j] = rb[j][1];
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int k = 0; k < kBK; k += 2) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const float a = As[(wrow + 32 * i + eli) * kRefLd + k + ehi];
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, Bs[(prow + 64 * j) * kRefLd + k + ehi], acc[i][j], 0, 0, 0);
+          }
+        }
+      }
+    }
+  }
+  store_tile(!redo);
+}
+
+template <bool CHAIN>
+__global__ __launch_bounds__(kThreads, 2) void rr_split_gemm_kernel(GemmParams prm) {
+  extern __shared__ __align__(16) _Float16 smem[];
+  Lds sh;
+  sh.stages = smem;
+  sh.ta = reinterpret_cast<int32_t*>(smem + 2 * kStage);
+  sh.tb = sh.ta + kBM;
+  sh.cmax = reinterpret_cast<uint2*>(sh.tb + kBN);
+  sh.src = reinterpret_cast<int32_t*>(sh.cmax + 4 * 64);
+  sh.w = reinterpret_cast<float*>(sh.src + kBM);
+  int32_t* s_off = reinterpret_cast<int32_t*>(sh.w + kBM);  // [E + 1]
+  int32_t* s_pre = s_off + prm.experts + 1;                 // [E + 1] full row tiles before expert e
+  int32_t* s_pre2 = s_pre + prm.experts + 1;                // [E + 1] short row tiles before expert e
+  const int tid = static_cast<int>(threadIdx.x);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int experts = prm.experts;
+
+  for (int e = tid; e <= experts; e += kThreads) s_off[e] = prm.offsets[e];
+  __syncthreads();
+  if (wave == 0) build_tile_prefix<kBM, true>(s_off, s_pre, s_pre2, experts, rr::dev::lane_id());
+  __syncthreads();
+  const int full_rows = s_pre[experts];
+  const int short_rows = s_pre2[experts];
+  const int col_tiles = (prm.N + kBN - 1) / kBN;
+  const long total_full = static_cast<long>(full_rows) * col_tiles;
+  const long total = total_full + static_cast<long>(short_rows) * col_tiles;
+  const int grid = static_cast<int>(gridDim.x);
+  const int worker = tile_worker(static_cast<int>(blockIdx.x), grid);
+
+#pragma unroll 1
+  for (long t = worker; t < total; t += grid) {
+    const bool is_short = t >= total_full;
+    int rt, ct;
+    decode_tile(static_cast<int>(is_short ? t - total_full : t), is_short ? short_rows : full_rows,
+                col_tiles, &rt, &ct);
+    const int e = __builtin_amdgcn_readfirstlane(tile_expert(is_short ? s_pre2 : s_pre, experts, rt));
+    const int first = __builtin_amdgcn_readfirstlane(s_off[e]);
+    const int end = __builtin_amdgcn_readfirstlane(s_off[e + 1]);
+    Tile tl;
+    tl.B = prm.W + static_cast<std::size_t>(e) * prm.K * prm.N;
+    tl.row0 = first + (is_short ? (end - first) / kBM : rt - __builtin_amdgcn_readfirstlane(s_pre[e])) * kBM;
+    tl.rows = end - tl.row0 < kBM ? end - tl.row0 : kBM;
+    tl.n0 = ct * kBN;
+    tl.ct = ct;
+
+    __syncthreads();  // the previous tile's epilogue is done with the LDS tables
+    if constexpr (CHAIN) {
+      if (tid < kBM) {
+        int32_t token = -1;
+        float w = 0.0F;
+        if (tid < tl.rows) {
+          const int32_t route = prm.sorted_route[tl.row0 + tid];
+          token = route / prm.top_k;  // route = top_k * token + rank
+          if (prm.y_out != nullptr) w = prm.route_weights[route];
+        }
+        sh.src[tid] = token;
+        sh.w[tid] = w;
+      }
+      __syncthreads();
+    }
+    if (tl.rows > 96) {
+      run_tile<Layout<2, true, 4>, CHAIN>(prm, tl, sh, col_tiles, wave);
+    } else if (tl.rows > 64) {
+      run_tile<Layout<3, false, 3>, CHAIN>(prm, tl, sh, col_tiles, wave);
+    } else if (tl.rows > 32) {
+      run_tile<Layout<1, true, 2>, CHAIN>(prm, tl, sh, col_tiles, wave);
+    } else {
+      run_tile<Layout<1, false, 1>, CHAIN>(prm, tl, sh, col_tiles, wave);
+    }
+  }
+}
+
+template <bool CHAIN>
+hipError_t launch(const GemmParams& prm, long rows_per_expert, int cus, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(rr_split_gemm_kernel<CHAIN>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+  if (attr != hipSuccess) return attr;
+  const long tiles = static_cast<long>(prm.experts) * ((rows_per_expert + kBM - 1) / kBM) *
+                     ((static_cast<long>(prm.N) + kBN - 1) / kBN);
+  const long cap = 2L * cus;
+  long grid = tiles < cap ? tiles : cap;
+  if (grid >= kXcds) grid = grid / kXcds * kXcds;
+  if (grid < 1) grid = 1;
+  const std::size_t lds = 2 * kStage * sizeof(_Float16) + (kBM + kBN) * sizeof(int32_t) + 4 * 64 * sizeof(uint2) +
+                          2 * kBM * sizeof(int32_t) + 3 * static_cast<std::size_t>(prm.experts + 1) * sizeof(int32_t);
+  rr_split_gemm_kernel<CHAIN><<<dim3(static_cast<unsigned>(grid)), kThreads, lds, stream>>>(prm);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+// K >= 256 and N >= 272 (three column tiles), a tile for every CU (the rows
+// of the whole problem plus a part tile per expert), and 16 rows an expert.
+// With fewer tiles a workgroup has its CU to itself and a slice's split, LDS
+// round trip and MFMAs run one after the other, where the FP32 kernels have
+// smaller tiles; with fewer rows the call reads weights for few products and
+// the split is work on top. FP32 kernels / this one, grouped GEMM alone:
+// E = 8, K = 1024, N = 2048 with 512 rows (192 tiles) 46 / 57 us, 1024 rows
+// (256) 83 / 69 us, 4096 rows (640) 192 / 100 us; E = 16, K = 2048, N = 300
+// with 4096 rows (144) 84 / 107 us; E = 64, K = 1024, N = 512 with 2048 rows
+// (320) 46 / 48 us, 4096 rows (384) 84 / 60 us; E = 128, K = 2048, N = 768 with
+// 128 rows (one an expert) 88 / 94 us, 2048 rows 181 / 175 us, 8192 rows 387 /
+// 212 us; E = 8, K = 4096, N = 14336 with 512 rows 763 / 414 us, 4096 rows
+// 3689 / 1883 us.
+bool split_gemm_ok(int k, int n, int experts, long rows, int cus) {
+  const long tiles = ((rows + kBM - 1) / kBM + experts) * ((static_cast<long>(n) + kBN - 1) / kBN);
+  return k >= 256 && n >= 272 && tiles >= cus && rows >= 16L * experts;
+}
+
+hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, int cus, hipStream_t stream) {
+  return prm.sorted_route != nullptr ? launch<true>(prm, rows_per_expert, cus, stream)
+                                     : launch<false>(prm, rows_per_expert, cus, stream);
+}
+
+}  // namespace rr::kern

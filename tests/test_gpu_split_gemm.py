@@ -1,0 +1,139 @@
+"""The grouped GEMM on the FP16 matrix cores, forced with RR_GEMM_STAGING=split
+(by default it takes large problems): row counts at the edges of its 32-row blocks and tiles, K and N at the edges of
+its slices, pairs and column tiles, offset pointers, and values that its scales
+cannot carry (infinities, NaN, overflow, subnormals, late outliers, leading
+zeros), which must come out as the FP32 instructions give them
+(RR_GEMM_STAGING=fp32).
+
+Tolerance: check_grouped's accumulation-aware bound 4 gamma_K sum |a b| + 1e-7
+of the float64 product. A split operand is off by at most 2^-23 of itself, so a
+product of two with the lx ly term left out by under 2^-21, inside 4 gamma_K for
+every K >= 2; the sums round no more often than FP32 ones.
+"""
+from __future__ import annotations
+
+import os
+
+import numpy as np
+import pytest
+
+import raggedroute_amd as rr
+from raggedroute_amd import workloads
+from test_gpu_chain import ChainRun, check_chain, run_stages
+from test_gpu_ops import NATIVE, check_grouped, run_grouped
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def staging():
+    saved = os.environ.get("RR_GEMM_STAGING")
+
+    def put(name):
+        os.environ["RR_GEMM_STAGING"] = name
+    put("split")
+    yield put
+    os.environ.pop("RR_GEMM_STAGING", None)
+    if saved is not None:
+        os.environ["RR_GEMM_STAGING"] = saved
+
+
+EDGE_ROWS = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 192, 193, 255, 256, 257]
+
+
+@pytest.mark.parametrize("counts,k,n,offset", [
+    (EDGE_ROWS, 256, 272, 0),
+    (EDGE_ROWS, 257, 273, 0),              # one float in the last slice, odd N: the last pair is half a pair
+    (EDGE_ROWS[::-1], 287, 383, 1),        # pointers off 16 bytes
+    ([5, 0, 200, 70], 288, 384, 0),        # whole slices, whole column tiles
+    ([5, 0, 200, 70], 319, 385, 3),        # a column tile of one column
+    ([300, 40, 129], 1023, 641, 0),
+    ([9] * 130, 256, 300, 0),              # more tiles than workgroups per XCD
+    ([3] * 1024, 256, 272, 0),             # E = 1024
+    ([70, 3], 1, 2, 0),                    # one float, one pair
+    ([70, 3], 33, 5, 1),                   # two slices
+    ([70, 3], 65, 131, 0),                 # three slices
+])
+def test_edges(ctx, device, counts, k, n, offset):
+    rng = np.random.default_rng(sum(counts) + k + n)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    rows = int(offsets[-1])
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (rng.standard_normal((len(counts), k, n)) / np.sqrt(k)).astype(np.float32)
+    y = run_grouped(ctx, device, x, w, offsets, NATIVE, max_tokens=max(counts), offset=offset, rows_total=rows)
+    check_grouped(y, x, w, offsets)
+
+
+def special_inputs(case, rng):
+    counts, k, n = [200, 40, 90, 20], 320, 400
+    x = rng.standard_normal((sum(counts), k)).astype(np.float32)
+    w = (rng.standard_normal((4, k, n)) / np.sqrt(k)).astype(np.float32)
+    if case == "infinity and NaN":
+        x[3, 100] = np.inf
+        x[210, 5] = np.nan
+        w[2, 7, 9] = -np.inf
+    elif case == "late outlier":      # 2^20 times the sampled slice
+        x[:, 200] *= 1e6
+    elif case == "zeros":             # zero rows, zero columns, leading zeros of both
+        x[7] = 0
+        x[:, :64] = 0
+        x[220] = 0
+        w[:, :100] = 0
+        w[1, :, 7] = 0
+    elif case == "all zero":
+        x[:] = 0
+    elif case == "tiny":
+        x *= np.float32(1e-34)
+    elif case == "subnormal":
+        x *= np.float32(1e-38)
+        w *= np.float32(1e3)
+    elif case == "huge":
+        x *= np.float32(1e37)
+        w *= np.float32(1e-5)
+    elif case == "overflow":          # the first rows' sums pass the FP32 range, whatever their order
+        x[:100] = np.minimum(np.abs(x[:100]), 1.5) * np.float32(2e38)
+        w = np.abs(w)
+    elif case == "row scales":
+        x *= np.logspace(-18, 18, x.shape[0], dtype=np.float32)[:, None]
+        w *= np.logspace(-9, 9, n, dtype=np.float32)
+    return counts, x, w
+
+
+@pytest.mark.parametrize("case", ["infinity and NaN", "late outlier", "zeros", "all zero", "tiny", "subnormal",
+                                  "huge", "overflow", "row scales"])
+def test_values_past_the_fp16_range(ctx, device, staging, case):
+    counts, x, w = special_inputs(case, np.random.default_rng(11))
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    staging("fp32")
+    want = run_grouped(ctx, device, x, w, offsets, NATIVE)
+    staging("split")
+    got = run_grouped(ctx, device, x, w, offsets, NATIVE)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    # the finite ones: both lie within 4 gamma_K sum |a b| of the exact sums
+    # (and a few subnormal steps: each product and sum may round to one)
+    gamma = x.shape[1] * 2.0 ** -24
+    with np.errstate(over="ignore", invalid="ignore"):
+        for e, c in enumerate(counts):
+            s = int(offsets[e])
+            mag = np.abs(x[s:s + c].astype(np.float64)) @ np.abs(w[e].astype(np.float64))
+            exact = x[s:s + c].astype(np.float64) @ w[e].astype(np.float64)
+            fin = np.isfinite(want[s:s + c])
+            err = np.abs(got[s:s + c].astype(np.float64) - exact)
+            assert (err <= 4 * gamma * mag + 2 * x.shape[1] * 2.0 ** -149)[fin].all(), (case, e)
+
+
+@pytest.mark.parametrize("tokens,experts,hidden,output", [
+    (700, 8, 256, 272), (333, 5, 289, 301), (64, 16, 512, 384), (1100, 7, 260, 640),
+])
+def test_chain_form_matches_stage_by_stage(ctx, device, tokens, experts, hidden, output):
+    cfg = workloads.ChainConfig("split", tokens, experts, hidden, output)
+    inp = workloads.chain_inputs(cfg, seed=6)
+    fused = ChainRun(cfg, inp, device).run(ctx)
+    ref = run_stages(cfg, inp, device, ctx)
+    for key in ("logits", "ids", "counts", "offsets", "route_pos", "x_permuted", "y_permuted", "y"):
+        a, b = fused[key], ref[key]
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"{key} differs"
+    check_chain(cfg, inp, fused)
