@@ -800,12 +800,12 @@ bool direct_any_disabled() {
 
 // Whether a grouped GEMM runs on the FP16 matrix cores (split_gemm.hip).
 // RR_GEMM_STAGING=fp32 keeps it on the FP32 instructions and RR_GEMM_STAGING=
-// split takes the split kernel wherever it is correct (N >= 2), for tests and
-// A/B runs.
+// split takes the split kernel wherever it can run, for tests and A/B runs.
 bool split_chosen(const GemmParams& prm, long rows, long cus) {
   const char* v = std::getenv("RR_GEMM_STAGING");
   if (v != nullptr && std::strcmp(v, "fp32") == 0) return false;
-  if (v != nullptr && std::strcmp(v, "split") == 0) return prm.K > 0 && prm.N >= 2;
+  if (!split_gemm_fits(prm)) return false;
+  if (v != nullptr && std::strcmp(v, "split") == 0) return true;
   return split_gemm_ok(prm.K, prm.N, prm.experts, rows, static_cast<int>(cus));
 }
 
@@ -910,7 +910,7 @@ hipError_t gemm_dispatch(const GemmParams& prm, long rows_per_expert, long total
   }
   if constexpr (MODE != kDense) {
     if (split_chosen(prm, total_rows_estimate, cus)) {
-      return split_grouped(prm, rows_per_expert, static_cast<int>(cus), stream);
+      return split_grouped(prm, rows_per_expert, total_rows_estimate, static_cast<int>(cus), stream);
     }
   }
   // Largest tile that still gives every CU work (two tiles per CU for the
@@ -979,7 +979,7 @@ hipError_t chain_grouped_mfma(const float* x, const float* expert_weights, const
                               int top_k, int experts, int hidden, int output, hipStream_t stream) {
   if (tokens <= 0 || output <= 0) return hipSuccess;
   if (y != nullptr && top_k != 2) return hipErrorInvalidValue;  // combine is top-2 only
-  GemmParams p = base_params(x, expert_weights, offsets, y_permuted, experts, 0, hidden, output);
+  GemmParams p = base_params(x, expert_weights, offsets, y_permuted, experts, tokens, hidden, output);
   p.sorted_route = sorted_route;
   p.route_weights = route_weights;
   p.x_permuted = x_permuted;

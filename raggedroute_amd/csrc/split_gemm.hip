@@ -4,17 +4,18 @@
 // with FP32 accumulation. Every operand x is scaled by a power of two of its
 // own row (A) or column (B), xs = x * s, and split into two FP16 numbers
 //     h = fp16(xs),   l = fp16(xs - h),
-// both rounded to nearest; xs - h is exact in FP32, so h + l carries x to
-// within half a unit in its 23rd bit (most values exactly). A product is
+// both rounded to nearest; xs - h is exact in FP32 and at most 2^-11 of xs, so
+// h + l carries x to within 2^-23 of itself (half of all values exactly). A
+// product is
 //     xs * ys = hx hy + (lx hy + hx ly) + lx ly;
-// the first three terms are computed (three MFMAs), the last is below 2^-24 of
-// the product and left out. hx hy is summed in one FP32 accumulator and the two
-// small terms in another, which are added once at the end: the large sum is
-// rounded once per 16 k instead of once per 4 k as on the FP32 instructions.
-// Against 64-bit sums the result is closer than the FP32 instructions' at
-// every K (2-norm error over N(0,1) operands, this / FP32 MFMA: K = 64 0.98 /
-// 1.43e-7, K = 256 1.31 / 2.87e-7, K = 1024 2.2 / 5.8e-7, K = 4096 4.1 /
-// 11.4e-7; likewise for non-negative and half-zero operands).
+// the first three terms are computed (three MFMAs), the last is at most 2^-22 of
+// the product (2^-25 in the mean) and left out. hx hy is summed in one FP32
+// accumulator and the two small terms in another, which are added once at the
+// end: the large sum is rounded once per 16 k instead of once per 4 k as on the
+// FP32 instructions. Against 64-bit sums the result is closer than the FP32
+// instructions' at every K (2-norm error over N(0,1) operands, this / FP32 MFMA:
+// K = 64 0.98 / 1.43e-7, K = 256 1.31 / 2.87e-7, K = 1024 2.2 / 5.8e-7, K = 4096
+// 4.1 / 11.4e-7; likewise for non-negative and half-zero operands).
 //
 // Range. The scale puts the largest of a row's (column's) first nonzero slice
 // of 32 k near 2^4, so later values may be 2^12 times larger before fp16(xs)
@@ -26,22 +27,28 @@
 // A tile that shows either is computed again on the FP32 instructions before
 // anything is stored (with the FP32 rules for infinities, NaN and overflow).
 //
-// Work split: 128 x 128 output tiles, four waves, two workgroups per CU, tiles
-// dealt as in gemm.hip. A slice of 32 k of both operands is loaded into
-// registers one slice ahead (16-byte A quads, 8-byte B pairs; rows may start at
-// any 4-byte boundary), split there, and written to LDS as FP16 planes in MFMA
-// operand order (k contiguous per row of A and per column of B), two stages of
-// 32 KiB; the split costs 2.5 instructions per element, under the MFMAs of the
-// other waves. Columns are paired: thread `pair` owns columns 2 pair and
-// 2 pair + 1, held in plane rows pair and 64 + pair, so its loads and the output
-// stores of a lane are pairs of adjacent columns.
-// Tiles with few rows use layouts of 32-row blocks, so padding costs no MFMA
-// work beyond that granule.
-// Measured, FP32 instructions / this: T = 8192, E = 8, K = 4096, N = 14336 (top-2,
-// 1.92 TFLOP) 14.2 / 7.3 ms (264 TFLOP/s of FP32 products, 790 of FP16: the
-// matrix pipes are 44 % busy at the 1.5 GHz that the power limit leaves, with
-// operands of ones it runs 16 % faster); T = 16384, E = 128, K = 2048, N = 768
-// chain 1031 / 657 us.
+// Work split: output tiles of 128 columns and 128 or 256 rows on four or eight
+// waves (split_grouped picks), tiles dealt as in gemm.hip. A slice of 32 k of
+// both operands is loaded into registers one slice ahead (16-byte A quads, 8-byte
+// B pairs; rows may start at any 4-byte boundary), split there, and written to
+// LDS as FP16 planes in MFMA operand order (k contiguous per row of A and per
+// column of B), two stages; the split costs three full-rate instructions per
+// element. Columns are paired: thread `pair` owns columns 2 pair and 2 pair + 1,
+// held in plane rows pair and 64 + pair, so its loads and the output stores of a
+// lane are pairs of adjacent columns. Four waves: two workgroups share a CU and
+// one's MFMAs run under the other's staging. Eight waves: the two halves of the
+// workgroup run a phase apart, so that one has the matrix pipe while the other
+// stages. Tiles with few rows take layouts of fewer 32-row blocks.
+// Loads are buffer loads (scalar base, 32-bit lane offset): with 64-bit lane
+// addresses the eight-wave loop spilled (256 registers).
+//
+// Bound by the power limit on large problems: T = 8192, E = 8, K = 4096, N = 14336
+// (top-2, 1.92 TFLOP), FP32 instructions 14.2 ms, four waves 7.2, eight waves
+// 6.1 ms (315 TFLOP/s of FP32 products, 945 of FP16 ones; a library FP16 product
+// of random 8192 x 8192 matrices reaches 1300 on this card), and 4.5 ms with
+// operands of ones, which draw less power. Elsewhere by each tile's serial
+// parts: T = 16384, E = 128, K = 2048, N = 768 chain 1031 / 641 us, T = 2048,
+// E = 64, K = 1024, N = 512 chain 132 / 82 us.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -61,29 +68,42 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
-constexpr int kBM = 128, kBN = 128, kBK = 32;
-constexpr int kThreads = 256;
-constexpr int kPlane = 128 * kBK;           // halfs of one operand plane (8 KiB)
-constexpr int kStage = 4 * kPlane;          // A high, A low, B high, B low
+constexpr int kBN = 128, kBK = 32;
+constexpr int kPlaneB = kBN * kBK;          // halfs of one plane of B (8 KiB)
+constexpr int kBufferFlags = 0x00027000;    // raw 32-bit buffer
 constexpr int kRefLd = kBK + 1;             // FP32 recomputation: padded LDS row (floats)
-static_assert(2 * kBM * kRefLd * sizeof(float) <= 2 * kStage * sizeof(_Float16), "the FP32 slices fit the stages");
 
-// Wave tiles of TM x TN blocks of 32 x 32. kGrid: 2 x 2 waves, the wave's TN
-// = 2 column blocks being the even and the odd columns of 64; kSlab: every wave
-// takes all rows and 32 columns (lanes 0-15 the even, 16-31 the odd ones).
-template <int TM_, bool GRID, int PASSES>
+// BM x 128 output tiles on W waves (four: two workgroups per CU; eight: one).
+template <int W, int BM>
+struct Shape {
+  static constexpr int kWaves = W;
+  static constexpr int kThreads = 64 * W;
+  static constexpr int kBM = BM;
+  static constexpr int kPassRows = 8 * W;                        // rows of A staged per pass
+  static constexpr int kKPer = kBK / W;                          // k rows of B a thread stages
+  static constexpr int kPlaneA = kBM * kBK;                      // halfs
+  static constexpr int kStage = 2 * (kPlaneA + kPlaneB);         // A high, A low, B high, B low
+  static_assert((kBM + kBN) * kRefLd * sizeof(float) <= 2 * kStage * sizeof(_Float16), "the FP32 slices fit the stages");
+};
+
+// Wave tiles of TM x TN blocks of 32 x 32. GRID: W / 2 x 2 waves, the wave's TN
+// = 2 column blocks being the even and the odd columns of 64; else W / 4 x 4
+// waves of 32 columns (lanes 0-15 the even, 16-31 the odd ones).
+template <int W, int TM_, bool GRID>
 struct Layout {
   static constexpr int TM = TM_;
-  static constexpr int kPasses = PASSES;  // 32-row passes that hold the tile's rows
   static constexpr int TN = GRID ? 2 : 1;
-  __device__ static int row(int wave) { return GRID ? (wave >> 1) * 32 * TM_ : 0; }
+  static constexpr int kRows = TM_ * 32 * (GRID ? W / 2 : W / 4);
+  static constexpr int kPasses = kRows / (8 * W);  // staging passes that hold the tile's rows
+  static_assert(kPasses * (8 * W) == kRows, "whole passes");
+  __device__ static int row(int wave) { return (GRID ? wave >> 1 : wave >> 2) * 32 * TM_; }
   // plane row of the lane's column in block 0 (block 1: 64 rows further)
   __device__ static int plane_row(int wave, int li) {
-    return GRID ? 32 * (wave & 1) + li : 16 * wave + (li & 15) + 64 * (li >> 4);
+    return GRID ? 32 * (wave & 1) + li : 16 * (wave & 3) + (li & 15) + 64 * (li >> 4);
   }
   // tile column of the lane in block 0 (block 1: the next column)
   __device__ static int col(int wave, int li) {
-    return GRID ? 64 * (wave & 1) + 2 * li : 32 * wave + 2 * (li & 15) + (li >> 4);
+    return GRID ? 64 * (wave & 1) + 2 * li : 32 * (wave & 3) + 2 * (li & 15) + (li >> 4);
   }
 };
 
@@ -91,13 +111,15 @@ struct Layout {
 // 16 rows read together land in 16 distinct 16-byte bank groups.
 __device__ __forceinline__ int plane_swizzle(int r) { return (r >> 2) & 3; }
 
-// x * s = h + l (see the file comment)
+// x * s = h + l (see the file comment): six full-rate instructions for two
+// values. (Four v_fma_mixlo / mixhi_f16 would do, but they issue at half rate:
+// 9.7 against 4.7 cycles.)
 __device__ __forceinline__ void split2(float x0, float x1, float s, h2& h, h2& l) {
-  h[0] = static_cast<_Float16>(__builtin_fmaf(x0, s, 0.0F));
-  h[1] = static_cast<_Float16>(__builtin_fmaf(x1, s, 0.0F));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  h = __builtin_convertvector(f2{x0 * s, x1 * s}, h2);
   asm("" : "+v"(h));  // both halves in their register: the next two read them there
-  l[0] = static_cast<_Float16>(__builtin_fmaf(x0, s, -static_cast<float>(h[0])));
-  l[1] = static_cast<_Float16>(__builtin_fmaf(x1, s, -static_cast<float>(h[1])));
+  l = __builtin_convertvector(f2{__builtin_fmaf(x0, s, -static_cast<float>(h[0])),
+                                 __builtin_fmaf(x1, s, -static_cast<float>(h[1]))}, h2);
 }
 
 __device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFU; }
@@ -128,17 +150,20 @@ struct Tile {
 };
 struct Lds {
   _Float16* stages;  // [2][kStage]
-  int32_t* ta;       // [128] scale exponents of the rows
+  int32_t* ta;       // [kBM] scale exponents of the rows
   int32_t* tb;       // [128] ... of the plane rows of B
-  uint2* cmax;       // [4][64] column samples
-  int32_t* src;      // [128] chain: token row of X per tile row (-1: none)
-  float* w;          // [128] chain: route weight per tile row
+  uint2* cmax;       // [W][64] column samples
+  int32_t* src;      // [kBM] chain: token row of X per tile row (-1: none)
+  float* w;          // [kBM] chain: route weight per tile row
 };
 
 // One output tile for one wave layout (L::kPasses 32-row passes hold its rows).
-template <class L, bool CHAIN>
+template <class S, class L, bool CHAIN>
 __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, const Lds& sh, int col_tiles, int wave) {
+  constexpr int W = S::kWaves;
   constexpr int P = L::kPasses;
+  constexpr int PR = S::kPassRows;
+  constexpr int KP = S::kKPer;
   constexpr int TM = L::TM, TN = L::TN;
   // (the thread id passes an empty asm so that nothing of this is built before
   // the tile loop, for all four layouts, and kept live across it)
@@ -154,41 +179,52 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   const int guarded = (K % kBK != 0 || (N & 1) != 0) ? nk - 1 : nk;
   const int li = lane & 31;
   const int hi = lane >> 5;
-  // staging: A quad ac of row 32 p + ar; B columns 2 pair, 2 pair + 1 at k
-  // 8 wave .. + 7
+  // staging: A quad ac of row PR p + ar; B columns 2 pair, 2 pair + 1 at k
+  // KP wave .. + KP - 1
   const int ar = tid >> 3;
   const int ac = tid & 7;
   const int pair = lane;
   const int a_put = ar * kBK + (((ac >> 1) ^ plane_swizzle(ar)) << 3) + ((ac & 1) << 2);
-  const int b_put = pair * kBK + ((wave ^ plane_swizzle(pair)) << 3);
+  const int b_k = KP * wave;
+  const int b_put = pair * kBK + (((b_k >> 3) ^ plane_swizzle(pair)) << 3) + (b_k & 7);
 
   // Rows past the tile's last read a row that exists (their products land in
   // output rows that are never stored); columns past N the last pair.
-  const float* asrc[P];
+  // Loads take a workgroup-uniform base, a 32-bit byte offset per lane and one
+  // per instruction in a scalar register (split_gemm_fits bounds the sizes), so
+  // that the slices need no address registers or arithmetic of the lanes.
+  const auto a_base = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(CHAIN ? prm.X : prm.X + static_cast<std::size_t>(tl.row0) * K), 0, -1, kBufferFlags);
+  const auto b_base = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(tl.B), 0, -1, kBufferFlags);
+  uint32_t a_lane[P];
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int r = 32 * p + ar;
-    int src = r < rows ? tl.row0 + r : tl.row0;
+    const int r = PR * p + ar;
+    int src = r < rows ? r : 0;
     if constexpr (CHAIN) {
       src = sh.src[r];
       if (src < 0) src = 0;
     }
-    asrc[p] = prm.X + static_cast<std::size_t>(src) * K + 4 * ac;
+    a_lane[p] = 4u * (static_cast<uint32_t>(src) * static_cast<uint32_t>(K) + 4u * static_cast<uint32_t>(ac));
   }
   const int n = tl.n0 + 2 * pair;
   const int nl = n < N ? n : N - 2;
-  const uint32_t b_lane = static_cast<uint32_t>(8 * wave) * static_cast<uint32_t>(N) + static_cast<uint32_t>(nl);
+  const uint32_t b_lane = 4u * (static_cast<uint32_t>(b_k) * static_cast<uint32_t>(N) + static_cast<uint32_t>(nl));
+  auto b_row = [&](int kt, int j) {  // bytes from tl.B to its k row kBK kt + j
+    return 4u * (static_cast<uint32_t>(kt) * kBK + static_cast<uint32_t>(j)) * static_cast<uint32_t>(N);
+  };
 
   f4u ra[P];
-  f2u rb[8];
+  f2u rb[KP];
   auto load = [&](int kt) {  // whole slices
-    const float* Bk = tl.B + static_cast<std::size_t>(kt) * kBK * N;
 #pragma unroll
-    for (int p = 0; p < P; ++p) ra[p] = *reinterpret_cast<const f4u*>(asrc[p] + kt * kBK);
+    for (int p = 0; p < P; ++p) {
+      ra[p] = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(a_base, a_lane[p], 4 * kBK * kt, 0));
+    }
     // (a pair that crosses N reads the next k row's first float)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      rb[j] = *reinterpret_cast<const f2u*>(Bk + static_cast<std::size_t>(j) * N + b_lane);
+    for (int j = 0; j < KP; ++j) {
+      rb[j] = __builtin_bit_cast(f2u, __builtin_amdgcn_raw_buffer_load_b64(b_base, b_lane, b_row(kt, j), 0));
     }
   };
   auto load_any = [&](int kt) {
@@ -196,23 +232,23 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       load(kt);
       return;
     }
-    const float* Bk = tl.B + static_cast<std::size_t>(kt) * kBK * N;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         float v = 0.0F;
-        if (kt * kBK + 4 * ac + q < K) v = asrc[p][kt * kBK + q];
+        if (kt * kBK + 4 * ac + q < K) {
+          v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(a_base, a_lane[p] + 4 * q, 4 * kBK * kt, 0));
+        }
         ra[p][q] = v;
       }
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float* b = Bk + static_cast<std::size_t>(j) * N + b_lane;
+    for (int j = 0; j < KP; ++j) {
       float v0 = 0.0F, v1 = 0.0F;
-      if (kt * kBK + 8 * wave + j < K) {
-        v0 = b[0];
-        if (nl + 1 < N) v1 = b[1];
+      if (kt * kBK + b_k + j < K) {
+        v0 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b_base, b_lane, b_row(kt, j), 0));
+        if (nl + 1 < N) v1 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b_base, b_lane + 4, b_row(kt, j), 0));
       }
       rb[j] = f2u{v0, v1};
     }
@@ -234,11 +270,11 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       m = umax(m, rr::dev::dpp_move<0x4E>(m));
       m = umax(m, rr::dev::dpp_move<0x141>(m));
       if (ma[p] == 0) ma[p] = m;
-      need = need || (ma[p] == 0 && 32 * p + ar < rows);
+      need = need || (ma[p] == 0 && PR * p + ar < rows);
     }
     uint32_t c0 = 0, c1 = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < KP; ++j) {
       c0 = umax(c0, abs_bits(rb[j][0]));
       c1 = umax(c1, abs_bits(rb[j][1]));
     }
@@ -246,7 +282,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     __syncthreads();
     c0 = c1 = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < W; ++w) {
       const uint2 m = sh.cmax[64 * w + pair];
       c0 = umax(c0, m.x);
       c1 = umax(c1, m.y);
@@ -266,8 +302,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   for (int p = 0; p < P; ++p) {
     const Scale sc = scale_of(ma[p]);
     sa[p] = sc.s;
-    bad = bad || (sc.bad && 32 * p + ar < rows);
-    if (ac == 0) sh.ta[32 * p + ar] = sc.t;
+    bad = bad || (sc.bad && PR * p + ar < rows);
+    if (ac == 0) sh.ta[PR * p + ar] = sc.t;
   }
   {
     const Scale x = scale_of(mb0), y = scale_of(mb1);
@@ -290,7 +326,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       const int k = kt * kBK + 4 * ac;
 #pragma unroll
       for (int p = 0; p < P; ++p) {
-        const int r = 32 * p + ar;
+        const int r = PR * p + ar;
         if (r < rows) {
           float* out = prm.x_permuted + static_cast<std::size_t>(tl.row0 + r) * K + k;
           if (k + 4 <= K) {
@@ -311,14 +347,15 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       h2 h0, l0, h1, l1;
       split2(ra[p][0], ra[p][1], sa[p], h0, l0);
       split2(ra[p][2], ra[p][3], sa[p], h1, l1);
-      *reinterpret_cast<h4*>(st + p * 32 * kBK + a_put) = h4{h0[0], h0[1], h1[0], h1[1]};
-      *reinterpret_cast<h4*>(st + kPlane + p * 32 * kBK + a_put) = h4{l0[0], l0[1], l1[0], l1[1]};
+      *reinterpret_cast<h4*>(st + p * PR * kBK + a_put) = h4{h0[0], h0[1], h1[0], h1[1]};
+      *reinterpret_cast<h4*>(st + S::kPlaneA + p * PR * kBK + a_put) = h4{l0[0], l0[1], l1[0], l1[1]};
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      h8 h, l;
+      typedef _Float16 hk __attribute__((ext_vector_type(KP)));
+      hk h, l;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < KP / 2; ++q) {
         h2 hh, ll;
         split2(rb[2 * q][j], rb[2 * q + 1][j], j == 0 ? sb0 : sb1, hh, ll);
         h[2 * q] = hh[0];
@@ -326,8 +363,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         l[2 * q] = ll[0];
         l[2 * q + 1] = ll[1];
       }
-      *reinterpret_cast<h8*>(st + 2 * kPlane + b_put + j * 64 * kBK) = h;
-      *reinterpret_cast<h8*>(st + 3 * kPlane + b_put + j * 64 * kBK) = l;
+      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + b_put + j * 64 * kBK) = h;
+      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + kPlaneB + b_put + j * 64 * kBK) = l;
     }
   };
 
@@ -347,63 +384,114 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     const int aget = (wrow + li) * kBK, bget = prow * kBK;
     const int achunk[2] = {(hi ^ plane_swizzle(li)) << 3, ((2 + hi) ^ plane_swizzle(li)) << 3};
     const int bchunk[2] = {(hi ^ plane_swizzle(prow)) << 3, ((2 + hi) ^ plane_swizzle(prow)) << 3};
-    auto multiply = [&](const _Float16* __restrict__ st, int ks) {
+    struct Operands {
       h8 ah[TM], al[TM], bh[TN], bl[TN];
+    };
+    auto fetch = [&](const _Float16* __restrict__ st, int ks, Operands& o) {
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        ah[i] = *reinterpret_cast<const h8*>(st + aget + achunk[ks] + i * 32 * kBK);
-        al[i] = *reinterpret_cast<const h8*>(st + kPlane + aget + achunk[ks] + i * 32 * kBK);
+        o.ah[i] = *reinterpret_cast<const h8*>(st + aget + achunk[ks] + i * 32 * kBK);
+        o.al[i] = *reinterpret_cast<const h8*>(st + S::kPlaneA + aget + achunk[ks] + i * 32 * kBK);
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        bh[j] = *reinterpret_cast<const h8*>(st + 2 * kPlane + bget + bchunk[ks] + j * 64 * kBK);
-        bl[j] = *reinterpret_cast<const h8*>(st + 3 * kPlane + bget + bchunk[ks] + j * 64 * kBK);
+        o.bh[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + bget + bchunk[ks] + j * 64 * kBK);
+        o.bl[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + kPlaneB + bget + bchunk[ks] + j * 64 * kBK);
+      }
+    };
+    auto multiply = [&](const Operands& o) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.ah[i], o.bh[j], acc[i][j], 0, 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.al[i], o.bh[j], low[i][j], 0, 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], low[i][j], 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], low[i][j], 0, 0, 0);
+        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.ah[i], o.bl[j], low[i][j], 0, 0, 0);
       }
     };
     put(sh.stages);
     store_xp(0);
     if (nk > 1) load_any(1);
     __syncthreads();
-    int kt = 0;
-    // slice kt is multiplied while slice kt + 2 is on its way; slice kt + 1 has
-    // landed and goes to the other stage first, so its registers take the loads
+    // Slice kt is multiplied while slice kt + 2 is on its way; slice kt + 1 has
+    // landed and goes to the other stage, and its registers take the loads.
+    if constexpr (W == 8) {
+      // Two waves share a SIMD, one of each half of the workgroup. The halves
+      // run a phase apart: while one fetches its operands of slice kt and stages
+      // its part of slice kt + 1, the other has the matrix pipe to itself.
+      // Slice kt + 1 is complete after the second half's phase, one barrier
+      // before the first half reads it, and the stage it takes was last read
+      // one barrier before the first half writes it.
+      if (wave >= W / 2) __syncthreads();
+      auto phases = [&](int kt, auto more) {
+        const _Float16* cur = sh.stages + (kt & 1) * S::kStage;
+        Operands o0, o1;
+        fetch(cur, 0, o0);
+        fetch(cur, 1, o1);
+        more();
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(1);
+        multiply(o0);
+        multiply(o1);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+      };
+      int kt = 0;
 #pragma unroll 1
-    for (; kt + 3 < nk; ++kt) {
-      put(sh.stages + (~kt & 1) * kStage);
-      store_xp(kt + 1);
-      load(kt + 2);
-      __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to the slice's end)
-      const _Float16* cur = sh.stages + (kt & 1) * kStage;
-      multiply(cur, 0);
-      multiply(cur, 1);
-      __syncthreads();
-    }
-#pragma unroll 1
-    for (; kt < nk; ++kt) {
-      if (kt + 1 < nk) {
-        put(sh.stages + (~kt & 1) * kStage);
-        store_xp(kt + 1);
+      for (; kt + 3 < nk; ++kt) {
+        phases(kt, [&]() {
+          put(sh.stages + (~kt & 1) * S::kStage);
+          store_xp(kt + 1);
+          load(kt + 2);
+        });
       }
-      if (kt + 2 < nk) load_any(kt + 2);
-      const _Float16* cur = sh.stages + (kt & 1) * kStage;
-      multiply(cur, 0);
-      multiply(cur, 1);
-      __syncthreads();
+#pragma unroll 1
+      for (; kt < nk; ++kt) {
+        phases(kt, [&]() {
+          if (kt + 1 < nk) {
+            put(sh.stages + (~kt & 1) * S::kStage);
+            store_xp(kt + 1);
+          }
+          if (kt + 2 < nk) load_any(kt + 2);
+        });
+      }
+      if (wave < W / 2) __syncthreads();
+    } else {
+      auto both = [&](const _Float16* cur) {
+        Operands o;
+        fetch(cur, 0, o);
+        multiply(o);
+        fetch(cur, 1, o);
+        multiply(o);
+        __syncthreads();
+      };
+      int kt = 0;
+#pragma unroll 1
+      for (; kt + 3 < nk; ++kt) {
+        put(sh.stages + (~kt & 1) * S::kStage);
+        store_xp(kt + 1);
+        load(kt + 2);
+        __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to the slice's end)
+        both(sh.stages + (kt & 1) * S::kStage);
+      }
+#pragma unroll 1
+      for (; kt < nk; ++kt) {
+        if (kt + 1 < nk) {
+          put(sh.stages + (~kt & 1) * S::kStage);
+          store_xp(kt + 1);
+        }
+        if (kt + 2 < nk) load_any(kt + 2);
+        both(sh.stages + (kt & 1) * S::kStage);
+      }
     }
   }
 
@@ -496,7 +584,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       }
     }
     float* As = reinterpret_cast<float*>(sh.stages);
-    float* Bs = As + kBM * kRefLd;
+    float* Bs = As + S::kBM * kRefLd;
 #pragma unroll 1
     for (int kt = 0; kt < nk; ++kt) {
       load_any(kt);
@@ -504,12 +592,12 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll
       for (int p = 0; p < P; ++p) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) As[(32 * p + ar) * kRefLd + 4 * ac + q] = ra[p][q];
+        for (int q = 0; q < 4; ++q) As[(PR * p + ar) * kRefLd + 4 * ac + q] = ra[p][q];
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        Bs[pair * kRefLd + 8 * wave + j] = rb[j][0];
-        Bs[(64 + pair) * kRefLd + 8 * wave + j] = rb[j][1];
+      for (int j = 0; j < KP; ++j) {
+        Bs[pair * kRefLd + b_k + j] = rb[j][0];
+        Bs[(64 + pair) * kRefLd + b_k + j] = rb[j][1];
       }
       __syncthreads();
 #pragma unroll 1
@@ -528,15 +616,17 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   store_tile(!redo);
 }
 
-template <bool CHAIN>
-__global__ __launch_bounds__(kThreads, 2) void rr_split_gemm_kernel(GemmParams prm) {
+template <int W, int BM, bool CHAIN>
+__global__ __launch_bounds__(64 * W, 2) void rr_split_gemm_kernel(GemmParams prm) {
+  using S = Shape<W, BM>;
+  constexpr int kBM = BM;
   extern __shared__ __align__(16) _Float16 smem[];
   Lds sh;
   sh.stages = smem;
-  sh.ta = reinterpret_cast<int32_t*>(smem + 2 * kStage);
+  sh.ta = reinterpret_cast<int32_t*>(smem + 2 * S::kStage);
   sh.tb = sh.ta + kBM;
   sh.cmax = reinterpret_cast<uint2*>(sh.tb + kBN);
-  sh.src = reinterpret_cast<int32_t*>(sh.cmax + 4 * 64);
+  sh.src = reinterpret_cast<int32_t*>(sh.cmax + W * 64);
   sh.w = reinterpret_cast<float*>(sh.src + kBM);
   int32_t* s_off = reinterpret_cast<int32_t*>(sh.w + kBM);  // [E + 1]
   int32_t* s_pre = s_off + prm.experts + 1;                 // [E + 1] full row tiles before expert e
@@ -545,7 +635,7 @@ __global__ __launch_bounds__(kThreads, 2) void rr_split_gemm_kernel(GemmParams p
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int experts = prm.experts;
 
-  for (int e = tid; e <= experts; e += kThreads) s_off[e] = prm.offsets[e];
+  for (int e = tid; e <= experts; e += S::kThreads) s_off[e] = prm.offsets[e];
   __syncthreads();
   if (wave == 0) build_tile_prefix<kBM, true>(s_off, s_pre, s_pre2, experts, rr::dev::lane_id());
   __syncthreads();
@@ -588,58 +678,99 @@ __global__ __launch_bounds__(kThreads, 2) void rr_split_gemm_kernel(GemmParams p
       }
       __syncthreads();
     }
-    if (tl.rows > 96) {
-      run_tile<Layout<2, true, 4>, CHAIN>(prm, tl, sh, col_tiles, wave);
-    } else if (tl.rows > 64) {
-      run_tile<Layout<3, false, 3>, CHAIN>(prm, tl, sh, col_tiles, wave);
-    } else if (tl.rows > 32) {
-      run_tile<Layout<1, true, 2>, CHAIN>(prm, tl, sh, col_tiles, wave);
+    if constexpr (BM == 32 * W) {
+      if (tl.rows > BM / 4 * 3) {
+        run_tile<S, Layout<W, 2, true>, CHAIN>(prm, tl, sh, col_tiles, wave);
+        continue;
+      }
+      if (tl.rows > BM / 2) {
+        run_tile<S, Layout<W, 3, false>, CHAIN>(prm, tl, sh, col_tiles, wave);
+        continue;
+      }
+    }
+    if (tl.rows > 8 * W) {
+      run_tile<S, Layout<W, 2, false>, CHAIN>(prm, tl, sh, col_tiles, wave);
     } else {
-      run_tile<Layout<1, false, 1>, CHAIN>(prm, tl, sh, col_tiles, wave);
+      run_tile<S, Layout<W, 1, false>, CHAIN>(prm, tl, sh, col_tiles, wave);
     }
   }
 }
 
-template <bool CHAIN>
+template <int W, int BM, bool CHAIN>
 hipError_t launch(const GemmParams& prm, long rows_per_expert, int cus, hipStream_t stream) {
+  using S = Shape<W, BM>;
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(rr_split_gemm_kernel<CHAIN>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+      reinterpret_cast<const void*>(rr_split_gemm_kernel<W, BM, CHAIN>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
   if (attr != hipSuccess) return attr;
-  const long tiles = static_cast<long>(prm.experts) * ((rows_per_expert + kBM - 1) / kBM) *
+  const long bound = static_cast<long>(prm.experts) * ((rows_per_expert + BM - 1) / BM) *
                      ((static_cast<long>(prm.N) + kBN - 1) / kBN);
-  const long cap = 2L * cus;
-  long grid = tiles < cap ? tiles : cap;
+  const long cap = static_cast<long>(8 / W) * cus;
+  long grid = bound < cap ? bound : cap;
   if (grid >= kXcds) grid = grid / kXcds * kXcds;
   if (grid < 1) grid = 1;
-  const std::size_t lds = 2 * kStage * sizeof(_Float16) + (kBM + kBN) * sizeof(int32_t) + 4 * 64 * sizeof(uint2) +
-                          2 * kBM * sizeof(int32_t) + 3 * static_cast<std::size_t>(prm.experts + 1) * sizeof(int32_t);
-  rr_split_gemm_kernel<CHAIN><<<dim3(static_cast<unsigned>(grid)), kThreads, lds, stream>>>(prm);
+  const std::size_t lds = 2 * S::kStage * sizeof(_Float16) + (S::kBM + kBN) * sizeof(int32_t) +
+                          W * 64 * sizeof(uint2) + 2 * S::kBM * sizeof(int32_t) +
+                          3 * static_cast<std::size_t>(prm.experts + 1) * sizeof(int32_t);
+  rr_split_gemm_kernel<W, BM, CHAIN><<<dim3(static_cast<unsigned>(grid)), S::kThreads, lds, stream>>>(prm);
   return hipGetLastError();
 }
 
+long ceil_div(long a, long b) { return (a + b - 1) / b; }
+
+// Tiles of the rows of the whole problem plus a part tile per expert.
+long tiles(long rows, int experts, int bm, int n, int bn) { return (ceil_div(rows, bm) + experts) * ceil_div(n, bn); }
+
 }  // namespace
 
-// K >= 256 and N >= 272 (three column tiles), a tile for every CU (the rows
-// of the whole problem plus a part tile per expert), and 16 rows an expert.
-// With fewer tiles a workgroup has its CU to itself and a slice's split, LDS
-// round trip and MFMAs run one after the other, where the FP32 kernels have
-// smaller tiles; with fewer rows the call reads weights for few products and
-// the split is work on top. FP32 kernels / this one, grouped GEMM alone:
-// E = 8, K = 1024, N = 2048 with 512 rows (192 tiles) 46 / 57 us, 1024 rows
-// (256) 83 / 69 us, 4096 rows (640) 192 / 100 us; E = 16, K = 2048, N = 300
-// with 4096 rows (144) 84 / 107 us; E = 64, K = 1024, N = 512 with 2048 rows
-// (320) 46 / 48 us, 4096 rows (384) 84 / 60 us; E = 128, K = 2048, N = 768 with
-// 128 rows (one an expert) 88 / 94 us, 2048 rows 181 / 175 us, 8192 rows 387 /
-// 212 us; E = 8, K = 4096, N = 14336 with 512 rows 763 / 414 us, 4096 rows
-// 3689 / 1883 us.
+// Where the FP32 kernels stay: problems of so few tiles that their smaller
+// tiles spread over more CUs (with K >= 512, below one 64 x 64 tile a CU; with
+// shorter K, where a tile's scales and first loads weigh more, below 2.5), and
+// K < 96 or N <= 64, where neither side is bound by the matrix instructions.
+// Grouped GEMM alone, FP32 kernels / this one: E = 8, K = 1024, N = 512 with 1024
+// rows (192 tiles) 37 / 38 us, 2048 rows (320) 48 / 41, 8192 rows 106 / 70;
+// E = 16, K = 2048, N = 300 with 2048 rows (240) 66 / 65 us, 8192 rows 157 / 73;
+// E = 64, K = 512, N = 768 with 64 rows 24 / 21 us, 4096 rows 69 / 37; E = 64,
+// K = 256, N = 200 with 4096 rows (512) 17 / 19 us, 8192 rows (768) 27 / 20;
+// E = 16, K = 250, N = 1024 with 1024 rows (512) 18 / 20 us, 2048 rows (768)
+// 31 / 22; E = 64, K = 64, N = 200 with 16384 rows 18 / 18 us.
 bool split_gemm_ok(int k, int n, int experts, long rows, int cus) {
-  const long tiles = ((rows + kBM - 1) / kBM + experts) * ((static_cast<long>(n) + kBN - 1) / kBN);
-  return k >= 256 && n >= 272 && tiles >= cus && rows >= 16L * experts;
+  if (k < 96 || n <= 64) return false;
+  const long t = tiles(rows, experts, 64, n, 64);
+  return k >= 512 ? t >= cus : 2 * t >= 5L * cus;
 }
 
-hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, int cus, hipStream_t stream) {
-  return prm.sorted_route != nullptr ? launch<true>(prm, rows_per_expert, cus, stream)
-                                     : launch<false>(prm, rows_per_expert, cus, stream);
+// 32-bit byte offsets: a tile's A rows (chain: all of X) and an expert's weights.
+bool split_gemm_fits(const GemmParams& prm) {
+  const long limit = 1L << 30;
+  const long a_rows = prm.sorted_route != nullptr ? prm.dense_rows : 256;
+  return prm.K > 0 && prm.N >= 2 && a_rows * prm.K < limit && static_cast<long>(prm.K + kBK) * prm.N < limit;
+}
+
+// Workgroup shape:
+//  - eight waves on 128-row tiles where a CU gets hardly more than one tile:
+//    more waves for it (E = 16, K = 2048, N = 300 with 8192 rows, 240 tiles: 73 us
+//    against 116 with four waves; E = 64, K = 1024, N = 512, 4096 rows, 384
+//    tiles: 40 / 59; 8192 rows, 512 tiles: 64 / 68; E = 64, K = 512, N = 768,
+//    512 rows, 408 tiles: 32 / 25);
+//  - eight waves on 256-row tiles where there are many of them and the experts
+//    have the rows (E = 8, K = 4096, N = 8192 with 16384 rows 3.45 ms against
+//    3.92; E = 64, K = 1024, N = 512, 256 rows an expert: 86 / 94 us uniform,
+//    95 / 102 skewed, but E = 64, K = 512, N = 768, 256 rows an expert: 86 / 74).
+//    Not for the chain: nothing runs under a tile's combine with one workgroup
+//    a CU (T = 16384, E = 128, K = 2048, N = 768 chain 724 against 641 us);
+//  - else four waves on 128-row tiles, two workgroups a CU.
+hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, long rows, int cus, hipStream_t stream) {
+  const bool chain = prm.sorted_route != nullptr;
+  if (2 * tiles(rows, prm.experts, 128, prm.N, kBN) <= 3L * cus) {
+    return chain ? launch<8, 128, true>(prm, rows_per_expert, cus, stream)
+                 : launch<8, 128, false>(prm, rows_per_expert, cus, stream);
+  }
+  if (chain) return launch<4, 128, true>(prm, rows_per_expert, cus, stream);
+  if (prm.K >= 512 && tiles(rows, prm.experts, 256, prm.N, kBN) >= 2L * cus &&
+      rows * prm.K >= (1L << 18) * prm.experts) {
+    return launch<8, 256, false>(prm, rows_per_expert, cus, stream);
+  }
+  return launch<4, 128, false>(prm, rows_per_expert, cus, stream);
 }
 
 }  // namespace rr::kern

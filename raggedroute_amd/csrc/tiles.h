@@ -21,7 +21,7 @@ struct GemmParams {
   const int32_t* offsets;
   float* Y;
   int experts;
-  int dense_rows;
+  int dense_rows;  // dense: rows of the one segment; chain: rows of X
   int K;
   int N;
   // chain: segment row r holds token sorted_route[r] / top_k of X; the
