@@ -27,8 +27,15 @@ using rr::dev::wave_lds_sync;
 
 constexpr int kBlock = 1024;  // 16 waves
 constexpr int kWavesPerBlock = kBlock / 64;
-// Route counts up to this size take the single-workgroup metadata kernels.
-constexpr int kSingleBlockRoutes = 65536;
+// Histograms of up to this many routes take the single-workgroup kernel. It has
+// 1024 threads for all ids; the two launches of the other path take 6.8-7.0 us at
+// every size below. Uniform ids, single workgroup: E = 256 4.5 us at 32768
+// routes, 5.7 at 49152; E = 64 5.2 / 6.6 (8.1 at 65536); E = 8 (many lanes of an
+// LDS atomic on one bin) 6.5 at 24000, 8.2 at 32768, 11.2 at 49152. Half of the ids
+// on one expert, E = 64, before the ballots below / with them: 16384 routes 9.0 /
+// 3.7 us, 32768 15.8 / 5.1, 65536 (then still single) 29.5 / 7.0; uniform ids
+// E = 256, 24000 routes 3.7 / 4.0.
+constexpr int single_block_routes(int experts) { return experts < 32 ? 24576 : 49152; }
 
 bool aligned16(const void* p) { return (reinterpret_cast<std::uintptr_t>(p) & 15u) == 0; }
 
@@ -137,6 +144,64 @@ __device__ __forceinline__ void wave_count_ids(int32_t* row, const int32_t* __re
   }
 }
 
+// The same for a whole histogram [0, routes), ids in quads (16-byte loads that
+// need 4-byte alignment), and for ids that crowd one expert: a wave whose first
+// 64 ids hold one expert on at least 12 lanes counts that expert with a ballot
+// per load instead of 64 lanes adding to one address. (Not in the recounts of the
+// permute ranks and of route preparation, where the probe alone cost 0.6 us of
+// the post-route chain T = 8192, top_k = 8.)
+__device__ __forceinline__ void wave_histogram(int32_t* row, const int32_t* __restrict__ ids, int routes,
+                                               int experts, int wave, int waves) {
+  typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int kQuads = 2;
+  const int lane = lane_id();
+  int hot = -1;       // the wave's dominant expert (-1: none)
+  int32_t hot_n = 0;  // its ids so far (wave-uniform)
+  bool probed = false;
+  for (int base = wave * 256; base < routes; base += waves * 256 * kQuads) {
+    i4u v[kQuads];
+#pragma unroll
+    for (int u = 0; u < kQuads; ++u) {
+      const int r = base + u * waves * 256 + 4 * lane;
+      if (r + 4 <= routes) {
+        v[u] = *reinterpret_cast<const i4u*>(ids + r);
+      } else {
+        v[u] = i4u{-1, -1, -1, -1};
+        for (int k = 0; r + k < routes; ++k) v[u][k] = ids[r + k];
+      }
+    }
+    if (!probed) {
+      probed = true;
+      int best = 11;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int cand = __builtin_amdgcn_readlane(v[0].x, 16 * k);
+        const int n = __popcll(__ballot(v[0].x == cand));
+        if (static_cast<unsigned>(cand) < static_cast<unsigned>(experts) && n > best) {
+          best = n;
+          hot = cand;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kQuads; ++u) {
+      if (hot >= 0) {  // (wave-uniform)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          hot_n += __popcll(__ballot(v[u][k] == hot));
+          if (v[u][k] != hot && static_cast<unsigned>(v[u][k]) < static_cast<unsigned>(experts)) atomicAdd(row + v[u][k], 1);
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (static_cast<unsigned>(v[u][k]) < static_cast<unsigned>(experts)) atomicAdd(row + v[u][k], 1);
+        }
+      }
+    }
+  }
+  if (hot >= 0 && lane == 0) atomicAdd(row + hot, hot_n);
+}
+
 // Number of LDS histogram rows: one per wave while 16 rows fit in 32 KB.
 __host__ __device__ __forceinline__ int private_rows(int experts) {
   return experts <= 512 ? kWavesPerBlock : kWavesPerBlock / 2;
@@ -176,7 +241,7 @@ __global__ __launch_bounds__(kBlock) void rr_hist_scan_single_kernel(
   const int wave = tid >> 6;
   for (int i = tid; i < rows * experts; i += kBlock) bins[i] = 0;
   __syncthreads();
-  wave_count_ids(bins + (wave % rows) * experts, ids, 0, routes, experts, wave, kWavesPerBlock);
+  wave_histogram(bins + (wave % rows) * experts, ids, routes, experts, wave, kWavesPerBlock);
   __syncthreads();
   // experts <= kBlock: thread e owns expert e.
   int32_t c = 0;
@@ -1429,7 +1494,7 @@ hipError_t histogram_native(const int32_t* ids, int32_t* counts, int routes, int
     rr_single_bin_kernel<<<1, 1, 0, stream>>>(counts, nullptr, routes);
     return hipGetLastError();
   }
-  if (routes <= kSingleBlockRoutes) {
+  if (routes <= single_block_routes(experts)) {
     rr_hist_scan_single_kernel<<<1, kBlock, bins_bytes(experts), stream>>>(
         ids, counts, nullptr, routes, experts);
     return hipGetLastError();
@@ -1449,7 +1514,7 @@ hipError_t histogram_exclusive_scan_native(const int32_t* ids, int32_t* counts, 
     rr_single_bin_kernel<<<1, 1, 0, stream>>>(counts, offsets, routes);
     return hipGetLastError();
   }
-  if (routes <= kSingleBlockRoutes) {
+  if (routes <= single_block_routes(experts)) {
     rr_hist_scan_single_kernel<<<1, kBlock, bins_bytes(experts), stream>>>(
         ids, counts, offsets, routes, experts);
     return hipGetLastError();
