@@ -924,6 +924,13 @@ hipError_t gemm_dispatch(const GemmParams& prm, long rows_per_expert, long total
   return launch_tile<TileNarrow, MODE>(prm, rows_per_expert, stream);
 }
 
+// Dense GEMMs of at most 128 columns that the strip kernel does not cover, up
+// to the row count from which the large tile has two tiles per CU.
+bool narrow_chosen(int m, int n, int k) {
+  return narrow_gemm_ok(m, n, k) &&
+         tile_estimate(m, 0, TileLarge::BM, n, TileLarge::BN) < 2L * device_cu_count();
+}
+
 GemmParams base_params(const float* x, const float* w, const int32_t* offsets, float* y,
                        int experts, int dense_rows, int K, int N) {
   GemmParams p{};
@@ -944,7 +951,14 @@ hipError_t dense_gemm_mfma(const float* a, const float* b, float* c, int m, int 
                            hipStream_t stream) {
   if (m <= 0 || n <= 0) return hipSuccess;
   if (tile_override() == 0 && strip_shape_ok(k, n, a, b)) return strip_dense(a, b, c, m, n, k, stream);
+  if (tile_override() == 0 && narrow_chosen(m, n, k)) {
+    return narrow_gemm(a, b, c, m, n, k, nullptr, nullptr, nullptr, 0, device_cu_count(), stream);
+  }
   return gemm_dispatch<kDense>(base_params(a, b, nullptr, c, 1, m, k, n), m, m, stream);
+}
+
+bool router_gate_ok(int tokens, int experts, int hidden, const float* x, const float* router_weights) {
+  return experts <= 128 && (strip_shape_ok(hidden, experts, x, router_weights) || narrow_chosen(tokens, experts, hidden));
 }
 
 hipError_t grouped_gemm_mfma(const float* x, const float* w, const int32_t* offsets, float* y,
@@ -966,9 +980,13 @@ hipError_t router_gate_mfma(const float* x, const float* router_weights, float* 
                             int32_t* ids, float* gate_weights, float* y_zero, int y_cols,
                             int tokens, int experts, int hidden, hipStream_t stream) {
   if (tokens <= 0) return hipSuccess;
-  // The strip kernel carries the gate epilogue (E <= 128, K <= 256); callers
-  // run the dense GEMM and the gate kernel for other shapes.
-  if (experts > 128 || !strip_shape_ok(hidden, experts, x, router_weights)) return hipErrorInvalidValue;
+  // The strip kernel and the narrow kernel carry the gate epilogue; callers run
+  // the dense GEMM and the gate kernel for other shapes.
+  if (!router_gate_ok(tokens, experts, hidden, x, router_weights)) return hipErrorInvalidValue;
+  if (!strip_shape_ok(hidden, experts, x, router_weights)) {
+    return narrow_gemm(x, router_weights, logits, tokens, experts, hidden, ids, gate_weights, y_zero, y_cols,
+                       device_cu_count(), stream);
+  }
   return strip_router_gate(x, router_weights, logits, ids, gate_weights, y_zero, y_cols, tokens,
                            experts, hidden, stream);
 }

@@ -19,9 +19,11 @@ hipError_t grouped_gemm_mfma(const float* x, const float* w, const int32_t* offs
                              hipStream_t stream);
 
 // ---- fused chain forms (gemm.hip) ----
+// Whether router_gate_mfma takes this shape.
+bool router_gate_ok(int tokens, int experts, int hidden, const float* x, const float* router_weights);
 // logits = x * router_weights with each row's top-2 ids / weights taken in the
-// epilogue; rows [0, tokens) of y_zero ([tokens, y_cols]) are zeroed. Strip
-// shapes only (E <= 128, K <= 256); hipErrorInvalidValue otherwise.
+// epilogue; rows [0, tokens) of y_zero ([tokens, y_cols]) are zeroed. Shapes of
+// router_gate_ok only; hipErrorInvalidValue otherwise.
 hipError_t router_gate_mfma(const float* x, const float* router_weights, float* logits,
                             int32_t* ids, float* gate_weights, float* y_zero, int y_cols,
                             int tokens, int experts, int hidden, hipStream_t stream);
@@ -33,6 +35,13 @@ hipError_t chain_grouped_mfma(const float* x, const float* expert_weights, const
                               const int32_t* sorted_route, const float* route_weights,
                               float* x_permuted, float* y_permuted, float* y, int tokens,
                               int top_k, int experts, int hidden, int output, hipStream_t stream);
+
+// ---- dense GEMM of at most 128 columns, any K and alignment (narrow.hip) ----
+bool narrow_gemm_ok(int m, int n, int k);
+// c = a * b; with gate_ids given also every row's top-2 ids / weights, and rows
+// [0, m) of y_zero ([m, y_cols], optional) zeroed.
+hipError_t narrow_gemm(const float* a, const float* b, float* c, int m, int n, int k, int32_t* gate_ids,
+                       float* gate_weights, float* y_zero, int y_cols, int cus, hipStream_t stream);
 
 // ---- narrow-output strip GEMMs (strip.hip): N <= 128, K <= 256 ----
 // Shape / alignment test shared by the strip entries (K and N multiples of 4,
