@@ -33,9 +33,7 @@
 // B pairs; rows may start at any 4-byte boundary), split there, and written to
 // LDS as FP16 planes in MFMA operand order (k contiguous per row of A and per
 // column of B), two stages; the split costs three full-rate instructions per
-// element. Columns are paired: thread `pair` owns columns 2 pair and 2 pair + 1,
-// held in plane rows pair and 64 + pair, so its loads and the output stores of a
-// lane are pairs of adjacent columns. Four waves: two workgroups share a CU and
+// element. Four waves: two workgroups share a CU and
 // one's MFMAs run under the other's staging. Eight waves: the two halves of the
 // workgroup run a phase apart, so that one has the matrix pipe while the other
 // stages. Tiles with few rows take layouts of fewer 32-row blocks.
@@ -86,9 +84,8 @@ struct Shape {
   static_assert((kBM + kBN) * kRefLd * sizeof(float) <= 2 * kStage * sizeof(_Float16), "the FP32 slices fit the stages");
 };
 
-// Wave tiles of TM x TN blocks of 32 x 32. GRID: W / 2 x 2 waves, the wave's TN
-// = 2 column blocks being the even and the odd columns of 64; else W / 4 x 4
-// waves of 32 columns (lanes 0-15 the even, 16-31 the odd ones).
+// Wave tiles of TM x TN blocks of 32 x 32. GRID: W / 2 x 2 waves of TN = 2 column
+// blocks; else W / 4 x 4 waves of one.
 template <int W, int TM_, bool GRID>
 struct Layout {
   static constexpr int TM = TM_;
@@ -97,14 +94,8 @@ struct Layout {
   static constexpr int kPasses = kRows / (8 * W);  // staging passes that hold the tile's rows
   static_assert(kPasses * (8 * W) == kRows, "whole passes");
   __device__ static int row(int wave) { return (GRID ? wave >> 1 : wave >> 2) * 32 * TM_; }
-  // plane row of the lane's column in block 0 (block 1: 64 rows further)
-  __device__ static int plane_row(int wave, int li) {
-    return GRID ? 32 * (wave & 1) + li : 16 * (wave & 3) + (li & 15) + 64 * (li >> 4);
-  }
-  // tile column of the lane in block 0 (block 1: the next column)
-  __device__ static int col(int wave, int li) {
-    return GRID ? 64 * (wave & 1) + 2 * li : 32 * (wave & 3) + 2 * (li & 15) + (li >> 4);
-  }
+  // first tile column (plane row of B)
+  __device__ static int col(int wave) { return GRID ? 64 * (wave & 1) : 32 * (wave & 3); }
 };
 
 // 16-byte chunk c (8 halfs) of plane row r sits at chunk c ^ ((r >> 2) & 3): the
@@ -186,7 +177,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   const int pair = lane;
   const int a_put = ar * kBK + (((ac >> 1) ^ plane_swizzle(ar)) << 3) + ((ac & 1) << 2);
   const int b_k = KP * wave;
-  const int b_put = pair * kBK + (((b_k >> 3) ^ plane_swizzle(pair)) << 3) + (b_k & 7);
+  const int b_put = 2 * pair * kBK + (((b_k >> 3) ^ plane_swizzle(2 * pair)) << 3) + (b_k & 7);
 
   // Rows past the tile's last read a row that exists (their products land in
   // output rows that are never stored); columns past N the last pair.
@@ -311,8 +302,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     sb1 = y.s;
     bad = bad || (x.bad && n < N) || (y.bad && n + 1 < N);
     if (wave == 0) {
-      sh.tb[pair] = x.t;
-      sh.tb[64 + pair] = y.t;
+      sh.tb[2 * pair] = x.t;
+      sh.tb[2 * pair + 1] = y.t;
     }
   }
 
@@ -363,8 +354,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         l[2 * q] = ll[0];
         l[2 * q + 1] = ll[1];
       }
-      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + b_put + j * 64 * kBK) = h;
-      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + kPlaneB + b_put + j * 64 * kBK) = l;
+      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + b_put + j * kBK) = h;
+      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + kPlaneB + b_put + j * kBK) = l;
     }
   };
 
@@ -379,7 +370,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     }
   }
   {
-    const int prow = L::plane_row(wave, li);
+    const int prow = L::col(wave) + li;
     // operand chunk of k step ks: k = 16 ks + 8 hi .. + 7
     const int aget = (wrow + li) * kBK, bget = prow * kBK;
     const int achunk[2] = {(hi ^ plane_swizzle(li)) << 3, ((2 + hi) ^ plane_swizzle(li)) << 3};
@@ -395,8 +386,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        o.bh[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + bget + bchunk[ks] + j * 64 * kBK);
-        o.bl[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + kPlaneB + bget + bchunk[ks] + j * 64 * kBK);
+        o.bh[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + bget + bchunk[ks] + j * 32 * kBK);
+        o.bl[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + kPlaneB + bget + bchunk[ks] + j * 32 * kBK);
       }
     };
     auto multiply = [&](const Operands& o) {
@@ -502,12 +493,12 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   const int eli = ln & 31;
   const int ehi = ln >> 5;
   // output rows of accumulator register r: 32 i + 8 (r / 4) + 4 hi + r % 4 of the wave's
-  const int col = tl.n0 + L::col(wave, eli);
-  const int prow = L::plane_row(wave, eli);
+  const int col = tl.n0 + L::col(wave) + eli;  // block j: 32 j further
+  const int prow = L::col(wave) + eli;
   auto store_tile = [&](bool scaled) {
     int tb[TN];
 #pragma unroll
-    for (int j = 0; j < TN; ++j) tb[j] = sh.tb[prow + 64 * j];
+    for (int j = 0; j < TN; ++j) tb[j] = sh.tb[prow + 32 * j];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -527,33 +518,17 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
             w = sh.w[rl];
           }
         }
-        auto put1 = [&](int j) {
-          if (comb != nullptr) {
-            __builtin_nontemporal_store(v[j], yrow + j);  // y_permuted is not read again by the chain
-          } else {
-            yrow[j] = v[j];
-          }
-        };
-        if constexpr (TN == 2) {
-          if (col + 1 < N) {
-            if (comb != nullptr) {
-              __builtin_nontemporal_store(f2u{v[0], v[1]}, reinterpret_cast<f2u*>(yrow));
-            } else {
-              *reinterpret_cast<f2u*>(yrow) = f2u{v[0], v[1]};
-            }
-          } else if (col < N) {
-            put1(0);
-          }
-        } else if (col < N) {
-          put1(0);
-        }
-        if (comb != nullptr) {
-          // Both routes of a token add into the zeroed output: fl(0 + a) + b
-          // is the same in either order, so the combine is deterministic
-          // and equals the rank-order unpermute.
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            if (col + j < N) unsafeAtomicAdd(comb + j, __fmul_rn(w, v[j]));
+        for (int j = 0; j < TN; ++j) {
+          if (col + 32 * j >= N) continue;
+          if (comb != nullptr) {
+            __builtin_nontemporal_store(v[j], yrow + 32 * j);  // y_permuted is not read again by the chain
+            // Both routes of a token add into the zeroed output: fl(0 + a) + b
+            // is the same in either order, so the combine is deterministic
+            // and equals the rank-order unpermute.
+            unsafeAtomicAdd(comb + 32 * j, __fmul_rn(w, v[j]));
+          } else {
+            yrow[32 * j] = v[j];
           }
         }
       }
@@ -568,7 +543,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       for (int r = 0; r < 16; ++r) {
         const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
         acc[i][j][r] += low[i][j][r];
-        overflow = overflow || (rl < rows && col + j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
+        overflow = overflow || (rl < rows && col + 32 * j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
       }
     }
   }
@@ -596,8 +571,8 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       }
 #pragma unroll
       for (int j = 0; j < KP; ++j) {
-        Bs[pair * kRefLd + b_k + j] = rb[j][0];
-        Bs[(64 + pair) * kRefLd + b_k + j] = rb[j][1];
+        Bs[2 * pair * kRefLd + b_k + j] = rb[j][0];
+        Bs[(2 * pair + 1) * kRefLd + b_k + j] = rb[j][1];
       }
       __syncthreads();
 #pragma unroll 1
@@ -607,7 +582,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
           const float a = As[(wrow + 32 * i + eli) * kRefLd + k + ehi];
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, Bs[(prow + 64 * j) * kRefLd + k + ehi], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, Bs[(prow + 32 * j) * kRefLd + k + ehi], acc[i][j], 0, 0, 0);
           }
         }
       }
@@ -725,7 +700,9 @@ long tiles(long rows, int experts, int bm, int n, int bn) { return (ceil_div(row
 // Where the FP32 kernels stay: problems of so few tiles that their smaller
 // tiles spread over more CUs (with K >= 512, below one 64 x 64 tile a CU; with
 // shorter K, where a tile's scales and first loads weigh more, below 2.5), and
-// K < 96 or N <= 64, where neither side is bound by the matrix instructions.
+// K < 128 or N <= 64, where neither side is bound by the matrix instructions, and
+// K and N both below 256 (chain T = 10296, E = 12, K = 100, N = 153 53 / 59 us, T =
+// 2523, E = 10, K = 106, N = 667 49 / 53; T = 14884, E = 75, K = 128, N = 608 125 / 112).
 // Grouped GEMM alone, FP32 kernels / this one: E = 8, K = 1024, N = 512 with 1024
 // rows (192 tiles) 37 / 38 us, 2048 rows (320) 48 / 41, 8192 rows 106 / 70;
 // E = 16, K = 2048, N = 300 with 2048 rows (240) 66 / 65 us, 8192 rows 157 / 73;
@@ -734,7 +711,7 @@ long tiles(long rows, int experts, int bm, int n, int bn) { return (ceil_div(row
 // E = 16, K = 250, N = 1024 with 1024 rows (512) 18 / 20 us, 2048 rows (768)
 // 31 / 22; E = 64, K = 64, N = 200 with 16384 rows 18 / 18 us.
 bool split_gemm_ok(int k, int n, int experts, long rows, int cus) {
-  if (k < 96 || n <= 64) return false;
+  if (k < 128 || n <= 64 || (k < 256 && n < 256)) return false;
   const long t = tiles(rows, experts, 64, n, 64);
   return k >= 512 ? t >= cus : 2 * t >= 5L * cus;
 }

@@ -51,7 +51,7 @@ EDGE_ROWS = [0, 1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 192, 193, 
     ([9] * 130, 256, 300, 0),              # more tiles than workgroups per XCD
     ([3] * 1024, 256, 272, 0),             # E = 1024
     # four waves (more than 1.5 tiles a CU), every layout
-    (EDGE_ROWS, 100, 1701, 1),
+    (EDGE_ROWS, 130, 1701, 1),
     # 256-row tiles (experts with the rows, two tiles a CU), every layout
     ([513, 700, 767, 1, 300, 1100], 515, 3301, 1),
     ([513, 447, 448, 576, 640, 832], 544, 3328, 0),
