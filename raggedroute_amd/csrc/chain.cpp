@@ -122,8 +122,11 @@ rr_status run_fused(const rr_chain_args* a, const rr_runtime_context& ctx, bool 
     return ok_status();
   }
   if (only < 0 || only == 1) {
+    // (scratch: y_permuted, whose every row the expert GEMM writes: the gate
+    // leaves no route without an expert)
     err = kern::route_prep(a->expert_ids, a->counts, a->offsets, cursors, a->route_pos,
-                           sorted_route, routes, a->experts, ctx.stream);
+                           sorted_route, routes, a->experts, a->y_permuted,
+                           static_cast<std::size_t>(routes) * a->output * sizeof(float), ctx.stream);
     if (err != hipSuccess) return device_status(err, "chain route preparation launch failed");
   }
   if (only < 0 || only == 2) {
@@ -297,8 +300,11 @@ rr_status run_route_chain_fused(const rr_route_chain_args* a,
                             a->output, ctx.stream);
     if (err != hipSuccess) return device_status(err, "route chain expert GEMM launch failed");
   } else {
+    // (scratch: y, whose every row the unpermute writes; rows of y_permuted
+    // without a route keep what the caller put there)
     err = kern::route_prep(a->expert_ids, a->counts, a->offsets, cursors, a->route_pos,
-                           sorted_route, routes, a->experts, ctx.stream);
+                           sorted_route, routes, a->experts, a->y,
+                           static_cast<std::size_t>(a->tokens) * a->output * sizeof(float), ctx.stream);
     if (err != hipSuccess) return device_status(err, "route chain preparation launch failed");
     err = kern::chain_grouped_mfma(a->x, a->expert_weights, a->offsets, sorted_route,
                                    a->route_weights, a->x_permuted, a->y_permuted, nullptr,

@@ -997,6 +997,11 @@ hipError_t chain_grouped_mfma(const float* x, const float* expert_weights, const
                               int top_k, int experts, int hidden, int output, hipStream_t stream) {
   if (tokens <= 0 || output <= 0) return hipSuccess;
   if (y != nullptr && top_k != 2) return hipErrorInvalidValue;  // combine is top-2 only
+  if (tile_override() == 0 && strip_gather_ok(static_cast<long>(tokens) * top_k, top_k, experts, hidden, output, x,
+                                              expert_weights, x_permuted)) {
+    return strip_gather(x, expert_weights, offsets, sorted_route, route_weights, x_permuted, y_permuted, y,
+                        tokens, top_k, experts, hidden, output, stream);
+  }
   GemmParams p = base_params(x, expert_weights, offsets, y_permuted, experts, tokens, hidden, output);
   p.sorted_route = sorted_route;
   p.route_weights = route_weights;

@@ -53,6 +53,14 @@ bool strip_segments_ok(int segments);
 // the route-id stage to fit in LDS.
 bool strip_chain_ok(int tokens, int top_k, int experts, int k, int n, const void* x,
                     const void* w, const void* ids, const void* x_permuted);
+// The expert GEMM of a chain over rows gathered through sorted_route (offsets and
+// sorted_route prepared before): chain_grouped_mfma's work on the strip kernel.
+bool strip_gather_ok(long routes, int top_k, int experts, int k, int n, const void* x, const void* w,
+                     const void* x_permuted);
+hipError_t strip_gather(const float* x, const float* expert_weights, const int32_t* offsets,
+                        const int32_t* sorted_route, const float* route_weights, float* x_permuted,
+                        float* y_permuted, float* y, int tokens, int top_k, int experts, int hidden,
+                        int output, hipStream_t stream);
 hipError_t strip_dense(const float* a, const float* b, float* c, int m, int n, int k,
                        hipStream_t stream);
 // rows_bound: upper bound on the total segment rows (sizes the grid only).
@@ -91,10 +99,12 @@ hipError_t token_permute_stable(const float* x, const int32_t* ids, const int32_
                                 int32_t* sorted_route, int tokens, int experts, int top_k,
                                 int hidden, hipStream_t stream);
 // Fused-chain route preparation: ids -> counts, offsets, stable route_pos,
-// sorted_route (required here) and cursors in one launch.
+// sorted_route (required here) and cursors. scratch (optional): device memory
+// that a later launch of the same call overwrites whole, 4-byte aligned; with
+// room for the counts of every chunk large problems take two launches.
 hipError_t route_prep(const int32_t* ids, int32_t* counts, int32_t* offsets, int32_t* cursors,
                       int32_t* route_pos, int32_t* sorted_route, int routes, int experts,
-                      hipStream_t stream);
+                      void* scratch, std::size_t scratch_bytes, hipStream_t stream);
 // Token-owned row copy x -> x_permuted through route_pos (second half of token_permute).
 hipError_t permute_copy(const float* x, const int32_t* route_pos, float* x_permuted, int tokens,
                         int top_k, int hidden, hipStream_t stream);

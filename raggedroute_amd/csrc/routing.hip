@@ -30,12 +30,12 @@ constexpr int kWavesPerBlock = kBlock / 64;
 // Histograms of up to this many routes take the single-workgroup kernel. It has
 // 1024 threads for all ids; the two launches of the other path take 6.8-7.0 us at
 // every size below. Uniform ids, single workgroup: E = 256 4.5 us at 32768
-// routes, 5.7 at 49152; E = 64 5.2 / 6.6 (8.1 at 65536); E = 8 (many lanes of an
+// routes, 5.7 at 49152, 6.8 at 65536; E = 64 5.2 / 6.6 / 8.1; E = 8 (many lanes of an
 // LDS atomic on one bin) 6.5 at 24000, 8.2 at 32768, 11.2 at 49152. Half of the ids
 // on one expert, E = 64, before the ballots below / with them: 16384 routes 9.0 /
 // 3.7 us, 32768 15.8 / 5.1, 65536 (then still single) 29.5 / 7.0; uniform ids
 // E = 256, 24000 routes 3.7 / 4.0.
-constexpr int single_block_routes(int experts) { return experts < 32 ? 24576 : 49152; }
+constexpr int single_block_routes(int experts) { return experts < 32 ? 24576 : (experts < 128 ? 49152 : 65536); }
 
 bool aligned16(const void* p) { return (reinterpret_cast<std::uintptr_t>(p) & 15u) == 0; }
 
@@ -562,17 +562,35 @@ __global__ __launch_bounds__(WAVES * 64) void rr_permute_rank_kernel(
   }
 }
 
+// Counts the ids of each chunk of kBlock routes: block_counts[b * experts + e].
+__global__ __launch_bounds__(kBlock) void rr_route_count_kernel(const int32_t* __restrict__ ids,
+                                                                int32_t* __restrict__ block_counts,
+                                                                int routes, int experts) {
+  extern __shared__ int32_t lds[];  // [experts]
+  const int tid = static_cast<int>(threadIdx.x);
+  const int r = static_cast<int>(blockIdx.x) * kBlock + tid;
+  const int id = r < routes ? ids[r] : -1;
+  for (int e = tid; e < experts; e += kBlock) lds[e] = 0;
+  __syncthreads();
+  if (static_cast<unsigned>(id) < static_cast<unsigned>(experts)) atomicAdd(lds + id, 1);
+  __syncthreads();
+  for (int e = tid; e < experts; e += kBlock) block_counts[static_cast<std::size_t>(blockIdx.x) * experts + e] = lds[e];
+}
+
 // Route preparation for the fused chain: ids -> counts, offsets, stable
-// route_pos, sorted_route and cursors in one launch. Block b ranks routes
+// route_pos, sorted_route and cursors. Block b ranks routes
 // [b*chunk, (b+1)*chunk) like rr_permute_rank_kernel, but derives the offsets
-// itself: it counts every route per expert (routes before its chunk give the
-// stable base, all routes give the totals) and scans the totals in LDS, so no
-// block waits for another. LDS: (WAVES + 2) * E + 1 + 16 ints.
-template <int WAVES>
+// itself, so no block waits for another: COUNTED, from the counts of every
+// chunk (rr_route_count_kernel, chunk = kBlock); else it counts every route per
+// expert (routes before its chunk give the stable base, all routes give the
+// totals). The totals are scanned in LDS. LDS: (WAVES + 2) * E + 1 + 16 ints,
+// COUNTED WAVES * E more.
+template <int WAVES, bool COUNTED>
 __global__ __launch_bounds__(WAVES * 64) void rr_route_prep_kernel(
-    const int32_t* __restrict__ ids, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-    int32_t* __restrict__ cursors, int32_t* __restrict__ route_pos,
-    int32_t* __restrict__ sorted_route, int routes, int experts, int bits, int chunk) {
+    const int32_t* __restrict__ ids, const int32_t* __restrict__ block_counts,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ cursors,
+    int32_t* __restrict__ route_pos, int32_t* __restrict__ sorted_route, int routes, int experts,
+    int bits, int chunk) {
   constexpr int kThreads = WAVES * 64;
   extern __shared__ int32_t lds[];
   int32_t* wc = lds;                       // [WAVES][experts]
@@ -585,28 +603,57 @@ __global__ __launch_bounds__(WAVES * 64) void rr_route_prep_kernel(
   const int begin = static_cast<int>(blockIdx.x) * chunk;
   const int end = begin + chunk < routes ? begin + chunk : routes;
 
-  for (int i = tid; i < WAVES * experts; i += kThreads) wc[i] = 0;
-  __syncthreads();
-  wave_count_ids(wc + wave * experts, ids, 0, begin, experts, wave, WAVES);
-  __syncthreads();
-  for (int e = tid; e < experts; e += kThreads) {
-    int32_t sum = 0;
-    for (int w = 0; w < WAVES; ++w) {
-      sum += wc[w * experts + e];
-      wc[w * experts + e] = 0;
+  if constexpr (COUNTED) {
+    // wave w sums the chunks w, w + WAVES, ...
+    int32_t* wb = wsum + kWavesPerBlock;  // [WAVES][experts]: of the chunks before mine
+    const int blocks = static_cast<int>(gridDim.x);
+    const int mine = static_cast<int>(blockIdx.x);
+    for (int e = lane; e < experts; e += 64) {
+      int32_t all = 0, before = 0;
+#pragma unroll 4
+      for (int b = wave; b < blocks; b += WAVES) {
+        const int32_t c = block_counts[static_cast<std::size_t>(b) * experts + e];
+        all += c;
+        before += b < mine ? c : 0;
+      }
+      wc[wave * experts + e] = all;
+      wb[wave * experts + e] = before;
     }
-    base[e] = sum;
-  }
-  __syncthreads();
-  wave_count_ids(wc + wave * experts, ids, begin, routes, experts, wave, WAVES);
-  __syncthreads();
-  for (int e = tid; e < experts; e += kThreads) {
-    int32_t sum = base[e];
-    for (int w = 0; w < WAVES; ++w) {
-      sum += wc[w * experts + e];
-      wc[w * experts + e] = 0;
+    __syncthreads();
+    for (int e = tid; e < experts; e += kThreads) {
+      int32_t all = 0, before = 0;
+      for (int w = 0; w < WAVES; ++w) {
+        all += wc[w * experts + e];
+        before += wb[w * experts + e];
+        wc[w * experts + e] = 0;
+      }
+      soff[e] = all;  // total count; scanned in place below
+      base[e] = before;
     }
-    soff[e] = sum;  // total count; scanned in place below
+  } else {
+    for (int i = tid; i < WAVES * experts; i += kThreads) wc[i] = 0;
+    __syncthreads();
+    wave_count_ids(wc + wave * experts, ids, 0, begin, experts, wave, WAVES);
+    __syncthreads();
+    for (int e = tid; e < experts; e += kThreads) {
+      int32_t sum = 0;
+      for (int w = 0; w < WAVES; ++w) {
+        sum += wc[w * experts + e];
+        wc[w * experts + e] = 0;
+      }
+      base[e] = sum;
+    }
+    __syncthreads();
+    wave_count_ids(wc + wave * experts, ids, begin, routes, experts, wave, WAVES);
+    __syncthreads();
+    for (int e = tid; e < experts; e += kThreads) {
+      int32_t sum = base[e];
+      for (int w = 0; w < WAVES; ++w) {
+        sum += wc[w * experts + e];
+        wc[w * experts + e] = 0;
+      }
+      soff[e] = sum;  // total count; scanned in place below
+    }
   }
   __syncthreads();
   // Exclusive scan of the totals: thread t owns `per` consecutive experts.
@@ -1573,10 +1620,31 @@ hipError_t token_permute_stable(const float* x, const int32_t* ids, const int32_
   return launch_permute_copy(x, route_pos, x_permuted, tokens, top_k, hidden, routes, stream);
 }
 
+// Routes from which route preparation counts the chunks in a launch of its own:
+// every block of the single launch counts all ids, 64 LDS atomics a lane at 65536
+// routes. Single launch / two: post-route chain T = 8192, E = 64, K = N = 64,
+// top_k = 8 (65536 routes) 31.6 / 27.5 us, T = 4096 (32768) 23.0 / 22.1; skewed
+// chain E = 64, K = 256, N = 160, 32768 routes 98 / 91 us, 8192 routes 37.2 / 36.3. Up to
+// 256 chunks, of which every block reads all counts.
+constexpr int kCountedRoutes = 8192;
+constexpr int kCountedChunks = 256;
+
 hipError_t route_prep(const int32_t* ids, int32_t* counts, int32_t* offsets, int32_t* cursors,
                       int32_t* route_pos, int32_t* sorted_route, int routes, int experts,
-                      hipStream_t stream) {
+                      void* scratch, std::size_t scratch_bytes, hipStream_t stream) {
   if (routes <= 0) return hipSuccess;
+  const int parts = static_cast<int>((static_cast<long>(routes) + kBlock - 1) / kBlock);
+  if (routes >= kCountedRoutes && experts <= 256 && scratch != nullptr && parts <= kCountedChunks &&
+      static_cast<std::size_t>(parts) * experts * sizeof(int32_t) <= scratch_bytes) {
+    auto* block_counts = static_cast<int32_t*>(scratch);
+    rr_route_count_kernel<<<parts, kBlock, experts * sizeof(int32_t), stream>>>(ids, block_counts, routes, experts);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    const std::size_t lds = ((2 * static_cast<std::size_t>(kWavesPerBlock) + 2) * experts + 1 + kWavesPerBlock) * sizeof(int32_t);
+    rr_route_prep_kernel<kWavesPerBlock, true><<<parts, kBlock, lds, stream>>>(
+        ids, block_counts, counts, offsets, cursors, route_pos, sorted_route, routes, experts, bits_for(experts), kBlock);
+    return hipGetLastError();
+  }
   const bool wide = experts > 512;
   const int threads = wide ? 512 : 1024;
   int chunk = threads;
@@ -1585,13 +1653,13 @@ hipError_t route_prep(const int32_t* ids, int32_t* counts, int32_t* offsets, int
   const std::size_t lds =
       ((static_cast<std::size_t>(threads / 64) + 2) * experts + 1 + kWavesPerBlock) * sizeof(int32_t);
   if (wide) {
-    rr_route_prep_kernel<8><<<blocks, threads, lds, stream>>>(ids, counts, offsets, cursors, route_pos,
-                                                              sorted_route, routes, experts,
-                                                              bits_for(experts), chunk);
+    rr_route_prep_kernel<8, false><<<blocks, threads, lds, stream>>>(ids, nullptr, counts, offsets, cursors, route_pos,
+                                                                     sorted_route, routes, experts,
+                                                                     bits_for(experts), chunk);
   } else {
-    rr_route_prep_kernel<16><<<blocks, threads, lds, stream>>>(ids, counts, offsets, cursors, route_pos,
-                                                               sorted_route, routes, experts,
-                                                               bits_for(experts), chunk);
+    rr_route_prep_kernel<16, false><<<blocks, threads, lds, stream>>>(ids, nullptr, counts, offsets, cursors, route_pos,
+                                                                      sorted_route, routes, experts,
+                                                                      bits_for(experts), chunk);
   }
   return hipGetLastError();
 }

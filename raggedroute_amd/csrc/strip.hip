@@ -27,6 +27,9 @@
 //   kStripRouterGate dense + every row's top-2 gate (ids, selected-softmax
 //                    weights) in the epilogue + zeroing of the row's y slice;
 //   kStripGrouped    segments from offsets (read on the device);
+//   kStripGather     segments from offsets, rows of x gathered through
+//                    sorted_route, otherwise as kStripChain (chains of more
+//                    routes than that launch holds);
 //   kStripChain      the chain's route preparation and expert GEMM in one
 //                    launch: every workgroup holds all route ids in
 //                    registers (a quarter per wave), counts them into offsets,
@@ -97,7 +100,7 @@ constexpr int kMaxRoutes = 16384; // chain: route ids held in registers
 constexpr int kMaxSegs = 8;       // chain: segments one workgroup's strips may span
 constexpr int kMaxBlocks = 4;     // segments <= 256, 64 per lane column
 
-enum StripMode : int { kStripDense = 0, kStripRouterGate = 1, kStripGrouped = 2, kStripChain = 3 };
+enum StripMode : int { kStripDense = 0, kStripRouterGate = 1, kStripGrouped = 2, kStripChain = 3, kStripGather = 4 };
 
 struct StripParams {
   const float* A;  // dense / grouped: [rows, K]; chain: x [T, K] gathered by token
@@ -379,9 +382,13 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
   constexpr int kThreads = kWaves * 64;
   constexpr int kIdChunks = kMaxRoutes / 256 / kWaves; // route-id chunks per wave
   constexpr int kRowThreads = kThreads / kRows;        // A staging: threads per row
-  constexpr int kALoads = 64 / kRowThreads;            // float4 per thread (K <= 256)
+  // float4 per row (K <= 256; the other K = 128 instances keep the loads of 256:
+  // with half of them the chain T = 512, E = 64, K = N = 128 took 12.7 us, not 12.4)
+  constexpr int kRowQuads = CHUNKS == 4 || (MODE == kStripGather && CHUNKS > 0) ? 4 * CHUNKS : 64;
+  constexpr int kALoads = (kRowQuads + kRowThreads - 1) / kRowThreads;  // ... per thread
   static_assert(BN == 64 || BN == 128, "BN is 64 or 128");
   constexpr bool kSingle = MODE == kStripDense || MODE == kStripRouterGate;  // one segment
+  constexpr bool kRouted = MODE == kStripChain || MODE == kStripGather;      // rows gathered by route
   extern __shared__ __align__(16) float lds[];
 
   const int K = p.K;
@@ -406,13 +413,13 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
   // one ds_read2st64_b32. No cross-wave dependency: no barrier for B.
   constexpr bool kBLds = MODE == kStripRouterGate && CHUNKS == kMaxChunks && WAVES == 4;
   float* s_bl = s_lg + kRows * kLgLd;  // router (kBLds): [waves][16][256]
-  int32_t* s_slot = s_seglist + (MODE == kStripChain ? kWaves * kMaxSegs * 4 : 0);  // chain: [max_strips * 16]
-  float* s_w = reinterpret_cast<float*>(s_slot + (MODE == kStripChain ? p.max_strips * kRows : 0));
+  int32_t* s_slot = s_seglist + (MODE == kStripChain ? kWaves * kMaxSegs * 4 : 0);  // routed: [max_strips * 16]
+  float* s_w = reinterpret_cast<float*>(s_slot + (kRouted ? p.max_strips * kRows : 0));
   // chain: [max_strips * 16] token of each slot's route (-1: none), [max_strips][4] strip info
-  int32_t* s_tok = reinterpret_cast<int32_t*>(s_w + (MODE == kStripChain ? p.max_strips * kRows : 0));
-  int32_t* s_info = s_tok + (MODE == kStripChain ? p.max_strips * kRows : 0);
+  int32_t* s_tok = reinterpret_cast<int32_t*>(s_w + (kRouted ? p.max_strips * kRows : 0));
+  int32_t* s_info = s_tok + (kRouted ? p.max_strips * kRows : 0);
   // chain: [waves][64 nblk] route-id histogram of each wave's chunks
-  int32_t* s_cntw = s_info + (MODE == kStripChain ? p.max_strips * 4 : 0);
+  int32_t* s_cntw = s_info + (kRouted ? p.max_strips * 4 : 0);
 
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = lane_id();
@@ -622,7 +629,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
       }
       tab.cnt[j] = total;
     }
-  } else if constexpr (MODE == kStripGrouped) {
+  } else if constexpr (MODE == kStripGrouped || MODE == kStripGather) {
 #pragma unroll
     for (int j = 0; j < kMaxBlocks; ++j) {
       const int e = 64 * j + lane;
@@ -637,7 +644,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
   } else {
     seg_scan(tab, nblk);
   }
-  if constexpr (MODE == kStripGrouped) {
+  if constexpr (MODE == kStripGrouped || MODE == kStripGather) {
     // rows keep the caller's offsets (the same as the prefix of the counts for
     // well-formed offsets; the caller's base is honoured)
 #pragma unroll
@@ -668,7 +675,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
     range = even_range(total, grid, worker);
   } else {
     range = assign_strips<kWaves == 8 ? 2 : 1>(tab, nblk, E, total, grid, worker,
-                                               MODE == kStripChain ? p.max_strips : INT_MAX);
+                                               kRouted ? p.max_strips : INT_MAX);
   }
   RR_STAMP(6);
   const int s0 = range.s0;
@@ -693,8 +700,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
   };
   StripInfo cur{};
   if (s0 < s1) cur = info(s0);
-  constexpr int kEarlyB = 12;  // chain: k chunks of B issued before the ranks
-  if constexpr (MODE == kStripChain) {
+  constexpr int kEarlyB = 12;  // routed: k chunks of B issued before the ranks
+  if constexpr (kRouted) {
     // k chunks 0..11 of B (48 loads per lane) as soon as the first segment is
     // known: they arrive while the ranks are computed. All of B here would
     // reach the wave's limit of outstanding loads (63) and stall the rank
@@ -704,7 +711,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
     // 0..7, 16.12 for 0..9 and 15.98 for 0..13).
     if (s0 < s1) load_b(cur.e, 0, kEarlyB);
   }
-  if constexpr (MODE == kStripChain) {
+  if constexpr (kRouted) {
     // Every strip's info, once and in parallel (wave w: strips s0 + w,
     // s0 + w + waves, ...), for the strip loop to read back from LDS (read
     // after the barrier that ends the rank passes).
@@ -715,7 +722,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
     }
   }
   auto next_info = [&](int s) -> StripInfo {
-    if constexpr (MODE == kStripChain) {
+    if constexpr (kRouted) {
       const int4 v = *reinterpret_cast<const int4*>(s_info + 4 * (s - s0));
       return StripInfo{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
                        __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w)};
@@ -844,6 +851,18 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
     __syncthreads();
     RR_STAMP(9);
   }
+  if constexpr (MODE == kStripGather) {
+    // The slots of my strips: their rows' routes, tokens and weights.
+    __syncthreads();  // strip info
+    for (int i = tid; i < (s1 - s0) * kRows; i += kThreads) {
+      const int row = s_info[4 * (i / kRows) + 1] + i % kRows;
+      const int32_t route = row < s_info[4 * (i / kRows) + 2] ? p.sorted_route[row] : -1;
+      s_slot[i] = route;
+      s_tok[i] = route >= 0 ? (p.top_k == 2 ? route >> 1 : route / p.top_k) : -1;
+      s_w[i] = route >= 0 && p.combine ? p.route_weights[route] : 0.0F;
+    }
+    __syncthreads();
+  }
 
   // ------------------------------------------------------------ strip loop
   // A staging: thread t loads row t / kRowThreads, float4 columns
@@ -856,9 +875,9 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
     return p.top_k == 2 ? (route >> 1) : route / p.top_k;
   };
   auto a_source = [&](int s, const StripInfo& si) -> int {
-    if constexpr (MODE == kStripChain) {
+    if constexpr (kRouted) {
       (void)si;
-      if (s == s0) {  // before the loop: s_tok is written after the last barrier
+      if (MODE == kStripChain && s == s0) {  // before the loop: s_tok is written after the last barrier
         const int32_t route = s_slot[a_row];
         return route >= 0 ? token_of(route) : -1;
       }
@@ -888,7 +907,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
   const int col0 = 16 * kTiles * wave + li;
   auto epilogue_row = [&](int r, const v4f (&a)[kTiles], const StripInfo& st) {
     const int rl = 4 * g + r;
-    if constexpr (MODE == kStripChain) {
+    if constexpr (kRouted) {
       const int32_t route = ep_route[r];
       if (route >= 0) {
         float* crow = p.C + static_cast<std::size_t>(st.row0 + rl) * N;
@@ -970,6 +989,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
       }
     }
     if (s0 < s1) load_b(cur.e, kEarlyB, kMaxChunks);  // the rest of B
+  } else if constexpr (MODE == kStripGather) {
+    if (s0 < s1) load_b(cur.e, kEarlyB, kMaxChunks);
   } else {
     if (s0 < s1) load_b(cur.e);
   }
@@ -990,7 +1011,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
         *reinterpret_cast<v4f*>(As + a_row * kLd + k) = zero_unless(src >= 0 && k < K, a_regs[u]);
       }
     }
-    if constexpr (MODE == kStripChain) {
+    if constexpr (kRouted) {
       if (src >= 0 && p.x_permuted != nullptr && owns_map(s)) {  // gathered rows -> x_permuted
         float* out = p.x_permuted + static_cast<std::size_t>(si.row0 + a_row) * K;
 #pragma unroll
@@ -999,7 +1020,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
           if (k < K) __builtin_nontemporal_store(a_regs[u], reinterpret_cast<v4f*>(out + k));
         }
       }
-      if (s == s0 && tid < (s1 - s0) * kRows) s_w[tid] = w_pending;
+      if (MODE == kStripChain && s == s0 && tid < (s1 - s0) * kRows) s_w[tid] = w_pending;
     }
     if (s - s0 < 6) RR_STAMP(12 + 4 * (s - s0));
     __syncthreads();
@@ -1120,7 +1141,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void rr_strip_gemm_kernel(StripParam
       for (int t = 0; t < kTiles; ++t) acc_prev[t] = acc[t];
       prev = si;
       prev.rank0 = (s - s0) * kRows;  // slot of the strip's first row (chain)
-      if constexpr (MODE == kStripChain) {
+      if constexpr (kRouted) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           ep_route[r] = s_slot[prev.rank0 + 4 * g + r];
@@ -1236,10 +1257,12 @@ std::size_t strip_lds(int bn, int mode, int K, int segments, int max_strips) {
   if (mode == kStripRouterGate && K == 256 && waves == 4) {
     bytes += static_cast<std::size_t>(waves) * kMaxChunks * 256 * sizeof(float);  // B in LDS
   }
-  if (mode == kStripChain) {
-    bytes += static_cast<std::size_t>(waves) * kMaxSegs * 4 * sizeof(int32_t);  // segment lists
+  if (mode == kStripChain || mode == kStripGather) {
     bytes += 3 * static_cast<std::size_t>(max_strips) * kRows * sizeof(int32_t);  // slots, weights, tokens
     bytes += static_cast<std::size_t>(max_strips) * 4 * sizeof(int32_t);          // strip info
+  }
+  if (mode == kStripChain) {
+    bytes += static_cast<std::size_t>(waves) * kMaxSegs * 4 * sizeof(int32_t);  // segment lists
     bytes += static_cast<std::size_t>(waves) * 64 * ((segments + 63) / 64) * sizeof(int32_t);  // per-wave histograms
   }
   return bytes;
@@ -1256,7 +1279,7 @@ hipError_t launch_strip_4(const StripParams& p, int grid, std::size_t lds, hipSt
 
 template <int BN, int MODE, int CHUNKS>
 hipError_t launch_strip_3(const StripParams& p, int grid, std::size_t lds, hipStream_t stream) {
-  if constexpr (MODE == kStripGrouped || MODE == kStripChain) {
+  if constexpr (MODE == kStripGrouped || MODE == kStripChain || MODE == kStripGather) {
     if (p.segments > 64) return launch_strip_4<BN, MODE, CHUNKS, kMaxBlocks>(p, grid, lds, stream);
   }
   return launch_strip_4<BN, MODE, CHUNKS, 1>(p, grid, lds, stream);
@@ -1270,7 +1293,11 @@ hipError_t launch_strip_2(const StripParams& p, int grid, std::size_t lds, hipSt
   if (p.K == 256) return launch_strip_3<BN, MODE, 16>(p, grid, lds, stream);
   if (p.K == 128) return launch_strip_3<BN, MODE, 8>(p, grid, lds, stream);
   if (p.K == 64) return launch_strip_3<BN, MODE, 4>(p, grid, lds, stream);
-  return launch_strip_3<BN, MODE, 0>(p, grid, lds, stream);
+  if constexpr (MODE == kStripGather) {
+    return hipErrorInvalidValue;  // strip_gather_ok
+  } else {
+    return launch_strip_3<BN, MODE, 0>(p, grid, lds, stream);
+  }
 }
 
 template <int MODE>
@@ -1328,6 +1355,31 @@ bool strip_chain_ok(int tokens, int top_k, int experts, int k, int n, const void
          strip_lds(bn_for(n), kStripChain, k, experts, max_strips) <= kLdsLimit;
 }
 
+// The gathered form takes K = 64, 128 and 256 (the instances; the general one
+// loses to the tiled kernel: T = 2895, E = 117, K = 224, N = 128, top_k = 8, skewed,
+// 56 against 45 us) with two workgroups a CU: one waits for its gathered rows
+// while the other multiplies. T = 8192, E = 64, K = N = 64, top_k = 8, one / two / four
+// a CU: post-route chain 36.4 / 31.6 / 31.4 us (tiled kernel 40.2); K = N = 128 50.5 /
+// 47.4 / 51.2 (51.8); K = 256, N = 128 67 / 64 / 70 (71); chain T = 16384, E = 64,
+// K = 256, N = 128 52 / 51 / 58 (78).
+int gather_grid(long strips) {
+  const long cap = 2L * cu_count();
+  long grid = strips < cap ? strips : cap;
+  if (grid >= kXcds) grid = grid / kXcds * kXcds;
+  return static_cast<int>(grid < 1 ? 1 : grid);
+}
+
+bool strip_gather_ok(long routes, int top_k, int experts, int k, int n, const void* x, const void* w,
+                     const void* x_permuted) {
+  if (!strip_shape_ok(k, n, x, w) || !aligned16(x_permuted)) return false;
+  if (k != 64 && k != 128 && k != 256) return false;
+  if (!strip_segments_ok(experts) || routes <= 0 || top_k < 1 || routes > INT_MAX - kRows) return false;
+  const long bound = (routes + kRows - 1) / kRows + experts;
+  const int grid = gather_grid(bound);
+  const int max_strips = static_cast<int>((bound + grid - 1) / grid) + 1;
+  return strip_lds(bn_for(n), kStripGather, k, experts, max_strips) <= kLdsLimit / 2;
+}
+
 hipError_t strip_dense(const float* a, const float* b, float* c, int m, int n, int k,
                        hipStream_t stream) {
   if (m <= 0) return hipSuccess;
@@ -1380,6 +1432,27 @@ hipError_t strip_chain(const float* x, const float* expert_weights, const int32_
   p.y = y;
   if (p.max_strips > kMaxSegs + 1) return hipErrorInvalidValue;  // strip_chain_ok excludes it
   return launch_strip<kStripChain>(p, grid, stream);
+}
+
+hipError_t strip_gather(const float* x, const float* expert_weights, const int32_t* offsets,
+                        const int32_t* sorted_route, const float* route_weights, float* x_permuted,
+                        float* y_permuted, float* y, int tokens, int top_k, int experts, int hidden,
+                        int output, hipStream_t stream) {
+  if (tokens <= 0) return hipSuccess;
+  if (y != nullptr && top_k != 2) return hipErrorInvalidValue;  // combine is top-2 only
+  const long routes = static_cast<long>(tokens) * top_k;
+  StripParams p = base(x, expert_weights, y_permuted, 0, hidden, output, experts);
+  const long bound = (routes + kRows - 1) / kRows + experts;
+  const int grid = gather_grid(bound);
+  p.max_strips = static_cast<int>((bound + grid - 1) / grid) + 1;
+  p.offsets = offsets;
+  p.top_k = top_k;
+  p.combine = y != nullptr ? 1 : 0;
+  p.route_weights = route_weights;
+  p.sorted_route = const_cast<int32_t*>(sorted_route);  // (read only in this mode)
+  p.x_permuted = x_permuted;
+  p.y = y;
+  return launch_strip<kStripGather>(p, grid, stream);
 }
 
 #ifdef RR_PHASE_STAMPS

@@ -1,5 +1,5 @@
 """histogram and histogram_exclusive_scan around the sizes where the kernel
-changes (24576 routes below 32 experts, 49152 from there), with ids that crowd
+changes (24576 routes below 32 experts, 49152 below 128, 65536 from there), with ids that crowd
 one expert (counted with ballots), ragged tails of the id quads, ids off 16
 bytes and ids outside [0, E): counts and offsets are whole numbers and exact."""
 from __future__ import annotations
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("experts,routes", [
     (8, 1), (8, 3), (31, 24575), (31, 24576), (31, 24577), (32, 24577), (64, 4097), (256, 16387),
-    (1000, 8191), (32, 49151), (64, 49152), (64, 49153), (1024, 49152), (2, 20000),
+    (1000, 8191), (32, 49151), (64, 49152), (64, 49153), (1024, 49152), (127, 49153), (128, 65536), (128, 65537), (2, 20000),
 ])
 @pytest.mark.parametrize("kind", ["uniform", "hot", "one", "two", "invalid"])
 def test_counts_and_offsets(ctx, device, experts, routes, kind):
