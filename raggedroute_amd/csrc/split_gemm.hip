@@ -45,8 +45,8 @@
 // 6.1 ms (315 TFLOP/s of FP32 products, 945 of FP16 ones; a library FP16 product
 // of random 8192 x 8192 matrices reaches 1300 on this card), and 4.5 ms with
 // operands of ones, which draw less power. Elsewhere by each tile's serial
-// parts: T = 16384, E = 128, K = 2048, N = 768 chain 1031 / 641 us, T = 2048,
-// E = 64, K = 1024, N = 512 chain 132 / 82 us.
+// parts and the combine: T = 16384, E = 128, K = 2048, N = 768 chain, expert GEMM
+// 927 / 510 us.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -623,7 +623,14 @@ __global__ __launch_bounds__(64 * W, 2) void rr_split_gemm_kernel(GemmParams prm
   const int worker = tile_worker(static_cast<int>(blockIdx.x), grid);
 
 #pragma unroll 1
-  for (long t = worker; t < total; t += grid) {
+  for (long dealt = 0; dealt < total; dealt += grid) {
+    // The last, partial round goes to the workgroups in dispatch order, over all
+    // XCDs and one a CU first, instead of filling the first XCDs (staged T = 3001,
+    // E = 9, K = 1023, N = 1535 153.6 -> 145.4 us; chain T = 16384, E = 64, K = N = 512
+    // 170 -> 161).
+    const int mine = total - dealt >= grid ? worker : static_cast<int>(blockIdx.x);
+    const long t = dealt + mine;
+    if (t >= total) break;
     const bool is_short = t >= total_full;
     int rt, ct;
     decode_tile(static_cast<int>(is_short ? t - total_full : t), is_short ? short_rows : full_rows,
