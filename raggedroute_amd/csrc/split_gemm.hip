@@ -3,28 +3,33 @@
 // The FP32 matrix instructions run at 157 TFLOP/s, the FP16 ones at 2.5 PFLOP/s
 // with FP32 accumulation. Every operand x is scaled by a power of two of its
 // own row (A) or column (B), xs = x * s, and split into two FP16 numbers
-//     h = fp16(xs),   l = fp16(xs - h),
+//     h = fp16(xs),   l = fp16(xs - h),   l stored times 2^11,
 // both rounded to nearest; xs - h is exact in FP32 and at most 2^-11 of xs, so
 // h + l carries x to within 2^-23 of itself (half of all values exactly). A
 // product is
 //     xs * ys = hx hy + (lx hy + hx ly) + lx ly;
 // the first three terms are computed (three MFMAs), the last is at most 2^-22 of
 // the product (2^-25 in the mean) and left out. hx hy is summed in one FP32
-// accumulator and the two small terms in another, which are added once at the
-// end: the large sum is rounded once per 16 k instead of once per 4 k as on the
-// FP32 instructions. Against 64-bit sums the result is closer than the FP32
-// instructions' at every K (2-norm error over N(0,1) operands, this / FP32 MFMA:
+// accumulator and the two small terms in another, which is added once, times
+// 2^-11, at the end: the large sum is rounded once per 16 k instead of once per
+// 4 k as on the FP32 instructions. Against 64-bit sums the result is closer than
+// the FP32 instructions' at every K (2-norm error over N(0,1) operands, this / FP32 MFMA:
 // K = 64 0.98 / 1.43e-7, K = 256 1.31 / 2.87e-7, K = 1024 2.2 / 5.8e-7, K = 4096
 // 4.1 / 11.4e-7; likewise for non-negative and half-zero operands).
 //
 // Range. The scale puts the largest of a row's (column's) first nonzero slice
-// of 32 k near 2^4, so later values may be 2^12 times larger before fp16(xs)
-// overflows, and values 2^-5 of it and up split without loss; below that the
-// split's error stops shrinking at 2^-25, which is 2^-29 of the sampled
-// maximum. Values this cannot carry are never computed this way: an operand
-// that is infinite, NaN or past the FP16 range makes every output it meets
-// non-finite, and sampled maxima below 2^-100 are seen when the scale is taken.
-// A tile that shows either is computed again on the FP32 instructions before
+// of 32 k near 2^6, so later values may be 2^9 times larger before fp16(xs)
+// overflows. Stored times 2^11, l keeps its 11 bits down to values 2^-20 of the
+// sampled maximum; below that the split's error stays at 2^-36, 2^-42 of that
+// maximum. (Without the factor, and the maximum near 2^4, that was 2^-29: a row
+// whose first slice was 2^20 times the rest and met zero weights came out 1e-3
+// of sum |x y| off, now 1.6e-7, on the FP32 instructions 2.6e-7. The factor is
+// a multiplication per element: T = 16384 rows in eight experts, K = 4096, N =
+// 14336 5.78 -> 5.86 ms, 128 experts of 256 rows, K = 2048, N = 768 377 -> 379 us,
+// 64 of 64, K = 1024, N = 512 33.7 -> 36.0 us.)
+// Values past all this are never computed this way: an operand that is infinite,
+// NaN or past the FP16 range makes every output it meets non-finite, and
+// sampled maxima below 2^-100 are seen when the scale is taken. A tile that shows either is computed again on the FP32 instructions before
 // anything is stored (with the FP32 rules for infinities, NaN and overflow).
 //
 // Work split: output tiles of 128 columns and 128 or 256 rows on four or eight
@@ -32,7 +37,7 @@
 // both operands is loaded into registers one slice ahead (16-byte A quads, 8-byte
 // B pairs; rows may start at any 4-byte boundary), split there, and written to
 // LDS as FP16 planes in MFMA operand order (k contiguous per row of A and per
-// column of B), two stages; the split costs three full-rate instructions per
+// column of B), two stages; the split costs four full-rate instructions per
 // element. Four waves: two workgroups share a CU and
 // one's MFMAs run under the other's staging. Eight waves: the two halves of the
 // workgroup run a phase apart, so that one has the matrix pipe while the other
@@ -68,6 +73,7 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int kBN = 128, kBK = 32;
 constexpr int kPlaneB = kBN * kBK;          // halfs of one plane of B (8 KiB)
+constexpr float kLowScale = 2048.0F;        // l is stored times 2^11
 constexpr int kBufferFlags = 0x00027000;    // raw 32-bit buffer
 constexpr int kRefLd = kBK + 1;             // FP32 recomputation: padded LDS row (floats)
 
@@ -102,22 +108,22 @@ struct Layout {
 // 16 rows read together land in 16 distinct 16-byte bank groups.
 __device__ __forceinline__ int plane_swizzle(int r) { return (r >> 2) & 3; }
 
-// x * s = h + l (see the file comment): six full-rate instructions for two
+// x * s = h + l (see the file comment): eight full-rate instructions for two
 // values. (Four v_fma_mixlo / mixhi_f16 would do, but they issue at half rate:
 // 9.7 against 4.7 cycles.)
 __device__ __forceinline__ void split2(float x0, float x1, float s, h2& h, h2& l) {
   typedef float f2 __attribute__((ext_vector_type(2)));
   h = __builtin_convertvector(f2{x0 * s, x1 * s}, h2);
   asm("" : "+v"(h));  // both halves in their register: the next two read them there
-  l = __builtin_convertvector(f2{__builtin_fmaf(x0, s, -static_cast<float>(h[0])),
-                                 __builtin_fmaf(x1, s, -static_cast<float>(h[1]))}, h2);
+  l = __builtin_convertvector(f2{__builtin_fmaf(x0, s, -static_cast<float>(h[0])) * kLowScale,
+                                 __builtin_fmaf(x1, s, -static_cast<float>(h[1])) * kLowScale}, h2);
 }
 
 __device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFU; }
 __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
 
 // The scale of a row or column whose sampled maximum has these bits: s = 2^t
-// with t = 4 - floor(log2(max)); 1 for an all-zero sample.
+// with t = 6 - floor(log2(max)); 1 for an all-zero sample.
 struct Scale {
   float s;
   int t;
@@ -127,9 +133,9 @@ __device__ __forceinline__ Scale scale_of(uint32_t bits) {
   Scale sc;
   int e = static_cast<int>(bits >> 23);
   sc.bad = bits != 0 && (e == 255 || e < 27);
-  e = bits == 0 ? 131 : (e < 27 ? 27 : e);
-  sc.t = 131 - e;
-  sc.s = __uint_as_float(static_cast<uint32_t>(258 - e) << 23);
+  e = bits == 0 ? 133 : (e < 27 ? 27 : e);
+  sc.t = 133 - e;
+  sc.s = __uint_as_float(static_cast<uint32_t>(260 - e) << 23);
   return sc;
 }
 
@@ -542,7 +548,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
-        acc[i][j][r] += low[i][j][r];
+        acc[i][j][r] = __builtin_fmaf(low[i][j][r], 1.0F / kLowScale, acc[i][j][r]);
         overflow = overflow || (rl < rows && col + 32 * j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
       }
     }

@@ -1,8 +1,8 @@
 """The grouped GEMM on the FP16 matrix cores, forced with RR_GEMM_STAGING=split
 (by default it takes large problems): row counts at the edges of its 32-row blocks and tiles, K and N at the edges of
 its slices, pairs and column tiles, offset pointers, and values that its scales
-cannot carry (infinities, NaN, overflow, subnormals, late outliers, leading
-zeros), which must come out as the FP32 instructions give them
+cannot carry (infinities, NaN, overflow, subnormals, late and early outliers,
+leading zeros), which must come out as the FP32 instructions give them
 (RR_GEMM_STAGING=fp32).
 
 Tolerance: check_grouped's accumulation-aware bound 4 gamma_K sum |a b| + 1e-7
@@ -79,6 +79,14 @@ def special_inputs(case, rng):
         w[2, 7, 9] = -np.inf
     elif case == "late outlier":      # 2^20 times the sampled slice
         x[:, 200] *= 1e6
+    elif case == "early outlier":     # the sampled slice 2^20 times the rest, and weights that do not meet it
+        x[:, :32] *= 2.0 ** 20
+        w[:, :32] = 0
+    elif case == "early outliers of both":  # 2^10, in separate halves of the sampled slice
+        x[:, :16] *= 2.0 ** 10
+        w[:, :16] = 0
+        w[:, 16:32] *= 2.0 ** 10
+        x[:, 16:32] = 0
     elif case == "zeros":             # zero rows, zero columns, leading zeros of both
         x[7] = 0
         x[:, :64] = 0
@@ -104,7 +112,8 @@ def special_inputs(case, rng):
     return counts, x, w
 
 
-@pytest.mark.parametrize("case", ["infinity and NaN", "late outlier", "zeros", "all zero", "tiny", "subnormal",
+@pytest.mark.parametrize("case", ["infinity and NaN", "late outlier", "early outlier", "early outliers of both",
+                                  "zeros", "all zero", "tiny", "subnormal",
                                   "huge", "overflow", "row scales"])
 def test_values_past_the_fp16_range(ctx, device, staging, case):
     counts, x, w = special_inputs(case, np.random.default_rng(11))
