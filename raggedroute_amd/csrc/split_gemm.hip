@@ -19,18 +19,28 @@
 //
 // Range. The scale puts the largest of a row's (column's) first nonzero slice
 // of 32 k near 2^6, so later values may be 2^9 times larger before fp16(xs)
-// overflows. Stored times 2^11, l keeps its 11 bits down to values 2^-20 of the
-// sampled maximum; below that the split's error stays at 2^-36, 2^-42 of that
-// maximum. (Without the factor, and the maximum near 2^4, that was 2^-29: a row
-// whose first slice was 2^20 times the rest and met zero weights came out 1e-3
-// of sum |x y| off, now 1.6e-7, on the FP32 instructions 2.6e-7. The factor is
-// a multiplication per element: T = 16384 rows in eight experts, K = 4096, N =
-// 14336 5.78 -> 5.86 ms, 128 experts of 256 rows, K = 2048, N = 768 377 -> 379 us,
-// 64 of 64, K = 1024, N = 512 33.7 -> 36.0 us.)
-// Values past all this are never computed this way: an operand that is infinite,
-// NaN or past the FP16 range makes every output it meets non-finite, and
-// sampled maxima below 2^-100 are seen when the scale is taken. A tile that shows either is computed again on the FP32 instructions before
-// anything is stored (with the FP32 rules for infinities, NaN and overflow).
+// overflows. l, stored times 2^11, keeps its 11 bits down to |xs| = 2^-14 (2^-20
+// of the sampled maximum); below, the split's error stays at 2^-36, so that values
+// much smaller than the sample lose their bits: with one feature 2^p times the
+// rest and its weights zero, K = 320, the 2-norm error was 1.8e-6 at p = 24, 1.1e-4
+// at 2^30, 0.1 at 2^40 (FP32 instructions 3.2e-7). Nothing of that kind is
+// computed this way. A row or column is marked when
+//  - its sample is below 2^-100, or 2^41 and more (or not finite);
+//  - four of its values in slice 0 are nonzero and scale to less than 2^-14;
+//  - of four consecutive k (4 i .. 4 i + 3) past slice 0 the largest does.
+// So of any four k of an unmarked row past slice 0 the split's error is at most
+// 2^-22 of the largest, and values whose xs is below 2^-14 are few among larger
+// ones. (A scaled value under 2^-149 counts as zero: |x| < 2^-115 in a row whose
+// sample is 2^40.) An operand past the FP16 range makes every output it meets
+// non-finite. A tile that holds a marked row or column or shows a non-finite sum
+// is computed again on the FP32 instructions before anything is stored (with the
+// FP32 rules for infinities, NaN and overflow). N(0,1) rows are marked once in
+// 10^9 (four values of 2^-20 side by side); rows of which half the values are zero,
+// five in 10^4 at K = 4096. The marks take 24 of 132 vector instructions of a slice of
+// the 256-row loop: T = 8192, E = 8, K = 4096, N = 14336 call 6.80 -> 7.21 ms, T = 3001,
+// E = 9, K = 1023, N = 1535 150 -> 156 us, chain T = 16384, E = 128, K = 2048, N = 768
+// 607 -> 626 us, T = 2048, E = 64, K = 1024, N = 512 70.2 -> 72.1 us. (Pairs of k, and
+// groups over two slices or two lanes, were slower: 7.1 - 8.0 ms in the first.)
 //
 // Work split: output tiles of 128 columns and 128 or 256 rows on four or eight
 // waves (split_grouped picks), tiles dealt as in gemm.hip. A slice of 32 k of
@@ -74,6 +84,9 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 constexpr int kBN = 128, kBK = 32;
 constexpr int kPlaneB = kBN * kBK;          // halfs of one plane of B (8 KiB)
 constexpr float kLowScale = 2048.0F;        // l is stored times 2^11
+constexpr float kLeast = 0x1p-14F;          // scaled values from here on keep all bits of l
+constexpr int kFewSmall = 4;                // too small values of slice 0 that send a row or column to FP32
+constexpr int kMarked = 1 << 16;            // scale exponent of a row or column that is not computed in FP16
 constexpr int kBufferFlags = 0x00027000;    // raw 32-bit buffer
 constexpr int kRefLd = kBK + 1;             // FP32 recomputation: padded LDS row (floats)
 
@@ -111,12 +124,24 @@ __device__ __forceinline__ int plane_swizzle(int r) { return (r >> 2) & 3; }
 // x * s = h + l (see the file comment): eight full-rate instructions for two
 // values. (Four v_fma_mixlo / mixhi_f16 would do, but they issue at half rate:
 // 9.7 against 4.7 cycles.)
-__device__ __forceinline__ void split2(float x0, float x1, float s, h2& h, h2& l) {
+// x0 and x1 are left scaled.
+__device__ __forceinline__ void split2(float& x0, float& x1, float s, h2& h, h2& l) {
   typedef float f2 __attribute__((ext_vector_type(2)));
-  h = __builtin_convertvector(f2{x0 * s, x1 * s}, h2);
+  const float s0 = x0 * s, s1 = x1 * s;
+  h = __builtin_convertvector(f2{s0, s1}, h2);
   asm("" : "+v"(h));  // both halves in their register: the next two read them there
   l = __builtin_convertvector(f2{__builtin_fmaf(x0, s, -static_cast<float>(h[0])) * kLowScale,
                                  __builtin_fmaf(x1, s, -static_cast<float>(h[1])) * kLowScale}, h2);
+  x0 = s0;
+  x1 = s1;
+}
+
+// The largest of four magnitudes (without the canonicalizing copies of fmaxf).
+__device__ __forceinline__ float most_of(float a, float b, float c, float d) {
+  float m;
+  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+  asm("v_max_f32 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(d));
+  return m;
 }
 
 __device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFU; }
@@ -127,17 +152,20 @@ __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b 
 struct Scale {
   float s;
   int t;
-  bool bad;  // not computed in FP16: not finite, or below 2^-100
+  bool bad;  // not computed in FP16: below 2^-100, or 2^41 and more (or not finite)
 };
 __device__ __forceinline__ Scale scale_of(uint32_t bits) {
   Scale sc;
   int e = static_cast<int>(bits >> 23);
-  sc.bad = bits != 0 && (e == 255 || e < 27);
+  sc.bad = bits != 0 && (e > 167 || e < 27);
   e = bits == 0 ? 133 : (e < 27 ? 27 : e);
   sc.t = 133 - e;
   sc.s = __uint_as_float(static_cast<uint32_t>(260 - e) << 23);
   return sc;
 }
+
+// Whether a scaled magnitude (its bits) is too small for the split: nonzero and below kLeast.
+__device__ __forceinline__ bool too_small(uint32_t m) { return m - 1U < __float_as_uint(kLeast) - 1U; }
 
 // What a tile needs from the kernel (all workgroup-uniform).
 struct Tile {
@@ -147,9 +175,10 @@ struct Tile {
 };
 struct Lds {
   _Float16* stages;  // [2][kStage]
-  int32_t* ta;       // [kBM] scale exponents of the rows
+  int32_t* ta;       // [kBM] scale exponents of the rows (kMarked: FP32)
   int32_t* tb;       // [128] ... of the plane rows of B
   uint2* cmax;       // [W][64] column samples
+  int32_t* few;      // [128] values of slice 0 too small for their column's scale
   int32_t* src;      // [kBM] chain: token row of X per tile row (-1: none)
   float* w;          // [kBM] chain: route weight per tile row
 };
@@ -254,6 +283,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   // ---- scales: the first slice with a nonzero value, per row and column ----
   // (almost always slice 0; a tile with an all-zero row or column reads on)
   load_any(0);
+  if (tid < kBN) sh.few[tid] = 0;
   uint32_t ma[P] = {};
   uint32_t mb0 = 0, mb1 = 0;
 #pragma unroll 1
@@ -293,24 +323,28 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     }
     load_any(++kt);
   }
-  bool bad = false;
-  float sa[P], sb0, sb1;
+  float sa[P], sb[2];
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const Scale sc = scale_of(ma[p]);
     sa[p] = sc.s;
-    bad = bad || (sc.bad && PR * p + ar < rows);
-    if (ac == 0) sh.ta[PR * p + ar] = sc.t;
+    uint32_t few = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) few += too_small(abs_bits(ra[p][q] * sc.s)) ? 1U : 0U;
+    few += rr::dev::dpp_move<0xB1>(few);
+    few += rr::dev::dpp_move<0x4E>(few);
+    few += rr::dev::dpp_move<0x141>(few);
+    if (ac == 0) sh.ta[PR * p + ar] = sc.bad || few >= kFewSmall ? kMarked : sc.t;
   }
-  {
-    const Scale x = scale_of(mb0), y = scale_of(mb1);
-    sb0 = x.s;
-    sb1 = y.s;
-    bad = bad || (x.bad && n < N) || (y.bad && n + 1 < N);
-    if (wave == 0) {
-      sh.tb[2 * pair] = x.t;
-      sh.tb[2 * pair + 1] = y.t;
-    }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const Scale sc = scale_of(j == 0 ? mb0 : mb1);
+    sb[j] = sc.s;
+    if (wave == 0) sh.tb[2 * pair + j] = sc.bad ? kMarked : sc.t;
+    int32_t few = 0;
+#pragma unroll
+    for (int q = 0; q < KP; ++q) few += too_small(abs_bits(rb[q][j] * sc.s)) ? 1 : 0;
+    if (few != 0) atomicAdd(sh.few + 2 * pair + j, few);
   }
 
   // Gathered rows go to x_permuted spread over the column tiles: tile ct
@@ -337,13 +371,18 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       (void)kt;
     }
   };
-  // the slice in registers, split, into an LDS stage
-  auto put = [&](_Float16* __restrict__ st) {
+  // The slice in registers, split, into an LDS stage; slices past the first also
+  // note the rows and columns with four k too small for the scale.
+  uint64_t small_a[P] = {}, small_b[2] = {};  // lane masks
+  auto put = [&](_Float16* __restrict__ st, int kt) {
+    float most_a[P], most_b[2][KP / 4];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       h2 h0, l0, h1, l1;
-      split2(ra[p][0], ra[p][1], sa[p], h0, l0);
-      split2(ra[p][2], ra[p][3], sa[p], h1, l1);
+      float x0 = ra[p][0], x1 = ra[p][1], x2 = ra[p][2], x3 = ra[p][3];
+      split2(x0, x1, sa[p], h0, l0);
+      split2(x2, x3, sa[p], h1, l1);
+      most_a[p] = most_of(x0, x1, x2, x3);
       *reinterpret_cast<h4*>(st + p * PR * kBK + a_put) = h4{h0[0], h0[1], h1[0], h1[1]};
       *reinterpret_cast<h4*>(st + S::kPlaneA + p * PR * kBK + a_put) = h4{l0[0], l0[1], l1[0], l1[1]};
     }
@@ -352,16 +391,28 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       typedef _Float16 hk __attribute__((ext_vector_type(KP)));
       hk h, l;
 #pragma unroll
-      for (int q = 0; q < KP / 2; ++q) {
-        h2 hh, ll;
-        split2(rb[2 * q][j], rb[2 * q + 1][j], j == 0 ? sb0 : sb1, hh, ll);
-        h[2 * q] = hh[0];
-        h[2 * q + 1] = hh[1];
-        l[2 * q] = ll[0];
-        l[2 * q + 1] = ll[1];
+      for (int q = 0; q < KP / 4; ++q) {
+        h2 h0, l0, h1, l1;
+        float x0 = rb[4 * q][j], x1 = rb[4 * q + 1][j], x2 = rb[4 * q + 2][j], x3 = rb[4 * q + 3][j];
+        split2(x0, x1, sb[j], h0, l0);
+        split2(x2, x3, sb[j], h1, l1);
+        most_b[j][q] = most_of(x0, x1, x2, x3);
+        h[4 * q] = h0[0], h[4 * q + 1] = h0[1], h[4 * q + 2] = h1[0], h[4 * q + 3] = h1[1];
+        l[4 * q] = l0[0], l[4 * q + 1] = l0[1], l[4 * q + 2] = l1[0], l[4 * q + 3] = l1[1];
       }
       *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + b_put + j * kBK) = h;
       *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + kPlaneB + b_put + j * kBK) = l;
+    }
+    if (kt > 0) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        small_a[p] |= __ballot(too_small(__float_as_uint(most_a[p])));
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int q = 0; q < KP / 4; ++q) small_b[j] |= __ballot(too_small(__float_as_uint(most_b[j][q])));
+      }
     }
   };
 
@@ -413,7 +464,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.ah[i], o.bl[j], low[i][j], 0, 0, 0);
       }
     };
-    put(sh.stages);
+    put(sh.stages, 0);
     store_xp(0);
     if (nk > 1) load_any(1);
     __syncthreads();
@@ -446,7 +497,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll 1
       for (; kt + 3 < nk; ++kt) {
         phases(kt, [&]() {
-          put(sh.stages + (~kt & 1) * S::kStage);
+          put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
           store_xp(kt + 1);
           load(kt + 2);
         });
@@ -455,7 +506,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       for (; kt < nk; ++kt) {
         phases(kt, [&]() {
           if (kt + 1 < nk) {
-            put(sh.stages + (~kt & 1) * S::kStage);
+            put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
             store_xp(kt + 1);
           }
           if (kt + 2 < nk) load_any(kt + 2);
@@ -474,7 +525,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       int kt = 0;
 #pragma unroll 1
       for (; kt + 3 < nk; ++kt) {
-        put(sh.stages + (~kt & 1) * S::kStage);
+        put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
         store_xp(kt + 1);
         load(kt + 2);
         __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to the slice's end)
@@ -483,7 +534,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll 1
       for (; kt < nk; ++kt) {
         if (kt + 1 < nk) {
-          put(sh.stages + (~kt & 1) * S::kStage);
+          put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
           store_xp(kt + 1);
         }
         if (kt + 2 < nk) load_any(kt + 2);
@@ -540,7 +591,18 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       }
     }
   };
-  bool overflow = bad;
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    if ((small_a[p] >> lane & 1) != 0) sh.ta[PR * p + ar] = kMarked;
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if ((small_b[j] >> lane & 1) != 0) sh.tb[2 * pair + j] = kMarked;
+  }
+  __syncthreads();
+  // (what lies outside the tile is not stored)
+  bool overflow = tid < rows && sh.ta[tid] == kMarked;
+  if (tid < kBN && tl.n0 + tid < N) overflow = overflow || sh.tb[tid] == kMarked || sh.few[tid] >= kFewSmall;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -607,7 +669,8 @@ __global__ __launch_bounds__(64 * W, 2) void rr_split_gemm_kernel(GemmParams prm
   sh.ta = reinterpret_cast<int32_t*>(smem + 2 * S::kStage);
   sh.tb = sh.ta + kBM;
   sh.cmax = reinterpret_cast<uint2*>(sh.tb + kBN);
-  sh.src = reinterpret_cast<int32_t*>(sh.cmax + W * 64);
+  sh.few = reinterpret_cast<int32_t*>(sh.cmax + W * 64);
+  sh.src = sh.few + kBN;
   sh.w = reinterpret_cast<float*>(sh.src + kBM);
   int32_t* s_off = reinterpret_cast<int32_t*>(sh.w + kBM);  // [E + 1]
   int32_t* s_pre = s_off + prm.experts + 1;                 // [E + 1] full row tiles before expert e
@@ -697,7 +760,7 @@ hipError_t launch(const GemmParams& prm, long rows_per_expert, int cus, hipStrea
   if (grid >= kXcds) grid = grid / kXcds * kXcds;
   if (grid < 1) grid = 1;
   const std::size_t lds = 2 * S::kStage * sizeof(_Float16) + (S::kBM + kBN) * sizeof(int32_t) +
-                          W * 64 * sizeof(uint2) + 2 * S::kBM * sizeof(int32_t) +
+                          W * 64 * sizeof(uint2) + kBN * sizeof(int32_t) + 2 * S::kBM * sizeof(int32_t) +
                           3 * static_cast<std::size_t>(prm.experts + 1) * sizeof(int32_t);
   rr_split_gemm_kernel<W, BM, CHAIN><<<dim3(static_cast<unsigned>(grid)), S::kThreads, lds, stream>>>(prm);
   return hipGetLastError();

@@ -139,6 +139,42 @@ def test_values_past_the_fp16_range(ctx, device, staging, case):
             assert (err <= 4 * gamma * mag + 2 * x.shape[1] * 2.0 ** -149)[fin].all(), (case, e)
 
 
+def two_norm_error(y, x, w, offsets):
+    num = den = 0.0
+    for e in range(len(w)):
+        rows = slice(int(offsets[e]), int(offsets[e + 1]))
+        exact = x[rows].astype(np.float64) @ w[e].astype(np.float64)
+        num += ((y[rows] - exact) ** 2).sum()
+        den += (exact ** 2).sum()
+    return np.sqrt(num / den)
+
+
+@pytest.mark.parametrize("side", ["row", "column"])
+@pytest.mark.parametrize("form", ["zero", "compensating", "alternating", "three of four", "first slices", "last slice"])
+@pytest.mark.parametrize("p", [22, 24, 27, 30, 36, 45, 60])
+def test_values_far_below_the_sample(ctx, device, staging, side, form, p):
+    """Features 2^p times the rest, met by zeros or by values 2^-p the rest's: the
+    results rest on the small ones alone, or on both. Either way they must be as
+    close to the exact ones as the FP32 instructions' (whose error differs by the
+    order of the sums only: a few percent over these 140000 outputs; 1.25 times
+    is allowed)."""
+    rng = np.random.default_rng(p)
+    counts, k, n = [200, 40, 90, 20], 320, 400
+    big = {"zero": slice(0, 1), "compensating": slice(0, 1), "alternating": slice(0, None, 2),
+           "three of four": np.arange(k) % 4 != 1, "first slices": slice(0, 96), "last slice": slice(0, 288)}[form]
+    x = rng.standard_normal((sum(counts), k)).astype(np.float32)
+    w = (rng.standard_normal((4, k, n)) / np.sqrt(k)).astype(np.float32)
+    a, b = (x.T, w.transpose(1, 0, 2)) if side == "row" else (w.transpose(1, 0, 2), x.T)  # views, k first
+    a[big] *= np.float32(2.0 ** p)
+    b[big] *= np.float32(2.0 ** -p if form == "compensating" else 0.0)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    err = {}
+    for path in ("fp32", "split"):
+        staging(path)
+        err[path] = two_norm_error(run_grouped(ctx, device, x, w, offsets, NATIVE), x, w, offsets)
+    assert err["split"] <= 1.25 * err["fp32"], err
+
+
 @pytest.mark.parametrize("tokens,experts,hidden,output", [
     (700, 8, 256, 272), (333, 5, 289, 301), (64, 16, 512, 384), (1100, 7, 260, 640),
 ])
