@@ -799,13 +799,20 @@ bool direct_any_disabled() {
 }
 
 // Whether a grouped GEMM runs on the FP16 matrix cores (split_gemm.hip).
-// RR_GEMM_STAGING=fp32 keeps it on the FP32 instructions and RR_GEMM_STAGING=
-// split takes the split kernel wherever it can run, for tests and A/B runs.
-bool split_chosen(const GemmParams& prm, long rows, long cus) {
+// RR_GEMM_STAGING=fp32 keeps it on the FP32 instructions; split takes the split
+// kernel wherever it can run, split4, split8 and split256 with one of its
+// workgroup shapes, for tests and A/B runs.
+bool split_chosen(const GemmParams& prm, long rows, long cus, SplitShape* shape) {
+  *shape = SplitShape::kBySize;
   const char* v = std::getenv("RR_GEMM_STAGING");
   if (v != nullptr && std::strcmp(v, "fp32") == 0) return false;
   if (!split_gemm_fits(prm)) return false;
-  if (v != nullptr && std::strcmp(v, "split") == 0) return true;
+  if (v != nullptr && std::strncmp(v, "split", 5) == 0) {
+    if (std::strcmp(v, "split4") == 0) *shape = SplitShape::kFourWaves;
+    if (std::strcmp(v, "split8") == 0) *shape = SplitShape::kEightWaves;
+    if (std::strcmp(v, "split256") == 0) *shape = SplitShape::kRows256;
+    return true;
+  }
   return split_gemm_ok(prm.K, prm.N, prm.experts, rows, static_cast<int>(cus));
 }
 
@@ -909,8 +916,9 @@ hipError_t gemm_dispatch(const GemmParams& prm, long rows_per_expert, long total
     default: break;
   }
   if constexpr (MODE != kDense) {
-    if (split_chosen(prm, total_rows_estimate, cus)) {
-      return split_grouped(prm, rows_per_expert, total_rows_estimate, static_cast<int>(cus), stream);
+    SplitShape shape;
+    if (split_chosen(prm, total_rows_estimate, cus, &shape)) {
+      return split_grouped(prm, rows_per_expert, total_rows_estimate, static_cast<int>(cus), shape, stream);
     }
   }
   // Largest tile that still gives every CU work (two tiles per CU for the

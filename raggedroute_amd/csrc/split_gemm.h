@@ -11,8 +11,10 @@ namespace rr::kern {
 bool split_gemm_fits(const GemmParams& prm);
 // Whether a grouped GEMM of this size takes the split kernel (rows: of all experts).
 bool split_gemm_ok(int k, int n, int experts, long rows, int cus);
-// Grouped (prm.sorted_route null) or chain form. rows: of all experts (picks the
-// tile shape); rows_per_expert sizes the grid only.
-hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, long rows, int cus, hipStream_t stream);
+enum class SplitShape { kBySize, kFourWaves, kEightWaves, kRows256 };
+// Grouped (prm.sorted_route null) or chain form (no 256-row tiles). rows: of all
+// experts (picks the tile shape); rows_per_expert sizes the grid only.
+hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, long rows, int cus, SplitShape shape,
+                         hipStream_t stream);
 
 }  // namespace rr::kern

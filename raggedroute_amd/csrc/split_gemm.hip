@@ -32,9 +32,15 @@
 // 2^-22 of the largest, and values whose xs is below 2^-14 are few among larger
 // ones. (A scaled value under 2^-149 counts as zero: |x| < 2^-115 in a row whose
 // sample is 2^40.) An operand past the FP16 range makes every output it meets
-// non-finite. A tile that holds a marked row or column or shows a non-finite sum
-// is computed again on the FP32 instructions before anything is stored (with the
-// FP32 rules for infinities, NaN and overflow). N(0,1) rows are marked once in
+// non-finite. Outputs of marked rows and columns and non-finite ones are computed
+// on the FP32 instructions instead, with the bits of the FP32 kernels. Which those
+// are is a matter of each output's own row and column, so that no row's bits
+// depend on the rows it shares a tile with, or on the tile's height. A tile
+// with such outputs goes through its slices once more, with FP32 products only
+// for the 16-row blocks that hold one: E = 8, 16384 rows, K = 4096, N = 14336, one
+// infinite row in a thousand 10.4 ms (17.4 when whole tiles were computed again, as
+// 32 x 32 products without a slice on its way; FP32 kernel 13.8); E = 128, 32768
+// rows, K = 2048, N = 768 569 us (979; 760). N(0,1) rows are marked once in
 // 10^9 (four values of 2^-20 side by side); rows of which half the values are zero,
 // five in 10^4 at K = 4096. The marks take 24 of 132 vector instructions of a slice of
 // the 256-row loop: T = 8192, E = 8, K = 4096, N = 14336 call 6.80 -> 7.21 ms, T = 3001,
@@ -75,6 +81,7 @@ namespace rr::kern {
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -88,7 +95,6 @@ constexpr float kLeast = 0x1p-14F;          // scaled values from here on keep a
 constexpr int kFewSmall = 4;                // too small values of slice 0 that send a row or column to FP32
 constexpr int kMarked = 1 << 16;            // scale exponent of a row or column that is not computed in FP16
 constexpr int kBufferFlags = 0x00027000;    // raw 32-bit buffer
-constexpr int kRefLd = kBK + 1;             // FP32 recomputation: padded LDS row (floats)
 
 // BM x 128 output tiles on W waves (four: two workgroups per CU; eight: one).
 template <int W, int BM>
@@ -100,7 +106,9 @@ struct Shape {
   static constexpr int kKPer = kBK / W;                          // k rows of B a thread stages
   static constexpr int kPlaneA = kBM * kBK;                      // halfs
   static constexpr int kStage = 2 * (kPlaneA + kPlaneB);         // A high, A low, B high, B low
-  static_assert((kBM + kBN) * kRefLd * sizeof(float) <= 2 * kStage * sizeof(_Float16), "the FP32 slices fit the stages");
+  static constexpr int kStage32 = (kBM + kBN) * kBK;             // floats
+  static_assert(2 * kStage32 * sizeof(float) <= 2 * kStage * sizeof(_Float16), "two FP32 slices fit the stages");
+  static_assert(kBM * (kBN / 32) * sizeof(uint32_t) <= W * 64 * sizeof(uint2), "the masks fit the column samples");
 };
 
 // Wave tiles of TM x TN blocks of 32 x 32. GRID: W / 2 x 2 waves of TN = 2 column
@@ -177,7 +185,7 @@ struct Lds {
   _Float16* stages;  // [2][kStage]
   int32_t* ta;       // [kBM] scale exponents of the rows (kMarked: FP32)
   int32_t* tb;       // [128] ... of the plane rows of B
-  uint2* cmax;       // [W][64] column samples
+  uint2* cmax;       // [W][64] column samples; after the slices [kBM][4] masks of the outputs to recompute
   int32_t* few;      // [128] values of slice 0 too small for their column's scale
   int32_t* src;      // [kBM] chain: token row of X per tile row (-1: none)
   float* w;          // [kBM] chain: route weight per tile row
@@ -543,54 +551,9 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     }
   }
 
-  // (the lane id passes an empty asm so that none of the epilogue's addresses
-  // is built before the loop and kept live across it)
-  int ln = lane;
-  asm volatile("" : "+v"(ln));
-  const int eli = ln & 31;
-  const int ehi = ln >> 5;
-  // output rows of accumulator register r: 32 i + 8 (r / 4) + 4 hi + r % 4 of the wave's
-  const int col = tl.n0 + L::col(wave) + eli;  // block j: 32 j further
-  const int prow = L::col(wave) + eli;
-  auto store_tile = [&](bool scaled) {
-    int tb[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) tb[j] = sh.tb[prow + 32 * j];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
-        if (rl >= rows) continue;
-        const int ta = sh.ta[rl];
-        float v[TN];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) v[j] = scaled ? ldexpf(acc[i][j][r], -(ta + tb[j])) : acc[i][j][r];
-        float* yrow = prm.Y + static_cast<std::size_t>(tl.row0 + rl) * N + col;
-        float* comb = nullptr;
-        float w = 0.0F;
-        if constexpr (CHAIN) {
-          if (prm.y_out != nullptr) {
-            comb = prm.y_out + static_cast<std::size_t>(sh.src[rl]) * N + col;
-            w = sh.w[rl];
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          if (col + 32 * j >= N) continue;
-          if (comb != nullptr) {
-            __builtin_nontemporal_store(v[j], yrow + 32 * j);  // y_permuted is not read again by the chain
-            // Both routes of a token add into the zeroed output: fl(0 + a) + b
-            // is the same in either order, so the combine is deterministic
-            // and equals the rank-order unpermute.
-            unsafeAtomicAdd(comb + 32 * j, __fmul_rn(w, v[j]));
-          } else {
-            yrow[32 * j] = v[j];
-          }
-        }
-      }
-    }
-  };
+  // What the scales could not carry: marked rows and columns, and sums that are
+  // not finite. (Each a matter of the output's own row and column, whatever else
+  // is in the tile.)
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     if ((small_a[p] >> lane & 1) != 0) sh.ta[PR * p + ar] = kMarked;
@@ -599,10 +562,19 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   for (int j = 0; j < 2; ++j) {
     if ((small_b[j] >> lane & 1) != 0) sh.tb[2 * pair + j] = kMarked;
   }
+  if (tid < kBN && sh.few[tid] >= kFewSmall) sh.tb[tid] = kMarked;
   __syncthreads();
-  // (what lies outside the tile is not stored)
-  bool overflow = tid < rows && sh.ta[tid] == kMarked;
-  if (tid < kBN && tl.n0 + tid < N) overflow = overflow || sh.tb[tid] == kMarked || sh.few[tid] >= kFewSmall;
+
+  // (the lane id passes an empty asm so that none of the epilogue's addresses
+  // is built before the loop and kept live across it)
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int eli = ln & 31;
+  const int ehi = ln >> 5;
+  // output rows of accumulator register r: 32 i + 8 (r / 4) + 4 hi + r % 4 of the wave's
+  const int ec = L::col(wave) + eli;  // tile column; block j: 32 j further
+  bool odd = tid < rows && sh.ta[tid] == kMarked;
+  if (tid < kBN && tl.n0 + tid < N) odd = odd || sh.tb[tid] == kMarked;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -611,52 +583,152 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       for (int r = 0; r < 16; ++r) {
         const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
         acc[i][j][r] = __builtin_fmaf(low[i][j][r], 1.0F / kLowScale, acc[i][j][r]);
-        overflow = overflow || (rl < rows && col + 32 * j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
+        odd = odd || (rl < rows && tl.n0 + ec + 32 * j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
       }
     }
   }
-  const bool redo = __syncthreads_or(overflow ? 1 : 0) != 0;
+  const bool redo = __syncthreads_or(odd ? 1 : 0) != 0;
+  // the combined row of tile row rl (chain) and an output's way to memory
+  auto combined_row = [&](int rl) -> float* {
+    if constexpr (CHAIN) {
+      if (prm.y_out != nullptr) return prm.y_out + static_cast<std::size_t>(sh.src[rl]) * N + tl.n0;
+    }
+    return nullptr;
+  };
+  auto emit = [&](float v, float* y, float* comb, float w) {
+    if (comb != nullptr) {
+      __builtin_nontemporal_store(v, y);  // y_permuted is not read again by the chain
+      // Both routes of a token add into the zeroed output: fl(0 + a) + b
+      // is the same in either order, so the combine is deterministic
+      // and equals the rank-order unpermute.
+      unsafeAtomicAdd(comb, __fmul_rn(w, v));
+    } else {
+      *y = v;
+    }
+  };
+  float* const ytile = prm.Y + static_cast<std::size_t>(tl.row0) * N + tl.n0;
+  uint32_t* mask = reinterpret_cast<uint32_t*>(sh.cmax);  // [row][column / 32]
+  int tb[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) tb[j] = sh.tb[ec + 32 * j];
+  uint32_t again[TM] = {};  // bit 16 j + r: output (i, j, r) is one of those
   if (redo) {
-    // the same tile on the FP32 instructions, slices staged unscaled
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
+      for (int r = 0; r < 16; ++r) {
+        const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
+        const int ta = sh.ta[rl];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0F;
-      }
-    }
-    float* As = reinterpret_cast<float*>(sh.stages);
-    float* Bs = As + S::kBM * kRefLd;
-#pragma unroll 1
-    for (int kt = 0; kt < nk; ++kt) {
-      load_any(kt);
-      __syncthreads();  // the previous slice is used up
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) As[(PR * p + ar) * kRefLd + 4 * ac + q] = ra[p][q];
-      }
-#pragma unroll
-      for (int j = 0; j < KP; ++j) {
-        Bs[2 * pair * kRefLd + b_k + j] = rb[j][0];
-        Bs[(2 * pair + 1) * kRefLd + b_k + j] = rb[j][1];
-      }
-      __syncthreads();
-#pragma unroll 1
-      for (int k = 0; k < kBK; k += 2) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const float a = As[(wrow + 32 * i + eli) * kRefLd + k + ehi];
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, Bs[(prow + 32 * j) * kRefLd + k + ehi], acc[i][j], 0, 0, 0);
-          }
+        for (int j = 0; j < TN; ++j) {
+          const bool a = rl < rows && tl.n0 + ec + 32 * j < N &&
+                         (ta == kMarked || tb[j] == kMarked || abs_bits(acc[i][j][r]) >= 0x7F800000U);
+          const uint64_t m = __ballot(a);
+          if (eli == 0) mask[4 * rl + (L::col(wave) >> 5) + j] = static_cast<uint32_t>(ehi == 0 ? m : m >> 32);
+          again[i] |= a ? 1U << (16 * j + r) : 0U;
         }
       }
     }
   }
-  store_tile(!redo);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
+      if (rl >= rows) continue;
+      const int ta = sh.ta[rl];
+      float* yrow = ytile + static_cast<std::size_t>(rl) * N + ec;
+      float* comb = combined_row(rl);
+      const float w = comb != nullptr ? sh.w[rl] : 0.0F;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if (tl.n0 + ec + 32 * j >= N || (again[i] >> (16 * j + r) & 1) != 0) continue;
+        emit(ldexpf(acc[i][j][r], -(ta + tb[j])), yrow + 32 * j, comb != nullptr ? comb + ec + 32 * j : nullptr, w);
+      }
+    }
+  }
+  if (!redo) return;
+
+  // ---- the masked outputs on the FP32 instructions (v_mfma_f32_16x16x4_f32) ----
+  // Slices of both operands as they are, k order as in every FP32 GEMM here
+  // (chunks of 16 k ascending, MFMA step s sums k = 16 c + 4 g + s over g): the bits
+  // of the FP32 kernels. Wave w takes kBN / W columns and those of the tile's
+  // 16-row blocks that have a masked output there.
+  constexpr int CW = kBN / W;
+  constexpr int NJ = CW / 16;
+  constexpr int NB = L::kRows / 16;
+  const int g = ln >> 4 & 3;
+  const int fl = ln & 15;
+  __syncthreads();  // masks
+  uint32_t blocks = 0;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const uint32_t m = mask[4 * (16 * i + fl) + (CW * wave >> 5)] >> (CW * wave & 31);
+    if (__ballot((CW == 32 ? m : m & 0xFFFFU) != 0) != 0) blocks |= 1U << i;
+  }
+  v4f sum[NB][NJ];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) sum[i][j] = v4f{0.0F, 0.0F, 0.0F, 0.0F};
+  }
+  // quad q of plane row r sits at quad q ^ (r & 7) (B: q ^ (r / 2 & 7))
+  load_any(0);
+#pragma unroll 1
+  for (int kt = 0; kt < nk; ++kt) {
+    float* As = reinterpret_cast<float*>(sh.stages) + (kt & 1) * S::kStage32;
+    float* Bs = As + S::kBM * kBK;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int r = PR * p + ar;
+      *reinterpret_cast<v4f*>(As + r * kBK + 4 * (ac ^ (r & 7))) = v4f{ra[p][0], ra[p][1], ra[p][2], ra[p][3]};
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int q = 0; q < KP / 4; ++q) {
+        *reinterpret_cast<v4f*>(Bs + (2 * pair + j) * kBK + 4 * ((b_k / 4 + q) ^ (pair & 7))) =
+            v4f{rb[4 * q][j], rb[4 * q + 1][j], rb[4 * q + 2][j], rb[4 * q + 3][j]};
+      }
+    }
+    if (kt + 1 < nk) load_any(kt + 1);
+    __syncthreads();  // (the other stage was last read before the previous slice's barrier)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      v4f b[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int col = CW * wave + 16 * j + fl;
+        b[j] = *reinterpret_cast<const v4f*>(Bs + col * kBK + 4 * ((4 * c + g) ^ (col >> 1 & 7)));
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        if ((blocks >> i & 1) == 0) continue;
+        const v4f a = *reinterpret_cast<const v4f*>(As + (16 * i + fl) * kBK + 4 * ((4 * c + g) ^ (fl & 7)));
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[j][s], sum[i][j], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    if ((blocks >> i & 1) == 0) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int rl = 16 * i + 4 * g + r;
+      float* comb = rl < rows ? combined_row(rl) : nullptr;
+      const float w = comb != nullptr ? sh.w[rl] : 0.0F;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int c = CW * wave + 16 * j + fl;
+        if ((mask[4 * rl + (c >> 5)] >> (c & 31) & 1) == 0) continue;
+        emit(sum[i][j][r], ytile + static_cast<std::size_t>(rl) * N + c, comb != nullptr ? comb + c : nullptr, w);
+      }
+    }
+  }
 }
 
 template <int W, int BM, bool CHAIN>
@@ -812,17 +884,23 @@ bool split_gemm_fits(const GemmParams& prm) {
 //    Not for the chain: nothing runs under a tile's combine with one workgroup
 //    a CU (T = 16384, E = 128, K = 2048, N = 768 chain 724 against 641 us);
 //  - else four waves on 128-row tiles, two workgroups a CU.
-hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, long rows, int cus, hipStream_t stream) {
+hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, long rows, int cus, SplitShape shape,
+                         hipStream_t stream) {
   const bool chain = prm.sorted_route != nullptr;
-  if (2 * tiles(rows, prm.experts, 128, prm.N, kBN) <= 3L * cus) {
+  if (shape == SplitShape::kBySize) {
+    if (2 * tiles(rows, prm.experts, 128, prm.N, kBN) <= 3L * cus) {
+      shape = SplitShape::kEightWaves;
+    } else if (prm.K >= 512 && tiles(rows, prm.experts, 256, prm.N, kBN) >= 2L * cus &&
+               rows * prm.K >= (1L << 18) * prm.experts) {
+      shape = SplitShape::kRows256;
+    }
+  }
+  if (shape == SplitShape::kEightWaves) {
     return chain ? launch<8, 128, true>(prm, rows_per_expert, cus, stream)
                  : launch<8, 128, false>(prm, rows_per_expert, cus, stream);
   }
   if (chain) return launch<4, 128, true>(prm, rows_per_expert, cus, stream);
-  if (prm.K >= 512 && tiles(rows, prm.experts, 256, prm.N, kBN) >= 2L * cus &&
-      rows * prm.K >= (1L << 18) * prm.experts) {
-    return launch<8, 256, false>(prm, rows_per_expert, cus, stream);
-  }
+  if (shape == SplitShape::kRows256) return launch<8, 256, false>(prm, rows_per_expert, cus, stream);
   return launch<4, 128, false>(prm, rows_per_expert, cus, stream);
 }
 

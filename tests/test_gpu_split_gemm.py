@@ -139,6 +139,71 @@ def test_values_past_the_fp16_range(ctx, device, staging, case):
             assert (err <= 4 * gamma * mag + 2 * x.shape[1] * 2.0 ** -149)[fin].all(), (case, e)
 
 
+SHAPES = ["split4", "split8", "split256"]
+
+
+@pytest.mark.parametrize("case", ["infinity and NaN", "late outlier", "tiny", "overflow", "row scales", "scattered"])
+def test_recomputed_outputs_are_the_fp32_kernels(ctx, device, staging, case):
+    """Each output is either the split's or the FP32 kernels', bit for bit, by its
+    own row and column: the same in every workgroup shape (so whatever other rows
+    its tile holds), and where rows or columns were changed, no other output moves."""
+    if case == "scattered":  # a few odd rows and columns in tiles of ordinary ones
+        rng = np.random.default_rng(12)
+        counts, k, n = [700, 3, 257, 130], 200, 300
+        x = rng.standard_normal((sum(counts), k)).astype(np.float32)
+        w = (rng.standard_normal((4, k, n)) / np.sqrt(k)).astype(np.float32)
+        plain = x.copy(), w.copy()
+        rows, cols = [5, 300, 511, 800], {0: [7, 290], 2: [131]}
+        x[5, 199] = np.inf
+        x[300, 0] = 2.0 ** 40
+        x[511, 100] = 1e5
+        x[800, 3] = np.nan
+        for e, cs in cols.items():
+            w[e][60, cs] = 3e4
+    else:
+        counts, x, w = special_inputs(case, np.random.default_rng(11))
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+
+    def bits(path, xs, ws):
+        staging(path)
+        return run_grouped(ctx, device, xs, ws, offsets, NATIVE).view(np.uint32)
+    fp32 = bits("fp32", x, w)
+    split = [bits(shape, x, w) for shape in SHAPES]
+    for other in split[1:]:
+        assert np.array_equal(split[0], other)
+    if case in ("late outlier", "tiny"):  # every row
+        assert np.array_equal(split[0], fp32)
+    if case == "scattered":
+        touched = np.zeros(fp32.shape, bool)
+        touched[rows] = True
+        for e, cs in cols.items():
+            touched[offsets[e]:offsets[e + 1], cs] = True
+        assert np.array_equal(split[0][touched], fp32[touched])
+        assert np.array_equal(split[0][~touched], bits("split4", *plain)[~touched])
+
+
+@pytest.mark.parametrize("shape", ["split4", "split8"])
+def test_chain_with_odd_rows(ctx, device, staging, shape):
+    """The chain's gathered form (128-row tiles) against the staged operators in
+    256-row tiles, with infinities, late and early outliers in x: every output
+    the same bits."""
+    cfg = workloads.ChainConfig("split", 700, 5, 256, 272)
+    inp = workloads.chain_inputs(cfg, seed=6)
+    x = inp["x"]
+    x[3, 100] = 3e5
+    x[77, 255] = -4e6
+    x[300, 2] = 2.0 ** 30
+    x[301, 200] = np.inf
+    x[555] = 0
+    staging(shape)
+    fused = ChainRun(cfg, inp, device).run(ctx)
+    staging("split256")
+    ref = run_stages(cfg, inp, device, ctx)
+    assert not np.isfinite(fused["y"]).all() and np.isfinite(fused["y"]).any()
+    for key in ("ids", "route_pos", "x_permuted", "y_permuted", "y"):
+        assert np.array_equal(fused[key].view(np.uint32), ref[key].view(np.uint32)), f"{key} differs"
+
+
 def two_norm_error(y, x, w, offsets):
     num = den = 0.0
     for e in range(len(w)):
