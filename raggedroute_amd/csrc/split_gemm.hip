@@ -17,9 +17,12 @@
 // K = 64 0.98 / 1.43e-7, K = 256 1.31 / 2.87e-7, K = 1024 2.2 / 5.8e-7, K = 4096
 // 4.1 / 11.4e-7; likewise for non-negative and half-zero operands).
 //
-// Range. The scale puts the largest of a row's (column's) first nonzero slice
-// of 32 k near 2^6, so later values may be 2^9 times larger before fp16(xs)
-// overflows. l, stored times 2^11, keeps its 11 bits down to |xs| = 2^-14 (2^-20
+// Range. The scale puts the largest of a row's (column's) first slice of 32 k
+// near 2^6, so later values may be 2^9 times larger before fp16(xs)
+// overflows. (Where that slice is all zero, 1 is taken for the largest; reading on
+// to the first value made a tile with one all-zero row, a padding token, scan all
+// of K first: E = 8, 16384 rows, K = 4096, N = 14336 11.7 ms, now 6.3 as without such
+// rows; E = 64, 4096 rows, K = 1024, N = 512 72 -> 36 us.) l, stored times 2^11, keeps its 11 bits down to |xs| = 2^-14 (2^-20
 // of the sampled maximum); below, the split's error stays at 2^-36, so that values
 // much smaller than the sample lose their bits: with one feature 2^p times the
 // rest and its weights zero, K = 320, the 2-norm error was 1.8e-6 at p = 24, 1.1e-4
@@ -40,7 +43,9 @@
 // for the 16-row blocks that hold one: E = 8, 16384 rows, K = 4096, N = 14336, one
 // infinite row in a thousand 10.4 ms (17.4 when whole tiles were computed again, as
 // 32 x 32 products without a slice on its way; FP32 kernel 13.8); E = 128, 32768
-// rows, K = 2048, N = 768 569 us (979; 760). N(0,1) rows are marked once in
+// rows, K = 2048, N = 768 569 us (979; 760). Where every row has such a value (a
+// feature 2^14 times the others) the second pass is a whole FP32 product and comes
+// on top: 23.0 ms and 1.36 ms. N(0,1) rows are marked once in
 // 10^9 (four values of 2^-20 side by side); rows of which half the values are zero,
 // five in 10^4 at K = 4096. The marks take 24 of 132 vector instructions of a slice of
 // the 256-row loop: T = 8192, E = 8, K = 4096, N = 14336 call 6.80 -> 7.21 ms, T = 3001,
@@ -156,7 +161,9 @@ __device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v
 __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
 
 // The scale of a row or column whose sampled maximum has these bits: s = 2^t
-// with t = 6 - floor(log2(max)); 1 for an all-zero sample.
+// with t = 6 - floor(log2(max)). An all-zero sample is taken for one of largest
+// value 1: an all-zero row or column is exact under any scale, and later values
+// between 2^-20 and 2^9 are carried.
 struct Scale {
   float s;
   int t;
@@ -166,7 +173,7 @@ __device__ __forceinline__ Scale scale_of(uint32_t bits) {
   Scale sc;
   int e = static_cast<int>(bits >> 23);
   sc.bad = bits != 0 && (e > 167 || e < 27);
-  e = bits == 0 ? 133 : (e < 27 ? 27 : e);
+  e = bits == 0 ? 127 : (e < 27 ? 27 : e);
   sc.t = 133 - e;
   sc.s = __uint_as_float(static_cast<uint32_t>(260 - e) << 23);
   return sc;
@@ -288,48 +295,31 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     }
   };
 
-  // ---- scales: the first slice with a nonzero value, per row and column ----
-  // (almost always slice 0; a tile with an all-zero row or column reads on)
+  // ---- scales, from the first slice ----
   load_any(0);
   if (tid < kBN) sh.few[tid] = 0;
-  uint32_t ma[P] = {};
+  uint32_t ma[P];
   uint32_t mb0 = 0, mb1 = 0;
-#pragma unroll 1
-  for (int kt = 0;;) {
-    bool need = false;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      uint32_t m = umax(umax(abs_bits(ra[p][0]), abs_bits(ra[p][1])), umax(abs_bits(ra[p][2]), abs_bits(ra[p][3])));
-      // over the row's eight lanes: quad neighbours, then the half row's mirror
-      m = umax(m, rr::dev::dpp_move<0xB1>(m));
-      m = umax(m, rr::dev::dpp_move<0x4E>(m));
-      m = umax(m, rr::dev::dpp_move<0x141>(m));
-      if (ma[p] == 0) ma[p] = m;
-      need = need || (ma[p] == 0 && PR * p + ar < rows);
-    }
-    uint32_t c0 = 0, c1 = 0;
+  for (int p = 0; p < P; ++p) {
+    uint32_t m = umax(umax(abs_bits(ra[p][0]), abs_bits(ra[p][1])), umax(abs_bits(ra[p][2]), abs_bits(ra[p][3])));
+    // over the row's eight lanes: quad neighbours, then the half row's mirror
+    m = umax(m, rr::dev::dpp_move<0xB1>(m));
+    m = umax(m, rr::dev::dpp_move<0x4E>(m));
+    ma[p] = umax(m, rr::dev::dpp_move<0x141>(m));
+  }
 #pragma unroll
-    for (int j = 0; j < KP; ++j) {
-      c0 = umax(c0, abs_bits(rb[j][0]));
-      c1 = umax(c1, abs_bits(rb[j][1]));
-    }
-    sh.cmax[64 * wave + pair] = make_uint2(c0, c1);
-    __syncthreads();
-    c0 = c1 = 0;
+  for (int j = 0; j < KP; ++j) {
+    mb0 = umax(mb0, abs_bits(rb[j][0]));
+    mb1 = umax(mb1, abs_bits(rb[j][1]));
+  }
+  sh.cmax[64 * wave + pair] = make_uint2(mb0, mb1);
+  __syncthreads();
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      const uint2 m = sh.cmax[64 * w + pair];
-      c0 = umax(c0, m.x);
-      c1 = umax(c1, m.y);
-    }
-    if (mb0 == 0) mb0 = c0;
-    if (mb1 == 0) mb1 = c1;
-    need = need || (mb0 == 0 && n < N) || (mb1 == 0 && n + 1 < N);
-    if (__syncthreads_or(need ? 1 : 0) == 0 || kt + 1 >= nk) {
-      if (kt > 0) load_any(0);
-      break;
-    }
-    load_any(++kt);
+  for (int w = 0; w < W; ++w) {
+    const uint2 m = sh.cmax[64 * w + pair];
+    mb0 = umax(mb0, m.x);
+    mb1 = umax(mb1, m.y);
   }
   float sa[P], sb[2];
 #pragma unroll

@@ -182,6 +182,30 @@ def test_recomputed_outputs_are_the_fp32_kernels(ctx, device, staging, case):
         assert np.array_equal(split[0][~touched], bits("split4", *plain)[~touched])
 
 
+@pytest.mark.parametrize("p", [-40, -20, -12, 0, 9, 11, 30])
+@pytest.mark.parametrize("side", ["row", "column"])
+def test_zero_first_slice(ctx, device, staging, side, p):
+    """All-zero rows and columns, and ones whose first slice is zero and whose
+    other values are 2^p: as close to the exact results as the FP32 instructions'
+    (the bound of test_values_far_below_the_sample)."""
+    rng = np.random.default_rng(p + 50)
+    counts, k, n = [200, 40, 90, 20], 320, 400
+    x = rng.standard_normal((sum(counts), k)).astype(np.float32)
+    w = (rng.standard_normal((4, k, n)) / np.sqrt(k)).astype(np.float32)
+    a = x.T if side == "row" else w.transpose(1, 0, 2)  # views, k first
+    a *= np.float32(2.0 ** p)
+    a[:32] = 0
+    a[..., 5::17] = 0
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    y = {}
+    for path in ("fp32", "split4", "split8", "split256"):
+        staging(path)
+        y[path] = run_grouped(ctx, device, x, w, offsets, NATIVE)
+    assert np.array_equal(y["split4"], y["split8"]) and np.array_equal(y["split4"], y["split256"])
+    assert two_norm_error(y["split4"], x, w, offsets) <= 1.25 * two_norm_error(y["fp32"], x, w, offsets)
+    assert (y["split4"] == 0)[y["fp32"] == 0].all()
+
+
 @pytest.mark.parametrize("shape", ["split4", "split8"])
 def test_chain_with_odd_rows(ctx, device, staging, shape):
     """The chain's gathered form (128-row tiles) against the staged operators in
