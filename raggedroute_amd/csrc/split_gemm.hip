@@ -835,23 +835,32 @@ long tiles(long rows, int experts, int bm, int n, int bn) { return (ceil_div(row
 
 }  // namespace
 
-// Where the FP32 kernels stay: problems of so few tiles that their smaller
-// tiles spread over more CUs (with K >= 512, below one 64 x 64 tile a CU; with
-// shorter K, where a tile's scales and first loads weigh more, below 2.5), and
-// K < 128 or N <= 64, where neither side is bound by the matrix instructions, and
-// K and N both below 256 (chain T = 10296, E = 12, K = 100, N = 153 53 / 59 us, T =
-// 2523, E = 10, K = 106, N = 667 49 / 53; T = 14884, E = 75, K = 128, N = 608 125 / 112).
-// Grouped GEMM alone, FP32 kernels / this one: E = 8, K = 1024, N = 512 with 1024
-// rows (192 tiles) 37 / 38 us, 2048 rows (320) 48 / 41, 8192 rows 106 / 70;
-// E = 16, K = 2048, N = 300 with 2048 rows (240) 66 / 65 us, 8192 rows 157 / 73;
-// E = 64, K = 512, N = 768 with 64 rows 24 / 21 us, 4096 rows 69 / 37; E = 64,
-// K = 256, N = 200 with 4096 rows (512) 17 / 19 us, 8192 rows (768) 27 / 20;
-// E = 16, K = 250, N = 1024 with 1024 rows (512) 18 / 20 us, 2048 rows (768)
-// 31 / 22; E = 64, K = 64, N = 200 with 16384 rows 18 / 18 us.
+// Where the FP32 kernels stay (grouped GEMM alone, experts' rows drawn at random,
+// FP32 kernels / this one):
+//  - K < 128 or N <= 64, where neither side is bound by the matrix instructions, and
+//    K and N both below 256 (chain T = 10296, E = 12, K = 100, N = 153 53 / 59 us, T =
+//    2523, E = 10, K = 106, N = 667 49 / 53);
+//  - problems of so few tiles that their smaller tiles spread over more CUs: with
+//    K >= 512 below one 64 x 64 tile a CU (E = 8, K = 1024, N = 512, 1024 rows, 192 tiles
+//    22 / 40 us; 4096 rows, 576 tiles 48 / 42), or 1.25 where the experts have less than
+//    eight rows each (E = 8, K = 512, N = 2048, 32 rows 16.3 / 20.0); with shorter K,
+//    where a tile's scales and first loads weigh more, below 2.5 (E = 16, K = 256,
+//    N = 1024, 1600 rows 17.8 / 18.9; E = 8, K = 256, N = 1536, 1200 rows, 648 tiles
+//    28.1 / 19.4), and up to 3 with K < 192 (E = 16, K = 128, N = 1024, 1600 rows, 656
+//    tiles 11.3 / 15.0; E = 64, K = 128, N = 768, 1536 rows, 1056 tiles 18.2 / 12.8);
+//  - few rows an expert where the FP32 side has its 128 x 128 tiles (two a CU): both
+//    are bound by the weights, which those load straight into LDS. E = 64, K = 128,
+//    N = 1024: 256 rows 8.6 / 11.7, 2048 rows 15.7 / 16.7, 3072 rows 19.6 / 18.0; E = 128,
+//    K = 320, N = 1024: 16 rows each 34.0 / 36.1, 24 rows 49.0 / 41.0; K = 1024: 4 rows each
+//    89 / 99, 16 rows 99 / 105, 24 rows 141 / 111; K = 4096: 4 rows each 314 / 349, 10 rows
+//    342 / 358, 16 rows 365 / 359 (chain K = 2048, N = 768, 10 rows each 222 / 215).
 bool split_gemm_ok(int k, int n, int experts, long rows, int cus) {
   if (k < 128 || n <= 64 || (k < 256 && n < 256)) return false;
+  const long few = k < 192 ? 36 : (k < 512 ? 20 : (k < 2048 ? 16 : 8));  // rows an expert
+  if (rows < few * experts && tiles(rows, experts, 128, n, 128) >= 2L * cus) return false;
   const long t = tiles(rows, experts, 64, n, 64);
-  return k >= 512 ? t >= cus : 2 * t >= 5L * cus;
+  if (k >= 512) return 4 * t >= (rows < 8L * experts ? 5L : 4L) * cus;
+  return k < 192 ? t > 3L * cus : 2 * t >= 5L * cus;
 }
 
 // 32-bit byte offsets: a tile's A rows (chain: all of X) and an expert's weights.

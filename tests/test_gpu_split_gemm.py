@@ -139,6 +139,29 @@ def test_values_past_the_fp16_range(ctx, device, staging, case):
             assert (err <= 4 * gamma * mag + 2 * x.shape[1] * 2.0 ** -149)[fin].all(), (case, e)
 
 
+@pytest.mark.parametrize("path,experts,rows,k,n", [
+    # few rows an expert, many tiles; few tiles; short K
+    ("fp32", 64, 256, 128, 1024), ("fp32", 64, 1024, 256, 1024), ("fp32", 32, 128, 1024, 2048),
+    ("fp32", 8, 32, 512, 2048), ("fp32", 8, 1024, 1024, 512), ("fp32", 16, 1600, 128, 1024),
+    # enough of both
+    ("split", 64, 3072, 128, 1024), ("split", 32, 512, 512, 500), ("split", 8, 4096, 1024, 512),
+    ("split", 16, 1600, 192, 1024), ("split", 8, 1200, 256, 1536),
+])
+def test_kernel_by_size(ctx, device, staging, path, experts, rows, k, n):
+    """The kernel that measures faster on MI355X (256 CUs), seen by its bits."""
+    rng = np.random.default_rng(rows + k)
+    counts = np.bincount(rng.integers(0, experts, rows), minlength=experts)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (rng.standard_normal((experts, k, n)) / np.sqrt(k)).astype(np.float32)
+    y = {}
+    for name in ("fp32", "split", "default"):
+        staging(name)
+        y[name] = run_grouped(ctx, device, x, w, offsets, NATIVE)
+    assert not np.array_equal(y["fp32"], y["split"])
+    assert np.array_equal(y["default"], y[path])
+
+
 SHAPES = ["split4", "split8", "split256"]
 
 
