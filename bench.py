@@ -45,7 +45,7 @@ FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix, vendor peak
 # FP32 products made of three FP16 ones (the split grouped GEMM): a third of the
 # dense FP16 vendor peak
 SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 3
-RIDGE = FP32_MFMA_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9)  # flop/byte
+RIDGE = FP32_MFMA_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9)  # flop/byte, FP32 instructions
 
 
 SUITES = ("chain_from_tokens", "chain_from_logits", "chain_from_route_ids")
@@ -131,14 +131,14 @@ def fused_work_model(t, e, k, n, active=None):
     }
 
 
-def roofline(name, nbytes, flops, seconds):
-    ai = flops / nbytes if nbytes else 0.0
-    if flops and ai > RIDGE:
+def roofline(name, nbytes, flops, seconds, split=False):
+    """Share of the bounding peak. split: the products ran on the split path (on_split)."""
+    peak = round(SPLIT_MFMA_PEAK_TFLOPS if split else FP32_MFMA_PEAK_TFLOPS, 1)
+    ridge = SPLIT_MFMA_PEAK_TFLOPS / FP32_MFMA_PEAK_TFLOPS * RIDGE if split else RIDGE
+    if flops and flops / nbytes > ridge:
         achieved = flops / seconds / 1e12
-        # (a rate past the FP32 peak was reached on the split path)
-        peak = FP32_MFMA_PEAK_TFLOPS if achieved <= FP32_MFMA_PEAK_TFLOPS else round(SPLIT_MFMA_PEAK_TFLOPS, 1)
-        return {"bound": "mfma", "achieved": round(achieved, 3), "peak": peak,
-                "unit": "TFLOP/s", "frac": round(achieved / peak, 4)}
+        return {"bound": "mfma", "products": "three fp16" if split else "fp32", "achieved": round(achieved, 3),
+                "peak": peak, "unit": "TFLOP/s", "frac": round(achieved / peak, 4)}
     achieved = nbytes / seconds / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4)}
@@ -456,14 +456,34 @@ def graph_report(torch, device, ch, reps=200):
     return out
 
 
+def on_split(torch, call, y):
+    """Whether the grouped GEMM that `call` runs into y takes the split kernel:
+    whether its bits change when RR_GEMM_STAGING=fp32 rules that kernel out."""
+    saved = os.environ.get("RR_GEMM_STAGING")
+    call()
+    default = y.clone()
+    try:
+        os.environ["RR_GEMM_STAGING"] = "fp32"
+        call()
+    finally:
+        os.environ.pop("RR_GEMM_STAGING")
+        if saved is not None:
+            os.environ["RR_GEMM_STAGING"] = saved
+    split = not torch.equal(default.view(torch.int32), y.view(torch.int32))
+    call()
+    torch.cuda.synchronize()
+    return split
+
+
 def stage_report(torch, device, ch, model, n=50):
     """Each stage operator alone, `n` calls per graph (graph_time)."""
     out = {}
     for name in ch.stage_args:
         sec = graph_time(torch, device, lambda s: ch.stage(name, s), n=n)
         nbytes, flops = model[name]
+        split = name == "grouped_gemm" and on_split(torch, lambda: ch.stage(name), ch.yp)
         out[name] = {"us": round(sec * 1e6, 2), "bytes": int(nbytes), "flops": flops,
-                     "roofline": roofline(name, nbytes, flops, sec)}
+                     "roofline": roofline(name, nbytes, flops, sec, split)}
     return out
 
 
@@ -474,8 +494,9 @@ def launch_report(torch, device, ch, model, n=50):
     for index, name in enumerate(ch.rr.chain_fused_launch_names(ch.chain_args, ch.cfg.from_tokens)):
         sec = graph_time(torch, device, lambda s: ch.fused_launch(index, s), n=n)
         nbytes, flops = model[name]
+        split = name == "expert_gemm" and on_split(torch, lambda: ch.fused_launch(index), ch.yp)
         out[name] = {"us": round(sec * 1e6, 2), "bytes": int(nbytes), "flops": flops,
-                     "roofline": roofline(name, nbytes, flops, sec)}
+                     "roofline": roofline(name, nbytes, flops, sec, split)}
     return out
 
 
@@ -557,7 +578,8 @@ def c4(torch, device, hidden=4096, output=14336, reps=5, samples=10, cpu_sample=
         nbytes, flops = model[name]
         if name == "grouped_gemm":
             sec = time_loop(torch, lambda: ch.stage(name), reps, warmup=2)  # (two calls: ~30 ms of load)
-            out[name] = {"us": round(sec * 1e6, 1), "roofline": roofline(name, nbytes, flops, sec)}
+            split = on_split(torch, lambda: ch.stage(name), ch.yp)
+            out[name] = {"us": round(sec * 1e6, 1), "roofline": roofline(name, nbytes, flops, sec, split)}
             continue
         warm = statistics.median(batch_means(torch, lambda: ch.stage(name), samples=samples, repeats=5))
         cold = sample_stats(cold_spans(torch, ch, device, samples, call=lambda: ch.stage(name)))
@@ -1202,7 +1224,8 @@ def run_runner(torch, device, args):
     if unit is not None:
         line.update(value=round(unit_count / p50, 1), unit=unit)
     else:
-        roof = roofline(target, nbytes, flops, p50)
+        split = args.operator == "grouped_gemm" and on_split(torch, call, ch.yp)
+        roof = roofline(target, nbytes, flops, p50, split)
         line.update(value=roof["achieved"], unit=roof["unit"], roofline=roof,
                     bytes=int(nbytes), flops=flops)
     del keep
