@@ -94,7 +94,8 @@ struct GroupedGemmArgs {
   int experts = 0;
   int hidden = 0;
   int output = 0;
-  // Caller-provided launch bound; offsets are never read on the host.
+  // Caller-provided launch bound on every expert's rows; offsets are never read
+  // on the host. Also chooses the kernel, as the row count of all experts.
   int max_expert_tokens = 0;
   ScalarType accumulator_dtype = ScalarType::kFp32;
   KernelSelection kernel;

@@ -215,7 +215,10 @@ typedef struct rr_grouped_gemm_args {
   int32_t experts;
   int32_t hidden;
   int32_t output;
-  int32_t max_expert_tokens; /* caller launch bound; offsets are read on device only */
+  /* caller launch bound on every expert's rows; offsets are read on device only.
+   * The kernel is chosen by it as if it were the row count of all experts: pass
+   * that where it is known. */
+  int32_t max_expert_tokens;
   int32_t accumulator_dtype;
   rr_kernel_selection kernel;
 } rr_grouped_gemm_args;
@@ -444,8 +447,8 @@ rr_status rr_chain_from_tokens_noalloc(const rr_chain_args* args, const rr_runti
  * order; their number (2 or 3) depends on the shape, and an index past the
  * last one returns RR_STATUS_INVALID_ARGUMENT. Launch 0 is the router GEMM +
  * top-2 gate (the gate only when from_tokens is 0) and zeroes y; the last
- * launch adds into y, so repeating it alone keeps accumulating. Same argument
- * checks as the chain. */
+ * launch adds into y, so repeating it alone keeps accumulating;
+ * "route_prep" may use y_permuted as scratch. Same argument checks as the chain. */
 rr_status rr_chain_fused_launch(const rr_chain_args* args, const rr_runtime_context* context,
                                 int32_t from_tokens, int32_t launch);
 /* No reference counterpart: name of fused launch `launch` for this shape

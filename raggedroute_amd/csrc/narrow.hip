@@ -18,9 +18,10 @@
 // Bound: few rows (one strip a workgroup), each wave's chain of K / 4 dependent
 // MFMAs, 44 cycles each; many rows, the FP32 matrix pipe. Measured, tiled kernel
 // / this: T = 2048, E = 64, K = 1024 15.2 / 9.6 us; T = 4096, E = 64, K = 333 8.3 /
-// 5.9; T = 8192, E = 128, K = 2048 51 / 39; T = 16384, E = 128, K = 2048 82.7 / 67.1 us
-// (128 TFLOP/s, 0.81 of the FP32 matrix peak), and the gate's own launch (5 - 10
-// us) is gone.
+// 5.8; T = 8192, E = 128, K = 2048 51 / 39; T = 16384, E = 128, K = 2048 82.8 / 67.1 us
+// (128 TFLOP/s, 0.81 of the FP32 matrix peak; a loop of this launch alone: the bench,
+// after minutes of other load, reads 77 - 79, before 85 - 95), and with the gate,
+// whose own launch is gone, 17.7 / 10.7, 10.9 / 6.9, 55.3 / 41.1 and 88.1 / 71.4 us.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>

@@ -12,22 +12,25 @@
 // the product (2^-25 in the mean) and left out. hx hy is summed in one FP32
 // accumulator and the two small terms in another, which is added once, times
 // 2^-11, at the end: the large sum is rounded once per 16 k instead of once per
-// 4 k as on the FP32 instructions. Against 64-bit sums the result is closer than
-// the FP32 instructions' at every K (2-norm error over N(0,1) operands, this / FP32 MFMA:
-// K = 64 0.98 / 1.43e-7, K = 256 1.31 / 2.87e-7, K = 1024 2.2 / 5.8e-7, K = 4096
-// 4.1 / 11.4e-7; likewise for non-negative and half-zero operands).
+// 4 k as on the FP32 instructions. Against 64-bit sums dense operands' results
+// are closer than the FP32 instructions' at every K (2-norm error over N(0,1) operands, this / FP32 MFMA:
+// K = 64 0.98 / 1.43e-7, K = 128 1.10 / 2.03e-7, K = 256 1.31 / 2.87e-7, K = 1024
+// 2.2 / 5.8e-7, K = 4096 4.1 / 11.4e-7; non-negative operands K = 128 0.64 / 1.59e-7;
+// both operands half zero K = 128 1.06 / 1.04e-7, K = 192 1.16 / 1.26e-7). Sums of few
+// products have the split's own error instead: K = 1024, rows of 64 nonzero values
+// 1.46 / 1.44e-7, of 16 1.03 / 0.74e-7, of one 0.77 / 0.25e-7.
 //
 // Range. The scale puts the largest of a row's (column's) first slice of 32 k
 // near 2^6, so later values may be 2^9 times larger before fp16(xs)
 // overflows. (Where that slice is all zero, 1 is taken for the largest; reading on
 // to the first value made a tile with one all-zero row, a padding token, scan all
 // of K first: E = 8, 16384 rows, K = 4096, N = 14336 11.7 ms, now 6.3 as without such
-// rows; E = 64, 4096 rows, K = 1024, N = 512 72 -> 36 us.) l, stored times 2^11, keeps its 11 bits down to |xs| = 2^-14 (2^-20
-// of the sampled maximum); below, the split's error stays at 2^-36, so that values
-// much smaller than the sample lose their bits: with one feature 2^p times the
-// rest and its weights zero, K = 320, the 2-norm error was 1.8e-6 at p = 24, 1.1e-4
-// at 2^30, 0.1 at 2^40 (FP32 instructions 3.2e-7). Nothing of that kind is
-// computed this way. A row or column is marked when
+// rows; E = 64, 4096 rows, K = 1024, N = 512 72 -> 36 us.) l, stored times 2^11,
+// keeps its 11 bits down to |xs| = 2^-14 (2^-20 of the sampled maximum); below, the
+// split's error stays at 2^-36, so that values much smaller than the sample lose
+// their bits: with one feature 2^p times the rest and its weights zero, K = 320, the
+// 2-norm error was 1.8e-6 at p = 24, 1.1e-4 at p = 30, 0.1 at p = 40 (FP32
+// instructions 3.2e-7). Nothing of that kind is computed this way. A row or column is marked when
 //  - its sample is below 2^-100, or 2^41 and more (or not finite);
 //  - four of its values in slice 0 are nonzero and scale to less than 2^-14;
 //  - of four consecutive k (4 i .. 4 i + 3) past slice 0 the largest does.
@@ -45,9 +48,9 @@
 // 32 x 32 products without a slice on its way; FP32 kernel 13.8); E = 128, 32768
 // rows, K = 2048, N = 768 569 us (979; 760). Where every row has such a value (a
 // feature 2^14 times the others) the second pass is a whole FP32 product and comes
-// on top: 23.0 ms and 1.36 ms. N(0,1) rows are marked once in
-// 10^9 (four values of 2^-20 side by side); rows of which half the values are zero,
-// five in 10^4 at K = 4096. The marks take 24 of 132 vector instructions of a slice of
+// on top: 23.0 ms and 1.36 ms. N(0,1) rows are as good as
+// never marked (four neighbours below 2^-19); of rows with every other value zero at
+// random, four in 10^4 at K = 4096. The marks take 24 of 132 vector instructions of a slice of
 // the 256-row loop: T = 8192, E = 8, K = 4096, N = 14336 call 6.80 -> 7.21 ms, T = 3001,
 // E = 9, K = 1023, N = 1535 150 -> 156 us, chain T = 16384, E = 128, K = 2048, N = 768
 // 607 -> 626 us, T = 2048, E = 64, K = 1024, N = 512 70.2 -> 72.1 us. (Pairs of k, and
@@ -66,13 +69,16 @@
 // Loads are buffer loads (scalar base, 32-bit lane offset): with 64-bit lane
 // addresses the eight-wave loop spilled (256 registers).
 //
-// Bound by the power limit on large problems: T = 8192, E = 8, K = 4096, N = 14336
-// (top-2, 1.92 TFLOP), FP32 instructions 14.2 ms, four waves 7.2, eight waves
-// 6.1 ms (315 TFLOP/s of FP32 products, 945 of FP16 ones; a library FP16 product
-// of random 8192 x 8192 matrices reaches 1300 on this card), and 4.5 ms with
-// operands of ones, which draw less power. Elsewhere by each tile's serial
-// parts and the combine: T = 16384, E = 128, K = 2048, N = 768 chain, expert GEMM
-// 927 / 549 us.
+// Large problems are bound by the staging phase (operand reads, split, marks and
+// plane writes of one half, longer than the other half's matrix instructions) at a
+// clock that the power limit holds down: E = 8, K = 4096, N = 14336, 16384 rows (1.92
+// TFLOP), matrix pipes busy 42 % of the cycles at 1.77 of 2.4 GHz. FP32
+// instructions 13.8 ms, four waves 7.1, eight waves 6.3 ms (304 TFLOP/s of FP32
+// products, 912 of FP16 ones; a library FP16 product of random 8192 x 8192 matrices
+// reaches 1300 on this card), 5.3 ms with operands of ones, which draw less
+// power. Elsewhere by each tile's serial parts and the combine: T = 16384, E = 128,
+// K = 2048, N = 768 chain, expert GEMM 927 / 557 us, matrix pipes 28 % busy at 2.0 GHz;
+// T = 2048, E = 64, K = 1024, N = 512 13 %.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -131,7 +137,9 @@ struct Layout {
 };
 
 // 16-byte chunk c (8 halfs) of plane row r sits at chunk c ^ ((r >> 2) & 3): the
-// 16 rows read together land in 16 distinct 16-byte bank groups.
+// 16 rows read together land in 16 distinct 16-byte bank groups. (B's writes do
+// not: 16 lanes write every second row, half of the groups; 30 % of the LDS's index
+// cycles at E = 8, K = 4096, N = 14336 are conflicts.)
 __device__ __forceinline__ int plane_swizzle(int r) { return (r >> 2) & 3; }
 
 // x * s = h + l (see the file comment): eight full-rate instructions for two
@@ -872,14 +880,13 @@ bool split_gemm_fits(const GemmParams& prm) {
 
 // Workgroup shape:
 //  - eight waves on 128-row tiles where a CU gets hardly more than one tile:
-//    more waves for it (E = 16, K = 2048, N = 300 with 8192 rows, 240 tiles: 73 us
-//    against 116 with four waves; E = 64, K = 1024, N = 512, 4096 rows, 384
-//    tiles: 40 / 59; 8192 rows, 512 tiles: 64 / 68; E = 64, K = 512, N = 768,
-//    512 rows, 408 tiles: 32 / 25);
+//    more waves for it (E = 16, K = 2048, N = 300 with 8192 rows, 240 tiles: 72 us
+//    against 89 with four waves; E = 64, K = 1024, N = 512, 4096 rows, 384
+//    tiles: 34 / 39; E = 64, K = 512, N = 768, 512 rows, 408 tiles: 36 / 22);
 //  - eight waves on 256-row tiles where there are many of them and the experts
-//    have the rows (E = 8, K = 4096, N = 8192 with 16384 rows 3.45 ms against
-//    3.92; E = 64, K = 1024, N = 512, 256 rows an expert: 86 / 94 us uniform,
-//    95 / 102 skewed, but E = 64, K = 512, N = 768, 256 rows an expert: 86 / 74).
+//    have the rows (E = 8, K = 4096, N = 8192 with 16384 rows 3.58 ms against
+//    3.90; E = 64, K = 1024, N = 512, 256 rows an expert: 68 / 71 us, but E = 64,
+//    K = 512, N = 768, 256 rows an expert: 76 / 67).
 //    Not for the chain: nothing runs under a tile's combine with one workgroup
 //    a CU (T = 16384, E = 128, K = 2048, N = 768 chain 724 against 641 us);
 //  - else four waves on 128-row tiles, two workgroups a CU.
