@@ -42,9 +42,9 @@ sys.path.insert(0, str(REPO))
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, vendor peak
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix, vendor peak
-# FP32 products made of three FP16 ones (the split grouped GEMM): a third of the
-# dense FP16 vendor peak
-SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 3
+# FP32 products made of six BF16 ones (the split grouped GEMM): a sixth of the
+# dense BF16 vendor peak
+SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 6
 RIDGE = FP32_MFMA_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9)  # flop/byte, FP32 instructions
 
 
@@ -137,7 +137,7 @@ def roofline(name, nbytes, flops, seconds, split=False):
     ridge = SPLIT_MFMA_PEAK_TFLOPS / FP32_MFMA_PEAK_TFLOPS * RIDGE if split else RIDGE
     if flops and flops / nbytes > ridge:
         achieved = flops / seconds / 1e12
-        return {"bound": "mfma", "products": "three fp16" if split else "fp32", "achieved": round(achieved, 3),
+        return {"bound": "mfma", "products": "six bf16" if split else "fp32", "achieved": round(achieved, 3),
                 "peak": peak, "unit": "TFLOP/s", "frac": round(achieved / peak, 4)}
     achieved = nbytes / seconds / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -798,7 +798,7 @@ bool direct_any_disabled() {
   return v != nullptr && std::strcmp(v, "aligned") == 0;
 }
 
-// Whether a grouped GEMM runs on the FP16 matrix cores (split_gemm.hip).
+// Whether a grouped GEMM runs on the BF16 matrix cores (split_gemm.hip).
 // RR_GEMM_STAGING=fp32 keeps it on the FP32 instructions; split takes the split
 // kernel wherever it can run, split4, split8 and split256 with one of its
 // workgroup shapes, for tests and A/B runs.

@@ -1,4 +1,4 @@
-// Grouped FP32 GEMM on the FP16 matrix cores (split_gemm.hip).
+// Grouped FP32 GEMM on the BF16 matrix cores (split_gemm.hip).
 #pragma once
 
 #include <hip/hip_runtime_api.h>

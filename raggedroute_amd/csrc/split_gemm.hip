@@ -1,86 +1,64 @@
-// Grouped FP32 GEMM on the FP16 matrix cores (v_mfma_f32_32x32x16_f16).
+// Grouped FP32 GEMM on the BF16 matrix cores (v_mfma_f32_32x32x16_bf16).
 //
-// The FP32 matrix instructions run at 157 TFLOP/s, the FP16 ones at 2.5 PFLOP/s
-// with FP32 accumulation. Every operand x is scaled by a power of two of its
-// own row (A) or column (B), xs = x * s, and split into two FP16 numbers
-//     h = fp16(xs),   l = fp16(xs - h),   l stored times 2^11,
-// both rounded to nearest; xs - h is exact in FP32 and at most 2^-11 of xs, so
-// h + l carries x to within 2^-23 of itself (half of all values exactly). A
-// product is
-//     xs * ys = hx hy + (lx hy + hx ly) + lx ly;
-// the first three terms are computed (three MFMAs), the last is at most 2^-22 of
-// the product (2^-25 in the mean) and left out. hx hy is summed in one FP32
-// accumulator and the two small terms in another, which is added once, times
-// 2^-11, at the end: the large sum is rounded once per 16 k instead of once per
-// 4 k as on the FP32 instructions. Against 64-bit sums dense operands' results
-// are closer than the FP32 instructions' at every K (2-norm error over N(0,1) operands, this / FP32 MFMA:
-// K = 64 0.98 / 1.43e-7, K = 128 1.10 / 2.03e-7, K = 256 1.31 / 2.87e-7, K = 1024
-// 2.2 / 5.8e-7, K = 4096 4.1 / 11.4e-7; non-negative operands K = 128 0.64 / 1.59e-7;
-// both operands half zero K = 128 1.06 / 1.04e-7, K = 192 1.16 / 1.26e-7). Sums of few
-// products have the split's own error instead: K = 1024, rows of 64 nonzero values
-// 1.46 / 1.44e-7, of 16 1.03 / 0.74e-7, of one 0.77 / 0.25e-7.
+// The FP32 matrix instructions run at 157 TFLOP/s, the BF16 ones at 2.5 PFLOP/s
+// with FP32 accumulation. Every operand is split into three BF16 numbers,
+//     x0 = bf16(x),   x1 = bf16(x - x0),   x2 = bf16(x - x0 - x1),
+// rounded to nearest; the differences are exact in FP32, and x0 + x1 + x2 = x: all 24
+// bits over FP32's own exponent range, without scales. A product is
+//     x y = x0 y0 + (x0 y1 + x1 y0) + (x1 y1 + x0 y2 + x2 y0) + ...;
+// the first six terms are computed (six MFMAs), the others are at most 2^-25 of the
+// product and left out. x0 y0 is summed in one FP32 accumulator and the five small
+// terms in another, which is added once at the end: the large sum is rounded once
+// per 16 k instead of once per 4 k as on the FP32 instructions. Against 64-bit sums
+// the result is closer than the FP32 instructions' (2-norm error, this / FP32 MFMA,
+// 1e-7: N(0,1) operands K = 128 0.65 / 2.03, K = 1024 1.86 / 5.73, K = 4096 3.96 / 11.4;
+// non-negative K = 128 0.62 / 1.59; both half zero K = 128 0.43 / 1.04; K = 1024 with 16
+// nonzero values a row 0.34 / 0.74, with one 0.26 / 0.25), whatever the scales of
+// features and weights, and a row of one 1 returns its weight row exactly.
+// (Two FP16 numbers, scaled per row and column, and three products took two thirds
+// of the time - T = 8192, E = 8, K = 4096, N = 14336 call 6.8 ms against 9.8, chain T =
+// 16384, E = 128, K = 2048, N = 768 600 us against 800 - but hold 23 bits over 2^30 of
+// range: values 2^-20 and less of the one that set the scale lost bits without a
+// sign. Marking rows that have such values for the FP32 instructions cost 3 to 7 %
+// and left single ones wrong; correcting those spilled the loop's registers.)
 //
-// Range. The scale puts the largest of a row's (column's) first slice of 32 k
-// near 2^6, so later values may be 2^9 times larger before fp16(xs)
-// overflows. (Where that slice is all zero, 1 is taken for the largest; reading on
-// to the first value made a tile with one all-zero row, a padding token, scan all
-// of K first: E = 8, 16384 rows, K = 4096, N = 14336 11.7 ms, now 6.3 as without such
-// rows; E = 64, 4096 rows, K = 1024, N = 512 72 -> 36 us.) l, stored times 2^11,
-// keeps its 11 bits down to |xs| = 2^-14 (2^-20 of the sampled maximum); below, the
-// split's error stays at 2^-36, so that values much smaller than the sample lose
-// their bits: with one feature 2^p times the rest and its weights zero, K = 320, the
-// 2-norm error was 1.8e-6 at p = 24, 1.1e-4 at p = 30, 0.1 at p = 40 (FP32
-// instructions 3.2e-7). Nothing of that kind is computed this way. A row or column is marked when
-//  - its sample is below 2^-100, or 2^41 and more (or not finite);
-//  - four of its values in slice 0 are nonzero and scale to less than 2^-14;
-//  - of four consecutive k (4 i .. 4 i + 3) past slice 0 the largest does.
-// So of any four k of an unmarked row past slice 0 the split's error is at most
-// 2^-22 of the largest, and values whose xs is below 2^-14 are few among larger
-// ones. (A scaled value under 2^-149 counts as zero: |x| < 2^-115 in a row whose
-// sample is 2^40.) An operand past the FP16 range makes every output it meets
-// non-finite. Outputs of marked rows and columns and non-finite ones are computed
-// on the FP32 instructions instead, with the bits of the FP32 kernels. Which those
-// are is a matter of each output's own row and column, so that no row's bits
-// depend on the rows it shares a tile with, or on the tile's height. A tile
-// with such outputs goes through its slices once more, with FP32 products only
-// for the 16-row blocks that hold one: E = 8, 16384 rows, K = 4096, N = 14336, one
-// infinite row in a thousand 10.4 ms (17.4 when whole tiles were computed again, as
-// 32 x 32 products without a slice on its way; FP32 kernel 13.8); E = 128, 32768
-// rows, K = 2048, N = 768 569 us (979; 760). Where every row has such a value (a
-// feature 2^14 times the others) the second pass is a whole FP32 product and comes
-// on top: 23.0 ms and 1.36 ms. N(0,1) rows are as good as
-// never marked (four neighbours below 2^-19); of rows with every other value zero at
-// random, four in 10^4 at K = 4096. The marks take 24 of 132 vector instructions of a slice of
-// the 256-row loop: T = 8192, E = 8, K = 4096, N = 14336 call 6.80 -> 7.21 ms, T = 3001,
-// E = 9, K = 1023, N = 1535 150 -> 156 us, chain T = 16384, E = 128, K = 2048, N = 768
-// 607 -> 626 us, T = 2048, E = 64, K = 1024, N = 512 70.2 -> 72.1 us. (Pairs of k, and
-// groups over two slices or two lanes, were slower: 7.1 - 8.0 ms in the first.)
+// Outputs that are not finite (an infinity or NaN in an operand, |x| that rounds past
+// BF16's range, an overflowing sum) or not zero and below 2^-80 (operands under 2^-109
+// have parts below BF16's least value; met by values up to 2^20 they are lost in
+// nothing larger) are computed again on the FP32 instructions, with the bits of the
+// FP32 kernels, in a second pass of the tile over its slices that multiplies only
+// 16-row blocks with such an output (E = 8, 16384 rows, K = 4096, N = 14336, one infinite
+// row in a thousand 9.0 -> 12.5 ms; all on the FP32 kernel 13.8). Which outputs those
+// are is a matter of each one's own value, so that no row's bits depend on the
+// rows it shares a tile with, or on the tile's height.
 //
 // Work split: output tiles of 128 columns and 128 or 256 rows on four or eight
-// waves (split_grouped picks), tiles dealt as in gemm.hip. A slice of 32 k of
-// both operands is loaded into registers one slice ahead (16-byte A quads, 8-byte
-// B pairs; rows may start at any 4-byte boundary), split there, and written to
-// LDS as FP16 planes in MFMA operand order (k contiguous per row of A and per
-// column of B), two stages; the split costs four full-rate instructions per
-// element. Four waves: two workgroups share a CU and
-// one's MFMAs run under the other's staging. Eight waves: the two halves of the
-// workgroup run a phase apart, so that one has the matrix pipe while the other
-// stages. Tiles with few rows take layouts of fewer 32-row blocks.
-// Loads are buffer loads (scalar base, 32-bit lane offset): with 64-bit lane
-// addresses the eight-wave loop spilled (256 registers).
+// waves (split_grouped picks), tiles dealt as in gemm.hip. A slice of 16 k of
+// both operands is loaded into registers one slice ahead, or two where registers
+// are left (16-byte A quads, 8-byte B pairs; rows may start at any 4-byte boundary;
+// two ahead: chain T = 16384, E = 128, K = 2048, N = 768 842 -> 798 us), split there (5.5
+// instructions an element), and written to LDS as three BF16 planes in MFMA
+// operand order (k contiguous per row of A and per column of B), two stages. Four
+// waves: two workgroups share a CU and one's MFMAs run under the other's staging.
+// Eight waves: the two halves of the workgroup run a phase apart, so that one has
+// the matrix pipe while the other stages. Tiles with few rows take layouts of fewer
+// 32-row blocks. (Slices of 32 k: 96 KiB of planes for four waves, one workgroup a
+// CU, and no registers for both halves' operands.)
+// Loads are buffer loads (scalar base, 32-bit lane offset), which need no address
+// registers or arithmetic of the lanes.
 //
-// Large problems are bound by the staging phase (operand reads, split, marks and
-// plane writes of one half, longer than the other half's matrix instructions) at a
-// clock that the power limit holds down: E = 8, K = 4096, N = 14336, 16384 rows (1.92
-// TFLOP), matrix pipes busy 42 % of the cycles at 1.77 of 2.4 GHz. FP32
-// instructions 13.8 ms, four waves 7.1, eight waves 6.3 ms (304 TFLOP/s of FP32
-// products, 912 of FP16 ones; a library FP16 product of random 8192 x 8192 matrices
-// reaches 1300 on this card), 5.3 ms with operands of ones, which draw less
-// power. Elsewhere by each tile's serial parts and the combine: T = 16384, E = 128,
-// K = 2048, N = 768 chain, expert GEMM 927 / 557 us, matrix pipes 28 % busy at 2.0 GHz;
-// T = 2048, E = 64, K = 1024, N = 512 13 %.
+// Large problems: matrix pipes busy 65 % of the cycles at 1.70 of 2.4 GHz (the power
+// limit holds the clock down): E = 8, K = 4096, N = 14336, 16384 rows (1.92 TFLOP) FP32
+// instructions 13.8 ms, four waves 10.8, eight waves on 256 rows 9.0 (213 TFLOP/s of
+// FP32 products, 1.28 PFLOP/s of BF16 ones), 6.7 ms with operands of ones, which
+// draw less power. Elsewhere by each tile's serial parts and the combine: pipes busy
+// 44 % in the chain T = 16384, E = 128, K = 2048, N = 768 at 1.9 GHz, 24 % in T = 2048, E =
+// 64, K = 1024, N = 512. (B staged as columns instead of column pairs in the eight-wave
+// shapes: a fifth of the LDS conflicts, 42 % of its index cycles, but twice the loads:
+// no faster anywhere, chain T = 2048 79 -> 82 us.)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 
@@ -95,16 +73,12 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
-constexpr int kBN = 128, kBK = 32;
-constexpr int kPlaneB = kBN * kBK;          // halfs of one plane of B (8 KiB)
-constexpr float kLowScale = 2048.0F;        // l is stored times 2^11
-constexpr float kLeast = 0x1p-14F;          // scaled values from here on keep all bits of l
-constexpr int kFewSmall = 4;                // too small values of slice 0 that send a row or column to FP32
-constexpr int kMarked = 1 << 16;            // scale exponent of a row or column that is not computed in FP16
+constexpr int kParts = 3;                   // BF16 parts of a value
+constexpr int kBN = 128, kBK = 16;
+constexpr int kPlaneB = kBN * kBK;          // values of one plane (part) of B (4 KiB)
 constexpr int kBufferFlags = 0x00027000;    // raw 32-bit buffer
 
 // BM x 128 output tiles on W waves (four: two workgroups per CU; eight: one).
@@ -113,13 +87,14 @@ struct Shape {
   static constexpr int kWaves = W;
   static constexpr int kThreads = 64 * W;
   static constexpr int kBM = BM;
-  static constexpr int kPassRows = 8 * W;                        // rows of A staged per pass
+  static constexpr int kPassRows = 16 * W;                       // rows of A staged per pass
   static constexpr int kKPer = kBK / W;                          // k rows of B a thread stages
-  static constexpr int kPlaneA = kBM * kBK;                      // halfs
-  static constexpr int kStage = 2 * (kPlaneA + kPlaneB);         // A high, A low, B high, B low
+  static constexpr int kPlaneA = kBM * kBK;                      // values
+  static constexpr int kStage = kParts * (kPlaneA + kPlaneB);    // A's planes, B's planes
   static constexpr int kStage32 = (kBM + kBN) * kBK;             // floats
-  static_assert(2 * kStage32 * sizeof(float) <= 2 * kStage * sizeof(_Float16), "two FP32 slices fit the stages");
-  static_assert(kBM * (kBN / 32) * sizeof(uint32_t) <= W * 64 * sizeof(uint2), "the masks fit the column samples");
+  static constexpr int kMaskAt = 2 * kStage32;                   // masks of the outputs to recompute: words from here
+  static_assert((kMaskAt + kBM * (kBN / 32)) * sizeof(float) <= 2 * kStage * sizeof(__bf16),
+                "two FP32 slices and the masks fit the stages");
 };
 
 // Wave tiles of TM x TN blocks of 32 x 32. GRID: W / 2 x 2 waves of TN = 2 column
@@ -129,84 +104,52 @@ struct Layout {
   static constexpr int TM = TM_;
   static constexpr int TN = GRID ? 2 : 1;
   static constexpr int kRows = TM_ * 32 * (GRID ? W / 2 : W / 4);
-  static constexpr int kPasses = kRows / (8 * W);  // staging passes that hold the tile's rows
-  static_assert(kPasses * (8 * W) == kRows, "whole passes");
+  static constexpr int kPasses = (kRows + 16 * W - 1) / (16 * W);  // staging passes that hold the tile's rows
   __device__ static int row(int wave) { return (GRID ? wave >> 1 : wave >> 2) * 32 * TM_; }
-  // first tile column (plane row of B)
+  // first tile column
   __device__ static int col(int wave) { return GRID ? 64 * (wave & 1) : 32 * (wave & 3); }
 };
 
-// 16-byte chunk c (8 halfs) of plane row r sits at chunk c ^ ((r >> 2) & 3): the
-// 16 rows read together land in 16 distinct 16-byte bank groups. (B's writes do
-// not: 16 lanes write every second row, half of the groups; 30 % of the LDS's index
-// cycles at E = 8, K = 4096, N = 14336 are conflicts.)
-__device__ __forceinline__ int plane_swizzle(int r) { return (r >> 2) & 3; }
+// A plane row holds 16 k, two 16-byte chunks; chunk c of row r sits at chunk
+// c ^ swizzle(r), so that the 16 rows read together, and 16 rows written together,
+// land in distinct bank groups. Column c of B has plane row c / 2 (odd columns 64
+// further): a thread stages columns 2 l and 2 l + 1, its wave adjacent rows.
+__device__ __forceinline__ int swizzle(int r) { return ((r >> 3) ^ (r >> 6)) & 1; }
+__device__ __forceinline__ int plane_row(int c) { return (c >> 1) | ((c & 1) << 6); }
 
-// x * s = h + l (see the file comment): eight full-rate instructions for two
-// values. (Four v_fma_mixlo / mixhi_f16 would do, but they issue at half rate:
-// 9.7 against 4.7 cycles.)
-// x0 and x1 are left scaled.
-__device__ __forceinline__ void split2(float& x0, float& x1, float s, h2& h, h2& l) {
+// The BF16 parts of two values (see the file comment): eleven instructions.
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t (&part)[kParts]) {
   typedef float f2 __attribute__((ext_vector_type(2)));
-  const float s0 = x0 * s, s1 = x1 * s;
-  h = __builtin_convertvector(f2{s0, s1}, h2);
-  asm("" : "+v"(h));  // both halves in their register: the next two read them there
-  l = __builtin_convertvector(f2{__builtin_fmaf(x0, s, -static_cast<float>(h[0])) * kLowScale,
-                                 __builtin_fmaf(x1, s, -static_cast<float>(h[1])) * kLowScale}, h2);
-  x0 = s0;
-  x1 = s1;
+#pragma unroll
+  for (int i = 0; i < kParts; ++i) {
+    part[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x0, x1}, b2));
+    if (i + 1 < kParts) {
+      x0 -= __uint_as_float(part[i] << 16);
+      x1 -= __uint_as_float(part[i] & 0xFFFF0000U);
+    }
+  }
 }
 
-// The largest of four magnitudes (without the canonicalizing copies of fmaxf).
-__device__ __forceinline__ float most_of(float a, float b, float c, float d) {
-  float m;
-  asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(a), "v"(b), "v"(c));
-  asm("v_max_f32 %0, %1, |%2|" : "=v"(m) : "v"(m), "v"(d));
-  return m;
+// Sums that the parts cannot be trusted with: not finite, or nonzero and below 2^-80.
+__device__ __forceinline__ bool untrusted(float v) {
+  constexpr uint32_t kLeast = (127U - 80U) << 23;
+  const uint32_t bits = __float_as_uint(v) & 0x7FFFFFFFU;
+  return bits - kLeast >= 0x7F800000U - kLeast && bits != 0;
 }
-
-__device__ __forceinline__ uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFU; }
-__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
-
-// The scale of a row or column whose sampled maximum has these bits: s = 2^t
-// with t = 6 - floor(log2(max)). An all-zero sample is taken for one of largest
-// value 1: an all-zero row or column is exact under any scale, and later values
-// between 2^-20 and 2^9 are carried.
-struct Scale {
-  float s;
-  int t;
-  bool bad;  // not computed in FP16: below 2^-100, or 2^41 and more (or not finite)
-};
-__device__ __forceinline__ Scale scale_of(uint32_t bits) {
-  Scale sc;
-  int e = static_cast<int>(bits >> 23);
-  sc.bad = bits != 0 && (e > 167 || e < 27);
-  e = bits == 0 ? 127 : (e < 27 ? 27 : e);
-  sc.t = 133 - e;
-  sc.s = __uint_as_float(static_cast<uint32_t>(260 - e) << 23);
-  return sc;
-}
-
-// Whether a scaled magnitude (its bits) is too small for the split: nonzero and below kLeast.
-__device__ __forceinline__ bool too_small(uint32_t m) { return m - 1U < __float_as_uint(kLeast) - 1U; }
 
 // What a tile needs from the kernel (all workgroup-uniform).
 struct Tile {
   const float* B;  // the expert's weights
-  int row0, rows;  // first segment row, rows in the tile (1..128)
+  int row0, rows;  // first segment row, rows in the tile (1..kBM)
   int n0, ct;      // first column, column tile
 };
 struct Lds {
-  _Float16* stages;  // [2][kStage]
-  int32_t* ta;       // [kBM] scale exponents of the rows (kMarked: FP32)
-  int32_t* tb;       // [128] ... of the plane rows of B
-  uint2* cmax;       // [W][64] column samples; after the slices [kBM][4] masks of the outputs to recompute
-  int32_t* few;      // [128] values of slice 0 too small for their column's scale
+  __bf16* stages;    // [2][kStage]
   int32_t* src;      // [kBM] chain: token row of X per tile row (-1: none)
   float* w;          // [kBM] chain: route weight per tile row
 };
 
-// One output tile for one wave layout (L::kPasses 32-row passes hold its rows).
+// One output tile for one wave layout (L::kPasses passes hold its rows).
 template <class S, class L, bool CHAIN>
 __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, const Lds& sh, int col_tiles, int wave) {
   constexpr int W = S::kWaves;
@@ -230,12 +173,15 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   const int hi = lane >> 5;
   // staging: A quad ac of row PR p + ar; B columns 2 pair, 2 pair + 1 at k
   // KP wave .. + KP - 1
-  const int ar = tid >> 3;
-  const int ac = tid & 7;
+  const int ar = tid >> 2;
+  const int ac = tid & 3;
   const int pair = lane;
-  const int a_put = ar * kBK + (((ac >> 1) ^ plane_swizzle(ar)) << 3) + ((ac & 1) << 2);
+  const int a_put = ar * kBK + (((ac >> 1) ^ swizzle(ar & 63)) << 3) + ((ac & 1) << 2);
   const int b_k = KP * wave;
-  const int b_put = 2 * pair * kBK + (((b_k >> 3) ^ plane_swizzle(2 * pair)) << 3) + (b_k & 7);
+  const int b_put = pair * kBK + (((b_k >> 3) ^ swizzle(pair)) << 3) + (b_k & 7);
+  const int b_put1 = (64 + pair) * kBK + (((b_k >> 3) ^ swizzle(64 + pair)) << 3) + (b_k & 7);
+  // passes that hold rows of the layout for this wave
+  auto staged = [&](int p) { return L::kRows % PR == 0 || PR * p + 16 * wave < L::kRows; };
 
   // Rows past the tile's last read a row that exists (their products land in
   // output rows that are never stored); columns past N the last pair.
@@ -263,22 +209,24 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     return 4u * (static_cast<uint32_t>(kt) * kBK + static_cast<uint32_t>(j)) * static_cast<uint32_t>(N);
   };
 
-  f4u ra[P];
-  f2u rb[KP];
-  auto load = [&](int kt) {  // whole slices
+  struct Slice {  // as loaded
+    f4u a[P];
+    f2u b[KP];
+  };
+  auto load = [&](int kt, Slice& s) {  // whole slices
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      ra[p] = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(a_base, a_lane[p], 4 * kBK * kt, 0));
+      if (staged(p)) s.a[p] = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(a_base, a_lane[p], 4 * kBK * kt, 0));
     }
     // (a pair that crosses N reads the next k row's first float)
 #pragma unroll
     for (int j = 0; j < KP; ++j) {
-      rb[j] = __builtin_bit_cast(f2u, __builtin_amdgcn_raw_buffer_load_b64(b_base, b_lane, b_row(kt, j), 0));
+      s.b[j] = __builtin_bit_cast(f2u, __builtin_amdgcn_raw_buffer_load_b64(b_base, b_lane, b_row(kt, j), 0));
     }
   };
-  auto load_any = [&](int kt) {
+  auto load_any = [&](int kt, Slice& s) {
     if (kt != guarded) {
-      load(kt);
+      load(kt, s);
       return;
     }
 #pragma unroll
@@ -289,7 +237,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         if (kt * kBK + 4 * ac + q < K) {
           v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(a_base, a_lane[p] + 4 * q, 4 * kBK * kt, 0));
         }
-        ra[p][q] = v;
+        s.a[p][q] = v;
       }
     }
 #pragma unroll
@@ -299,67 +247,17 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         v0 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b_base, b_lane, b_row(kt, j), 0));
         if (nl + 1 < N) v1 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b_base, b_lane + 4, b_row(kt, j), 0));
       }
-      rb[j] = f2u{v0, v1};
+      s.b[j] = f2u{v0, v1};
     }
   };
 
-  // ---- scales, from the first slice ----
-  load_any(0);
-  if (tid < kBN) sh.few[tid] = 0;
-  uint32_t ma[P];
-  uint32_t mb0 = 0, mb1 = 0;
-#pragma unroll
-  for (int p = 0; p < P; ++p) {
-    uint32_t m = umax(umax(abs_bits(ra[p][0]), abs_bits(ra[p][1])), umax(abs_bits(ra[p][2]), abs_bits(ra[p][3])));
-    // over the row's eight lanes: quad neighbours, then the half row's mirror
-    m = umax(m, rr::dev::dpp_move<0xB1>(m));
-    m = umax(m, rr::dev::dpp_move<0x4E>(m));
-    ma[p] = umax(m, rr::dev::dpp_move<0x141>(m));
-  }
-#pragma unroll
-  for (int j = 0; j < KP; ++j) {
-    mb0 = umax(mb0, abs_bits(rb[j][0]));
-    mb1 = umax(mb1, abs_bits(rb[j][1]));
-  }
-  sh.cmax[64 * wave + pair] = make_uint2(mb0, mb1);
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < W; ++w) {
-    const uint2 m = sh.cmax[64 * w + pair];
-    mb0 = umax(mb0, m.x);
-    mb1 = umax(mb1, m.y);
-  }
-  float sa[P], sb[2];
-#pragma unroll
-  for (int p = 0; p < P; ++p) {
-    const Scale sc = scale_of(ma[p]);
-    sa[p] = sc.s;
-    uint32_t few = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) few += too_small(abs_bits(ra[p][q] * sc.s)) ? 1U : 0U;
-    few += rr::dev::dpp_move<0xB1>(few);
-    few += rr::dev::dpp_move<0x4E>(few);
-    few += rr::dev::dpp_move<0x141>(few);
-    if (ac == 0) sh.ta[PR * p + ar] = sc.bad || few >= kFewSmall ? kMarked : sc.t;
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const Scale sc = scale_of(j == 0 ? mb0 : mb1);
-    sb[j] = sc.s;
-    if (wave == 0) sh.tb[2 * pair + j] = sc.bad ? kMarked : sc.t;
-    int32_t few = 0;
-#pragma unroll
-    for (int q = 0; q < KP; ++q) few += too_small(abs_bits(rb[q][j] * sc.s)) ? 1 : 0;
-    if (few != 0) atomicAdd(sh.few + 2 * pair + j, few);
-  }
-
   // Gathered rows go to x_permuted spread over the column tiles: tile ct
-  // writes the k slices kt with kt % col_tiles == ct.
+  // writes the pairs of k slices 2 i, 2 i + 1 (128 bytes a row) with i % col_tiles == ct.
   int next_xp = CHAIN && prm.x_permuted != nullptr ? tl.ct : -1;
-  auto store_xp = [&](int kt) {
+  auto store_xp = [&](int kt, const Slice& s) {
     if constexpr (CHAIN) {
-      if (kt != next_xp) return;
-      next_xp += col_tiles;
+      if (kt >> 1 != next_xp) return;
+      if ((kt & 1) != 0) next_xp += col_tiles;
       const int k = kt * kBK + 4 * ac;
 #pragma unroll
       for (int p = 0; p < P; ++p) {
@@ -367,57 +265,42 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         if (r < rows) {
           float* out = prm.x_permuted + static_cast<std::size_t>(tl.row0 + r) * K + k;
           if (k + 4 <= K) {
-            __builtin_nontemporal_store(ra[p], reinterpret_cast<f4u*>(out));
+            __builtin_nontemporal_store(s.a[p], reinterpret_cast<f4u*>(out));
           } else {
-            for (int q = 0; k + q < K; ++q) out[q] = ra[p][q];
+            for (int q = 0; k + q < K; ++q) out[q] = s.a[p][q];
           }
         }
       }
     } else {
-      (void)kt;
+      (void)kt, (void)s;
     }
   };
-  // The slice in registers, split, into an LDS stage; slices past the first also
-  // note the rows and columns with four k too small for the scale.
-  uint64_t small_a[P] = {}, small_b[2] = {};  // lane masks
-  auto put = [&](_Float16* __restrict__ st, int kt) {
-    float most_a[P], most_b[2][KP / 4];
+  // a slice, split, into an LDS stage
+  auto put = [&](__bf16* __restrict__ st, const Slice& s) {
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      h2 h0, l0, h1, l1;
-      float x0 = ra[p][0], x1 = ra[p][1], x2 = ra[p][2], x3 = ra[p][3];
-      split2(x0, x1, sa[p], h0, l0);
-      split2(x2, x3, sa[p], h1, l1);
-      most_a[p] = most_of(x0, x1, x2, x3);
-      *reinterpret_cast<h4*>(st + p * PR * kBK + a_put) = h4{h0[0], h0[1], h1[0], h1[1]};
-      *reinterpret_cast<h4*>(st + S::kPlaneA + p * PR * kBK + a_put) = h4{l0[0], l0[1], l1[0], l1[1]};
+      if (!staged(p)) continue;
+      uint32_t lo[kParts], up[kParts];
+      split2(s.a[p][0], s.a[p][1], lo);
+      split2(s.a[p][2], s.a[p][3], up);
+#pragma unroll
+      for (int i = 0; i < kParts; ++i) {
+        *reinterpret_cast<uint2*>(st + i * S::kPlaneA + p * PR * kBK + a_put) = make_uint2(lo[i], up[i]);
+      }
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      typedef _Float16 hk __attribute__((ext_vector_type(KP)));
-      hk h, l;
+      __bf16* out = st + kParts * S::kPlaneA + (j == 0 ? b_put : b_put1);
+      uint32_t part[KP / 2][kParts];
 #pragma unroll
-      for (int q = 0; q < KP / 4; ++q) {
-        h2 h0, l0, h1, l1;
-        float x0 = rb[4 * q][j], x1 = rb[4 * q + 1][j], x2 = rb[4 * q + 2][j], x3 = rb[4 * q + 3][j];
-        split2(x0, x1, sb[j], h0, l0);
-        split2(x2, x3, sb[j], h1, l1);
-        most_b[j][q] = most_of(x0, x1, x2, x3);
-        h[4 * q] = h0[0], h[4 * q + 1] = h0[1], h[4 * q + 2] = h1[0], h[4 * q + 3] = h1[1];
-        l[4 * q] = l0[0], l[4 * q + 1] = l0[1], l[4 * q + 2] = l1[0], l[4 * q + 3] = l1[1];
-      }
-      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + b_put + j * kBK) = h;
-      *reinterpret_cast<hk*>(st + 2 * S::kPlaneA + kPlaneB + b_put + j * kBK) = l;
-    }
-    if (kt > 0) {
+      for (int q = 0; q < KP / 2; ++q) split2(s.b[2 * q][j], s.b[2 * q + 1][j], part[q]);
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        small_a[p] |= __ballot(too_small(__float_as_uint(most_a[p])));
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-#pragma unroll
-        for (int q = 0; q < KP / 4; ++q) small_b[j] |= __ballot(too_small(__float_as_uint(most_b[j][q])));
+      for (int i = 0; i < kParts; ++i) {
+        if constexpr (KP == 4) {
+          *reinterpret_cast<uint2*>(out + i * kPlaneB) = make_uint2(part[0][i], part[1][i]);
+        } else {
+          *reinterpret_cast<uint32_t*>(out + i * kPlaneB) = part[0][i];
+        }
       }
     }
   };
@@ -433,49 +316,69 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     }
   }
   {
-    const int prow = L::col(wave) + li;
-    // operand chunk of k step ks: k = 16 ks + 8 hi .. + 7
-    const int aget = (wrow + li) * kBK, bget = prow * kBK;
-    const int achunk[2] = {(hi ^ plane_swizzle(li)) << 3, ((2 + hi) ^ plane_swizzle(li)) << 3};
-    const int bchunk[2] = {(hi ^ plane_swizzle(prow)) << 3, ((2 + hi) ^ plane_swizzle(prow)) << 3};
+    // operand chunk: k = 8 hi .. + 7 of a plane row
+    const int aget = (wrow + li) * kBK + ((hi ^ swizzle(li)) << 3);
+    const int brow = plane_row(L::col(wave) + li);  // (block j: 16 j rows further, whose swizzle is the same)
+    const int bget = brow * kBK + ((hi ^ swizzle(brow)) << 3);
     struct Operands {
-      h8 ah[TM], al[TM], bh[TN], bl[TN];
+      b8 a[kParts][TM], b[kParts][TN];
     };
-    auto fetch = [&](const _Float16* __restrict__ st, int ks, Operands& o) {
+    auto fetch_a = [&](const __bf16* __restrict__ st, int part, b8 (&a)[TM]) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        o.ah[i] = *reinterpret_cast<const h8*>(st + aget + achunk[ks] + i * 32 * kBK);
-        o.al[i] = *reinterpret_cast<const h8*>(st + S::kPlaneA + aget + achunk[ks] + i * 32 * kBK);
-      }
+      for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const b8*>(st + part * S::kPlaneA + aget + i * 32 * kBK);
+    };
+    auto fetch_b = [&](const __bf16* __restrict__ st, int part, b8 (&b)[TN]) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        o.bh[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + bget + bchunk[ks] + j * 32 * kBK);
-        o.bl[j] = *reinterpret_cast<const h8*>(st + 2 * S::kPlaneA + kPlaneB + bget + bchunk[ks] + j * 32 * kBK);
+        b[j] = *reinterpret_cast<const b8*>(st + kParts * S::kPlaneA + part * kPlaneB + bget + j * 16 * kBK);
       }
     };
+    auto fetch = [&](const __bf16* __restrict__ st, Operands& o) {
+#pragma unroll
+      for (int t = 0; t < kParts; ++t) {
+        fetch_a(st, t, o.a[t]);
+        fetch_b(st, t, o.b[t]);
+      }
+    };
+    auto product = [&](const b8 (&a)[TM], const b8 (&b)[TN], v16f (&sum)[TM][TN]) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], sum[i][j], 0, 0, 0);
+      }
+    };
+    // (one order of the sums in every shape)
     auto multiply = [&](const Operands& o) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.ah[i], o.bh[j], acc[i][j], 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.al[i], o.bh[j], low[i][j], 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.ah[i], o.bl[j], low[i][j], 0, 0, 0);
-      }
+      product(o.a[0], o.b[0], acc);
+      product(o.a[0], o.b[1], low);
+      product(o.a[0], o.b[2], low);
+      product(o.a[1], o.b[0], low);
+      product(o.a[1], o.b[1], low);
+      product(o.a[2], o.b[0], low);
     };
-    put(sh.stages, 0);
-    store_xp(0);
-    if (nk > 1) load_any(1);
+    // Slice kt is multiplied while slices kt + 2 .. kt + D are on their way; slice
+    // kt + 1 has landed and goes to the other stage, and its registers take the
+    // loads of slice kt + 1 + D. D = 2 where registers are left (slice i in set i & 1).
+    constexpr int D = S::kBM == 128 ? 2 : 1;
+    Slice even, odd;  // (D = 1: the first only)
+    load_any(0, even);
+    put(sh.stages, even);
+    store_xp(0, even);
+    if (nk > 1) load_any(1, D == 2 ? odd : even);
+    if (D == 2 && nk > 2) load_any(2, even);
     __syncthreads();
-    // Slice kt is multiplied while slice kt + 2 is on its way; slice kt + 1 has
-    // landed and goes to the other stage, and its registers take the loads.
+    auto next = [&](int kt, Slice& s) {
+      if (kt + 1 < nk) {
+        put(sh.stages + (~kt & 1) * S::kStage, s);
+        store_xp(kt + 1, s);
+      }
+      if (kt + 1 + D < nk) load_any(kt + 1 + D, s);
+    };
+    auto next_whole = [&](int kt, Slice& s) {
+      put(sh.stages + (~kt & 1) * S::kStage, s);
+      store_xp(kt + 1, s);
+      load(kt + 1 + D, s);
+    };
     if constexpr (W == 8) {
       // Two waves share a SIMD, one of each half of the workgroup. The halves
       // run a phase apart: while one fetches its operands of slice kt and stages
@@ -484,84 +387,78 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
       // before the first half reads it, and the stage it takes was last read
       // one barrier before the first half writes it.
       if (wave >= W / 2) __syncthreads();
-      auto phases = [&](int kt, auto more) {
-        const _Float16* cur = sh.stages + (kt & 1) * S::kStage;
-        Operands o0, o1;
-        fetch(cur, 0, o0);
-        fetch(cur, 1, o1);
-        more();
+      auto phases = [&](int kt, Slice& s, auto more) {
+        Operands o;
+        fetch(sh.stages + (kt & 1) * S::kStage, o);
+        more(kt, s);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
         __builtin_amdgcn_s_setprio(1);
-        multiply(o0);
-        multiply(o1);
+        multiply(o);
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
       };
       int kt = 0;
+      if constexpr (D == 2) {
 #pragma unroll 1
-      for (; kt + 3 < nk; ++kt) {
-        phases(kt, [&]() {
-          put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
-          store_xp(kt + 1);
-          load(kt + 2);
-        });
-      }
+        for (; kt + 5 < nk; kt += 2) {
+          phases(kt, odd, next_whole);
+          phases(kt + 1, even, next_whole);
+        }
 #pragma unroll 1
-      for (; kt < nk; ++kt) {
-        phases(kt, [&]() {
-          if (kt + 1 < nk) {
-            put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
-            store_xp(kt + 1);
-          }
-          if (kt + 2 < nk) load_any(kt + 2);
-        });
+        for (; kt < nk; kt += 2) {
+          phases(kt, odd, next);
+          if (kt + 1 < nk) phases(kt + 1, even, next);
+        }
+      } else {
+#pragma unroll 1
+        for (; kt + 3 < nk; ++kt) phases(kt, even, next_whole);
+#pragma unroll 1
+        for (; kt < nk; ++kt) phases(kt, even, next);
       }
       if (wave < W / 2) __syncthreads();
     } else {
-      auto both = [&](const _Float16* cur) {
-        Operands o;
-        fetch(cur, 0, o);
-        multiply(o);
-        fetch(cur, 1, o);
-        multiply(o);
+      static_assert(D == 2, "two sets of slice registers");
+      auto slice = [&](int kt) {
+        const __bf16* st = sh.stages + (kt & 1) * S::kStage;
+        // (parts read as they are needed: all at once leave no registers for the
+        // second slice on its way)
+        b8 a[TM], b[kParts][TN];
+        fetch_a(st, 0, a);
+#pragma unroll
+        for (int t = 0; t < kParts; ++t) fetch_b(st, t, b[t]);
+        product(a, b[0], acc);
+        product(a, b[1], low);
+        product(a, b[2], low);
+        fetch_a(st, 1, a);
+        product(a, b[0], low);
+        product(a, b[1], low);
+        fetch_a(st, 2, a);
+        product(a, b[0], low);
         __syncthreads();
       };
       int kt = 0;
 #pragma unroll 1
-      for (; kt + 3 < nk; ++kt) {
-        put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
-        store_xp(kt + 1);
-        load(kt + 2);
+      for (; kt + 5 < nk; kt += 2) {
+        next_whole(kt, odd);
         __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to the slice's end)
-        both(sh.stages + (kt & 1) * S::kStage);
+        slice(kt);
+        next_whole(kt + 1, even);
+        __builtin_amdgcn_sched_barrier(0);
+        slice(kt + 1);
       }
 #pragma unroll 1
-      for (; kt < nk; ++kt) {
+      for (; kt < nk; kt += 2) {
+        next(kt, odd);
+        slice(kt);
         if (kt + 1 < nk) {
-          put(sh.stages + (~kt & 1) * S::kStage, kt + 1);
-          store_xp(kt + 1);
+          next(kt + 1, even);
+          slice(kt + 1);
         }
-        if (kt + 2 < nk) load_any(kt + 2);
-        both(sh.stages + (kt & 1) * S::kStage);
       }
     }
   }
-
-  // What the scales could not carry: marked rows and columns, and sums that are
-  // not finite. (Each a matter of the output's own row and column, whatever else
-  // is in the tile.)
-#pragma unroll
-  for (int p = 0; p < P; ++p) {
-    if ((small_a[p] >> lane & 1) != 0) sh.ta[PR * p + ar] = kMarked;
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    if ((small_b[j] >> lane & 1) != 0) sh.tb[2 * pair + j] = kMarked;
-  }
-  if (tid < kBN && sh.few[tid] >= kFewSmall) sh.tb[tid] = kMarked;
-  __syncthreads();
 
   // (the lane id passes an empty asm so that none of the epilogue's addresses
   // is built before the loop and kept live across it)
@@ -571,8 +468,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
   const int ehi = ln >> 5;
   // output rows of accumulator register r: 32 i + 8 (r / 4) + 4 hi + r % 4 of the wave's
   const int ec = L::col(wave) + eli;  // tile column; block j: 32 j further
-  bool odd = tid < rows && sh.ta[tid] == kMarked;
-  if (tid < kBN && tl.n0 + tid < N) odd = odd || sh.tb[tid] == kMarked;
+  bool any = false;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -580,12 +476,12 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
-        acc[i][j][r] = __builtin_fmaf(low[i][j][r], 1.0F / kLowScale, acc[i][j][r]);
-        odd = odd || (rl < rows && tl.n0 + ec + 32 * j < N && abs_bits(acc[i][j][r]) >= 0x7F800000U);
+        acc[i][j][r] += low[i][j][r];
+        any = any || (rl < rows && tl.n0 + ec + 32 * j < N && untrusted(acc[i][j][r]));
       }
     }
   }
-  const bool redo = __syncthreads_or(odd ? 1 : 0) != 0;
+  const bool redo = __syncthreads_or(any ? 1 : 0) != 0;
   // the combined row of tile row rl (chain) and an output's way to memory
   auto combined_row = [&](int rl) -> float* {
     if constexpr (CHAIN) {
@@ -605,10 +501,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     }
   };
   float* const ytile = prm.Y + static_cast<std::size_t>(tl.row0) * N + tl.n0;
-  uint32_t* mask = reinterpret_cast<uint32_t*>(sh.cmax);  // [row][column / 32]
-  int tb[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) tb[j] = sh.tb[ec + 32 * j];
+  uint32_t* mask = reinterpret_cast<uint32_t*>(sh.stages) + S::kMaskAt;  // [row][column / 32]
   uint32_t again[TM] = {};  // bit 16 j + r: output (i, j, r) is one of those
   if (redo) {
 #pragma unroll
@@ -616,11 +509,9 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
-        const int ta = sh.ta[rl];
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const bool a = rl < rows && tl.n0 + ec + 32 * j < N &&
-                         (ta == kMarked || tb[j] == kMarked || abs_bits(acc[i][j][r]) >= 0x7F800000U);
+          const bool a = rl < rows && tl.n0 + ec + 32 * j < N && untrusted(acc[i][j][r]);
           const uint64_t m = __ballot(a);
           if (eli == 0) mask[4 * rl + (L::col(wave) >> 5) + j] = static_cast<uint32_t>(ehi == 0 ? m : m >> 32);
           again[i] |= a ? 1U << (16 * j + r) : 0U;
@@ -634,14 +525,13 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
     for (int r = 0; r < 16; ++r) {
       const int rl = wrow + 32 * i + 8 * (r >> 2) + 4 * ehi + (r & 3);
       if (rl >= rows) continue;
-      const int ta = sh.ta[rl];
       float* yrow = ytile + static_cast<std::size_t>(rl) * N + ec;
       float* comb = combined_row(rl);
       const float w = comb != nullptr ? sh.w[rl] : 0.0F;
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         if (tl.n0 + ec + 32 * j >= N || (again[i] >> (16 * j + r) & 1) != 0) continue;
-        emit(ldexpf(acc[i][j][r], -(ta + tb[j])), yrow + 32 * j, comb != nullptr ? comb + ec + 32 * j : nullptr, w);
+        emit(acc[i][j][r], yrow + 32 * j, comb != nullptr ? comb + ec + 32 * j : nullptr, w);
       }
     }
   }
@@ -670,8 +560,9 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll
     for (int j = 0; j < NJ; ++j) sum[i][j] = v4f{0.0F, 0.0F, 0.0F, 0.0F};
   }
-  // quad q of plane row r sits at quad q ^ (r & 7) (B: q ^ (r / 2 & 7))
-  load_any(0);
+  // quad q of row r sits at quad q ^ (r & 3) (B: q ^ (r / 2 & 3))
+  Slice s;
+  load_any(0, s);
 #pragma unroll 1
   for (int kt = 0; kt < nk; ++kt) {
     float* As = reinterpret_cast<float*>(sh.stages) + (kt & 1) * S::kStage32;
@@ -679,35 +570,30 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int r = PR * p + ar;
-      *reinterpret_cast<v4f*>(As + r * kBK + 4 * (ac ^ (r & 7))) = v4f{ra[p][0], ra[p][1], ra[p][2], ra[p][3]};
+      if (staged(p)) *reinterpret_cast<v4f*>(As + r * kBK + 4 * (ac ^ (r & 3))) = v4f{s.a[p][0], s.a[p][1], s.a[p][2], s.a[p][3]};
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
+      float* out = Bs + (2 * pair + j) * kBK + 4 * ((b_k >> 2) ^ (pair & 3)) + (b_k & 3);
 #pragma unroll
-      for (int q = 0; q < KP / 4; ++q) {
-        *reinterpret_cast<v4f*>(Bs + (2 * pair + j) * kBK + 4 * ((b_k / 4 + q) ^ (pair & 7))) =
-            v4f{rb[4 * q][j], rb[4 * q + 1][j], rb[4 * q + 2][j], rb[4 * q + 3][j]};
-      }
+      for (int q = 0; q < KP; ++q) out[q] = s.b[q][j];
     }
-    if (kt + 1 < nk) load_any(kt + 1);
+    if (kt + 1 < nk) load_any(kt + 1, s);
     __syncthreads();  // (the other stage was last read before the previous slice's barrier)
+    v4f b[NJ];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      v4f b[NJ];
+    for (int j = 0; j < NJ; ++j) {
+      const int col = CW * wave + 16 * j + fl;
+      b[j] = *reinterpret_cast<const v4f*>(Bs + col * kBK + 4 * (g ^ (col >> 1 & 3)));
+    }
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int col = CW * wave + 16 * j + fl;
-        b[j] = *reinterpret_cast<const v4f*>(Bs + col * kBK + 4 * ((4 * c + g) ^ (col >> 1 & 7)));
-      }
+    for (int i = 0; i < NB; ++i) {
+      if ((blocks >> i & 1) == 0) continue;
+      const v4f a = *reinterpret_cast<const v4f*>(As + (16 * i + fl) * kBK + 4 * (g ^ (fl & 3)));
 #pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        if ((blocks >> i & 1) == 0) continue;
-        const v4f a = *reinterpret_cast<const v4f*>(As + (16 * i + fl) * kBK + 4 * ((4 * c + g) ^ (fl & 7)));
+      for (int q = 0; q < 4; ++q) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[j][s], sum[i][j], 0, 0, 0);
-        }
+        for (int j = 0; j < NJ; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[j][q], sum[i][j], 0, 0, 0);
       }
     }
   }
@@ -733,14 +619,10 @@ template <int W, int BM, bool CHAIN>
 __global__ __launch_bounds__(64 * W, 2) void rr_split_gemm_kernel(GemmParams prm) {
   using S = Shape<W, BM>;
   constexpr int kBM = BM;
-  extern __shared__ __align__(16) _Float16 smem[];
+  extern __shared__ __align__(16) __bf16 smem[];
   Lds sh;
   sh.stages = smem;
-  sh.ta = reinterpret_cast<int32_t*>(smem + 2 * S::kStage);
-  sh.tb = sh.ta + kBM;
-  sh.cmax = reinterpret_cast<uint2*>(sh.tb + kBN);
-  sh.few = reinterpret_cast<int32_t*>(sh.cmax + W * 64);
-  sh.src = sh.few + kBN;
+  sh.src = reinterpret_cast<int32_t*>(smem + 2 * S::kStage);
   sh.w = reinterpret_cast<float*>(sh.src + kBM);
   int32_t* s_off = reinterpret_cast<int32_t*>(sh.w + kBM);  // [E + 1]
   int32_t* s_pre = s_off + prm.experts + 1;                 // [E + 1] full row tiles before expert e
@@ -829,8 +711,7 @@ hipError_t launch(const GemmParams& prm, long rows_per_expert, int cus, hipStrea
   long grid = bound < cap ? bound : cap;
   if (grid >= kXcds) grid = grid / kXcds * kXcds;
   if (grid < 1) grid = 1;
-  const std::size_t lds = 2 * S::kStage * sizeof(_Float16) + (S::kBM + kBN) * sizeof(int32_t) +
-                          W * 64 * sizeof(uint2) + kBN * sizeof(int32_t) + 2 * S::kBM * sizeof(int32_t) +
+  const std::size_t lds = 2 * S::kStage * sizeof(__bf16) + 2 * S::kBM * sizeof(int32_t) +
                           3 * static_cast<std::size_t>(prm.experts + 1) * sizeof(int32_t);
   rr_split_gemm_kernel<W, BM, CHAIN><<<dim3(static_cast<unsigned>(grid)), S::kThreads, lds, stream>>>(prm);
   return hipGetLastError();
@@ -846,29 +727,29 @@ long tiles(long rows, int experts, int bm, int n, int bn) { return (ceil_div(row
 // Where the FP32 kernels stay (grouped GEMM alone, experts' rows drawn at random,
 // FP32 kernels / this one):
 //  - K < 128 or N <= 64, where neither side is bound by the matrix instructions, and
-//    K and N both below 256 (chain T = 10296, E = 12, K = 100, N = 153 53 / 59 us, T =
-//    2523, E = 10, K = 106, N = 667 49 / 53);
+//    K and N both below 256;
 //  - problems of so few tiles that their smaller tiles spread over more CUs: with
-//    K >= 512 below one 64 x 64 tile a CU (E = 8, K = 1024, N = 512, 1024 rows, 192 tiles
-//    22 / 40 us; 4096 rows, 576 tiles 48 / 42), or 1.25 where the experts have less than
-//    eight rows each (E = 8, K = 512, N = 2048, 32 rows 16.3 / 20.0); with shorter K,
-//    where a tile's scales and first loads weigh more, below 2.5 (E = 16, K = 256,
-//    N = 1024, 1600 rows 17.8 / 18.9; E = 8, K = 256, N = 1536, 1200 rows, 648 tiles
-//    28.1 / 19.4), and up to 3 with K < 192 (E = 16, K = 128, N = 1024, 1600 rows, 656
-//    tiles 11.3 / 15.0; E = 64, K = 128, N = 768, 1536 rows, 1056 tiles 18.2 / 12.8);
+//    K >= 512 below 1.1 64 x 64 tiles a CU (E = 32, K = 1024, N = 256, 2048 rows, 256 tiles
+//    47 / 49 us; E = 8, K = 2048, N = 1536, 192 rows, 264 tiles 82 / 66), or 1.25 where the
+//    experts have less than eight rows each (E = 8, K = 512, N = 2048, 32 rows 16.4 /
+//    21.8); with shorter K, where a tile's first loads and last stores weigh more,
+//    below 2.5 (E = 16, K = 256, N = 1024, 1600 rows, 656 tiles 17.5 / 19.4; E = 16,
+//    K = 320, N = 768, 768 rows, 336 tiles 20.0 / 16.4, but E = 8, K = 256, N = 1536, 1200
+//    rows, 648 tiles 28 / 20), and 3.25 with K < 192 (E = 64, K = 128, N = 768, 640 rows, 888
+//    tiles 17.0 / 19.0);
 //  - few rows an expert where the FP32 side has its 128 x 128 tiles (two a CU): both
-//    are bound by the weights, which those load straight into LDS. E = 64, K = 128,
-//    N = 1024: 256 rows 8.6 / 11.7, 2048 rows 15.7 / 16.7, 3072 rows 19.6 / 18.0; E = 128,
-//    K = 320, N = 1024: 16 rows each 34.0 / 36.1, 24 rows 49.0 / 41.0; K = 1024: 4 rows each
-//    89 / 99, 16 rows 99 / 105, 24 rows 141 / 111; K = 4096: 4 rows each 314 / 349, 10 rows
-//    342 / 358, 16 rows 365 / 359 (chain K = 2048, N = 768, 10 rows each 222 / 215).
+//    are bound by the weights, which those load straight into LDS. E = 128, K = 128,
+//    N = 2048: 24 rows each 43 / 54 us, 48 rows 52 / 57; E = 128, K = 1024, N = 2048: 16 rows
+//    each 192 / 225; E = 128, K = 512, N = 1536: 16 rows 82 / 96, 24 rows 98 / 103, and E = 64,
+//    K = 4096, N = 2048 24 rows 442 / 458, but most shapes of 24 rows 1.0 to 1.4 times
+//    faster here.
 bool split_gemm_ok(int k, int n, int experts, long rows, int cus) {
   if (k < 128 || n <= 64 || (k < 256 && n < 256)) return false;
-  const long few = k < 192 ? 36 : (k < 512 ? 20 : (k < 2048 ? 16 : 8));  // rows an expert
+  const long few = k < 192 ? 40 : 20;  // rows an expert
   if (rows < few * experts && tiles(rows, experts, 128, n, 128) >= 2L * cus) return false;
   const long t = tiles(rows, experts, 64, n, 64);
-  if (k >= 512) return 4 * t >= (rows < 8L * experts ? 5L : 4L) * cus;
-  return k < 192 ? t > 3L * cus : 2 * t >= 5L * cus;
+  if (k >= 512) return 20 * t >= (rows < 8L * experts ? 25L : 22L) * cus;
+  return k < 192 ? 4 * t > 13L * cus : 2 * t >= 5L * cus;
 }
 
 // 32-bit byte offsets: a tile's A rows (chain: all of X) and an expert's weights.
@@ -879,22 +760,24 @@ bool split_gemm_fits(const GemmParams& prm) {
 }
 
 // Workgroup shape:
-//  - eight waves on 128-row tiles where a CU gets hardly more than one tile:
-//    more waves for it (E = 16, K = 2048, N = 300 with 8192 rows, 240 tiles: 72 us
-//    against 89 with four waves; E = 64, K = 1024, N = 512, 4096 rows, 384
-//    tiles: 34 / 39; E = 64, K = 512, N = 768, 512 rows, 408 tiles: 36 / 22);
+//  - eight waves on 128-row tiles where there are no more tiles than CUs: more waves
+//    for the one a CU gets (E = 16, K = 2048, N = 300 with 8192 rows: 95 us against 132 with
+//    four waves; chain T = 2048, E = 64, K = 1024, N = 512 77 / 89, but T = 4096, E = 16,
+//    K = 2048, N = 512, just past one tile a CU, 195 / 159). Tiles: full ones, and half
+//    of the experts with a part tile, but every expert that can have rows has one;
 //  - eight waves on 256-row tiles where there are many of them and the experts
-//    have the rows (E = 8, K = 4096, N = 8192 with 16384 rows 3.58 ms against
-//    3.90; E = 64, K = 1024, N = 512, 256 rows an expert: 68 / 71 us, but E = 64,
-//    K = 512, N = 768, 256 rows an expert: 76 / 67).
-//    Not for the chain: nothing runs under a tile's combine with one workgroup
-//    a CU (T = 16384, E = 128, K = 2048, N = 768 chain 724 against 641 us);
+//    have the rows (E = 8, K = 4096, N = 8192 with 16384 rows 5.09 ms against
+//    6.11; E = 64, K = 1024, N = 512, 256 rows an expert: 90 / 100 us, but E = 64,
+//    K = 512, N = 768, 256 rows an expert: 90 / 87). Not for the chain: nothing runs
+//    under a tile's combine with one workgroup a CU (T = 8192, E = 64, K = 1024, N = 768
+//    275 / 237 us, T = 16384, E = 128, K = 2048, N = 768 836 / 835);
 //  - else four waves on 128-row tiles, two workgroups a CU.
 hipError_t split_grouped(const GemmParams& prm, long rows_per_expert, long rows, int cus, SplitShape shape,
                          hipStream_t stream) {
   const bool chain = prm.sorted_route != nullptr;
   if (shape == SplitShape::kBySize) {
-    if (2 * tiles(rows, prm.experts, 128, prm.N, kBN) <= 3L * cus) {
+    const long halves = std::max(2 * ceil_div(rows, 128) + prm.experts, 2 * std::min<long>(rows, prm.experts));
+    if (halves * ceil_div(prm.N, kBN) <= 2L * cus) {
       shape = SplitShape::kEightWaves;
     } else if (prm.K >= 512 && tiles(rows, prm.experts, 256, prm.N, kBN) >= 2L * cus &&
                rows * prm.K >= (1L << 18) * prm.experts) {
