@@ -24,8 +24,9 @@
 //
 // Outputs that are not finite (an infinity or NaN in an operand, |x| that rounds past
 // BF16's range, an overflowing sum) or not zero and below 2^-80 (operands under 2^-109
-// have parts below BF16's least value; met by values up to 2^20 they are lost in
-// nothing larger) are computed again on the FP32 instructions, with the bits of the
+// have parts below BF16's least value, 2^-133; met by values up to 2^20 they make
+// nothing larger: x of 2^-114 times w of 2^40, 2^-74, is off by 5.6e-7, of 2^-110 by
+// 1.05e-7) are computed again on the FP32 instructions, with the bits of the
 // FP32 kernels, in a second pass of the tile over its slices that multiplies only
 // 16-row blocks with such an output (E = 8, 16384 rows, K = 4096, N = 14336, one infinite
 // row in a thousand 9.0 -> 12.5 ms; all on the FP32 kernel 13.8). Which outputs those
