@@ -254,6 +254,11 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
 
   // Gathered rows go to x_permuted spread over the column tiles: tile ct
   // writes the pairs of k slices 2 i, 2 i + 1 (128 bytes a row) with i % col_tiles == ct.
+  // Plain stores: rows of odd lengths share 64-byte blocks between slices, which only the
+  // cache puts together. Against stores past the caches, the chain at T = 9723, E = 68,
+  // K = 1345: N = 128 151 -> 90 us, N = 164 181 -> 140, N = 256 190 -> 150; where a slice
+  // is a whole block (K = 1344 or 2048) the two are within 1 %, at T = 12000, E = 24,
+  // K = 2000, N = 400 322 -> 340, and choosing by K keeps both in one loop and gains neither.
   int next_xp = CHAIN && prm.x_permuted != nullptr ? tl.ct : -1;
   auto store_xp = [&](int kt, const Slice& s) {
     if constexpr (CHAIN) {
@@ -266,7 +271,7 @@ __device__ __forceinline__ void run_tile(const GemmParams& prm, const Tile& tl, 
         if (r < rows) {
           float* out = prm.x_permuted + static_cast<std::size_t>(tl.row0 + r) * K + k;
           if (k + 4 <= K) {
-            __builtin_nontemporal_store(s.a[p], reinterpret_cast<f4u*>(out));
+            *reinterpret_cast<f4u*>(out) = s.a[p];
           } else {
             for (int q = 0; k + q < K; ++q) out[q] = s.a[p][q];
           }
