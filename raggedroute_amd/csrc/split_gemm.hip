@@ -749,6 +749,12 @@ long tiles(long rows, int experts, int bm, int n, int bn) { return (ceil_div(row
 //    each 192 / 225; E = 128, K = 512, N = 1536: 16 rows 82 / 96, 24 rows 98 / 103, and E = 64,
 //    K = 4096, N = 2048 24 rows 442 / 458, but most shapes of 24 rows 1.0 to 1.4 times
 //    faster here.
+// The lines are those of the whole range. Where N leaves a fifth or more of its 128-column
+// tiles empty, problems just past them are up to 15 % slower here (E = 24, K = 512, N = 400,
+// 3600 rows 26.5 / 30.3; E = 128, K = 512, N = 72, 8192 rows 25.5 / 29.4; 78 of 1344
+// combinations by more than 4 %), but of the same tile counts others are up to 1.9 times
+// faster (E = 8, K = 2048, N = 130, 12000 rows), and over 1344 combinations no line by
+// the padded columns came nearer to the faster side of each (2.0 % off on average).
 bool split_gemm_ok(int k, int n, int experts, long rows, int cus) {
   if (k < 128 || n <= 64 || (k < 256 && n < 256)) return false;
   const long few = k < 192 ? 40 : 20;  // rows an expert
@@ -768,8 +774,8 @@ bool split_gemm_fits(const GemmParams& prm) {
 // Workgroup shape:
 //  - eight waves on 128-row tiles where there are no more tiles than CUs: more waves
 //    for the one a CU gets (E = 16, K = 2048, N = 300 with 8192 rows: 95 us against 132 with
-//    four waves; chain T = 2048, E = 64, K = 1024, N = 512 77 / 89, but T = 4096, E = 16,
-//    K = 2048, N = 512, just past one tile a CU, 195 / 159). Tiles: full ones, and half
+//    four waves; chain T = 2048, E = 64, K = 1024, N = 512 75 / 83, but T = 4096, E = 16,
+//    K = 2048, N = 512, just past one tile a CU, 200 / 159). Tiles: full ones, and half
 //    of the experts with a part tile, but every expert that can have rows has one;
 //  - eight waves on 256-row tiles where there are many of them and the experts
 //    have the rows (E = 8, K = 4096, N = 8192 with 16384 rows 5.09 ms against
